@@ -38,8 +38,12 @@ int fbk_cell_fill(const DView &v, const int *atom_cell, int *cursor, int *cell_a
 int fbk_neighbors_fill(const DView &v, const int64_t *noff, int *neigh_j, int *neigh_b, int *neigh_self,
                        int *pair_atom, int *status, hipStream_t st);
 int fbk_neigh_back(const DView &v, int *neigh_back, int *status, hipStream_t st);
-int fbk_common_count(const DView &v, int *ncommon, int *status, hipStream_t st);
-int fbk_common_fill(const DView &v, const int64_t *toff, int4 *trip, int *trip_pair, int *status, hipStream_t st);
+int fbk_common_count(const DView &v, int scan, int *ncommon, hipStream_t st);
+int fbk_common_fill(const DView &v, int scan, const int64_t *toff, int4 *trip, int *trip_pair, hipStream_t st);
+int fbk_targets_nmax(void);
+int fbk_targets_count(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, hipStream_t st);
+int fbk_targets_fill(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, const TgtOut &out,
+                     hipStream_t st);
 int fbk_block_sizes(const DView &v, int64_t *sz, int4 *rec, hipStream_t st);
 int fbk_pair_perm(const DView &v, unsigned char *perm, hipStream_t st);
 int fbk_scan_i32(const int *in, int64_t *out, int64_t n, void *tmp, size_t *tmp_bytes, hipStream_t st);
@@ -129,6 +133,7 @@ struct HStruct {
   std::vector<double> ratom;
   std::vector<int> imass;
   double lattice[9];
+  bool coincident = false;   // two of its images coincide (images_coincide)
   std::vector<double> dQ;  // [natoms][FB_MAXSH]
   std::vector<double> qin; // [natoms][FB_MAXSH] input shell charges Qin (McWEDA densities)
   bool has_qin = false;
@@ -251,12 +256,15 @@ struct fb_ctx {
 
   DevBuf d_neighn, d_noff, d_neigh_j, d_neigh_b, d_neigh_back, d_neigh_self, d_pair_atom, d_pair_rec, d_pair_perm, d_bsz, d_boff;
   DevBuf d_ncommon, d_toff, d_trip_orig, d_tpair_orig, d_trip, d_tpair, d_perm_in, d_perm, d_flag, d_segincl,
-      d_seg_off, d_seg_pair, d_trip_seg, d_pair_tgt, d_trip_aux, d_tiles[3];
+      d_seg_off, d_seg_pair, d_trip_seg, d_pair_tgt, d_trip_aux, d_tiles[3], d_tgt_sum, d_tgt_mask, d_tgt_cnt;
+  int64_t order_gen = -1;        // lists_gen whose triplets are also there in the reference's list order
   int ntiles[3] = {0, 0, 0};
   DevBuf d_tmp, d_status;
   DevBuf d_mat[FB_NMAT];
   int64_t npairs = 0, ntrip = 0, nseg = 0, blen = 0;
   std::vector<int64_t> h_noff, h_toff, h_boff_struct;
+  std::vector<TgtSum> h_tgt;
+  int64_t order_ntrip = 0;
   bool lists_ok = false;
   int done[5] = {0, 0, 0, 0, 0};
 
@@ -561,7 +569,7 @@ struct fb_ctx {
                       &d_mu, &d_nu, &d_mv, &d_grid2c, &d_pden, &d_wg2c, &d_cell_cnt, &d_cell_start, &d_cell_atoms, &d_atom_cell, &d_pair_disp, &d_tile_cnt, &d_tile_off, &d_gidx, &d_gout, &d_st, &d_xl, &d_ratom, &d_imass, &d_atom_struct, &d_dQ,
                       &d_neighn, &d_noff, &d_neigh_j, &d_neigh_b, &d_neigh_back, &d_neigh_self, &d_pair_atom, &d_pair_rec, &d_pair_perm,
                       &d_bsz, &d_boff, &d_ncommon, &d_toff, &d_trip_orig, &d_tpair_orig, &d_trip, &d_tpair,
-                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
+                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
                       &d_mlp, &d_mlp_err, &d_mlp_count, &d_queue, &d_meth3c,
                       &d_status, &d_idx3r, &d_qin, &d_wbsz, &d_wboff, &d_pp_map, &d_px_map, &d_px_point,
                       &d_inv_pp, &d_inv_px, &d_cand_cnt, &d_cand_off, &d_cand_j, &d_cand_b, &d_pc_n, &d_pc_off,
@@ -618,6 +626,22 @@ static int make_cells(const double *lat, int icluster, double *xl) {
         mbeta++;
       }
   return mbeta - 1;
+}
+
+// two different images of the set within 1e-3 A of each other (a lattice of
+// no volume): then an image's number does not follow from its displacement
+static bool images_coincide(const double *lat, int icluster) {
+  if (icluster == 1) return false;
+  for (int iz = 0; iz <= 8; iz++)
+    for (int iy = -8; iy <= 8; iy++)
+      for (int ix = -8; ix <= 8; ix++) {
+        if (iz == 0 && (iy < 0 || (iy == 0 && ix <= 0))) continue;   // one of each pair k, -k
+        bool zero = true;
+        for (int k = 0; k < 3; k++)
+          zero &= !(std::fabs((double)ix * lat[k] + (double)iy * lat[3 + k] + (double)iz * lat[6 + k]) > 1.0e-3);
+        if (zero) return true;
+      }
+  return false;
 }
 
 // ------------------------------------------------------------------- C ABI
@@ -1212,6 +1236,7 @@ int fb_add_structure(fb_ctx *ctx, int natoms, const double *ratom, const int *im
   for (int i = 0; i < natoms; i++)
     if (imass[i] < 1 || imass[i] > ctx->sp.ns) return ctx->fail(FB_E_ARG, "add_structure: species out of range");
   std::memcpy(s.lattice, lattice, sizeof(s.lattice));
+  s.coincident = images_coincide(lattice, icluster);
   s.dQ.assign((size_t)natoms * FB_MAXSH, 0.0);
   if (dQ) std::memcpy(s.dQ.data(), dQ, sizeof(double) * natoms * FB_MAXSH);
   ctx->structs.push_back(std::move(s));
@@ -1394,6 +1419,164 @@ static int gather_to_host(fb_ctx *ctx, const int64_t *src, const std::vector<int
   return FB_OK;
 }
 
+static bool any_coincident(const fb_ctx *ctx) {
+  for (auto &s : ctx->structs)
+    if (s.coincident) return true;
+  return false;
+}
+
+// the arrays of T triplets sorted by target pair
+static int ensure_triplets(fb_ctx *ctx, int64_t T) {
+  if (T >= (1ll << 31)) return ctx->fail(FB_E_CAPACITY, "more than 2^31 pairs or triplets");
+  FB_HIP(ctx->d_trip.ensure(sizeof(int4) * T));
+  FB_HIP(ctx->d_tpair.ensure(sizeof(int) * T));
+  FB_HIP(ctx->d_trip_seg.ensure(sizeof(int) * T));
+  FB_HIP(ctx->d_trip_aux.ensure(sizeof(int) * T));
+  return FB_OK;
+}
+
+// Triplets, segments and tiles formed directly in target order (k_targets):
+// count, scan, fill.
+static int triplets_by_target(fb_ctx *ctx, int nmax) {
+  const int N = ctx->natoms;
+  const int64_t P = ctx->npairs;
+  hipStream_t st = ctx->stream;
+  FB_HIP(ctx->d_tgt_sum.ensure(sizeof(TgtSum) * (N + 1)));
+  FB_HIP(ctx->d_tgt_mask.ensure(sizeof(unsigned long long) * P * ((nmax + 63) / 64)));
+  FB_HIP(ctx->d_tgt_cnt.ensure(sizeof(int) * P));
+  TgtSum *sum = ctx->d_tgt_sum.as<TgtSum>();
+  unsigned long long *mask = ctx->d_tgt_mask.as<unsigned long long>();
+  int *cnt = ctx->d_tgt_cnt.as<int>();
+  DView v = ctx->view();
+  RC(ctx->launch("targets_count", [&] { return fbk_targets_count(v, nmax, sum, mask, cnt, st); }));
+  ctx->h_tgt.resize(N + 1);
+  FB_HIP(hipMemcpyAsync(ctx->h_tgt.data(), sum, sizeof(TgtSum) * (N + 1), hipMemcpyDeviceToHost, st));
+  FB_HIP(hipStreamSynchronize(st));
+  const TgtSum &tot = ctx->h_tgt[N];
+  const int64_t T = tot.trip;
+  RC(ensure_triplets(ctx, T));
+  FB_HIP(ctx->d_seg_off.ensure(sizeof(int64_t) * (tot.seg + 1)));
+  FB_HIP(ctx->d_seg_pair.ensure(sizeof(int) * tot.seg));
+  for (int k = 0; k < 3; k++) FB_HIP(ctx->d_tiles[k].ensure(sizeof(int4) * tot.tile[k]));
+  ctx->ntrip = T;
+  ctx->nseg = tot.seg;
+  TgtOut out{ctx->d_trip.as<int4>(),       ctx->d_tpair.as<int>(),    ctx->d_trip_seg.as<int>(),
+             ctx->d_trip_aux.as<int>(),    ctx->d_seg_off.as<int64_t>(), ctx->d_seg_pair.as<int>(),
+             ctx->d_pair_tgt.as<int>(),    {}};
+  for (int k = 0; k < 3; k++) {
+    ctx->ntiles[k] = tot.tile[k];
+    out.tiles[k] = ctx->d_tiles[k].as<int4>();
+  }
+  // of an atom's triplets only the structure's totals are kept on the host:
+  // the same whether an atom owns the targets or is the third atom
+  for (int i = 0; i <= N; i++) ctx->h_toff[i] = ctx->h_tgt[i].trip;
+  return ctx->launch("targets_fill", [&] { return fbk_targets_fill(v, nmax, sum, mask, cnt, out, st); });
+}
+
+// The triplets in the reference's list order with their target pairs, formed
+// when something asks for that order: the force assemblers, fb_get_common and
+// triplets_by_sort.
+static int list_order(fb_ctx *ctx) {
+  if (ctx->order_gen == ctx->lists_gen) return FB_OK;
+  const int N = ctx->natoms, scan = any_coincident(ctx);
+  hipStream_t st = ctx->stream;
+  DView v = ctx->view();
+  FB_HIP(ctx->d_ncommon.ensure(sizeof(int) * N));
+  FB_HIP(ctx->d_toff.ensure(sizeof(int64_t) * (N + 1)));
+  RC(ctx->launch("common_count", [&] { return fbk_common_count(v, scan, ctx->d_ncommon.as<int>(), st); }));
+  RC(scan_i32(ctx, ctx->d_ncommon.as<int>(), ctx->d_toff.as<int64_t>(), N));
+  int64_t T = 0;
+  FB_HIP(hipMemcpyAsync(&T, ctx->d_toff.as<int64_t>() + N, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  FB_HIP(hipStreamSynchronize(st));
+  if (T >= (1ll << 31)) return ctx->fail(FB_E_CAPACITY, "more than 2^31 pairs or triplets");
+  FB_HIP(ctx->d_trip_orig.ensure(sizeof(int4) * T));
+  FB_HIP(ctx->d_tpair_orig.ensure(sizeof(int) * T));
+  RC(ctx->launch("common_fill", [&] {
+    return fbk_common_fill(v, scan, ctx->d_toff.as<int64_t>(), ctx->d_trip_orig.as<int4>(),
+                           ctx->d_tpair_orig.as<int>(), st);
+  }));
+  ctx->order_ntrip = T;
+  ctx->order_gen = ctx->lists_gen;
+  return FB_OK;
+}
+
+// stable radix sort of the list-order triplets by target pair: their indices
+// into d_perm, the sorted targets into `sorted`
+static int sort_by_target(fb_ctx *ctx, int *sorted) {
+  const int64_t T = ctx->order_ntrip;
+  hipStream_t st = ctx->stream;
+  FB_HIP(ctx->d_perm_in.ensure(sizeof(int) * T));
+  FB_HIP(ctx->d_perm.ensure(sizeof(int) * T));
+  int end_bit = 1;
+  while ((1ll << end_bit) <= ctx->npairs) end_bit++;
+  RC(ctx->launch("iota", [&] { return fbk_iota(ctx->d_perm_in.as<int>(), T, st); }));
+  size_t bytes = 0;
+  int rc = fbk_sort_pairs(ctx->d_tpair_orig.as<int>(), sorted, ctx->d_perm_in.as<int>(), ctx->d_perm.as<int>(), T,
+                          end_bit, nullptr, &bytes, st);
+  if (rc) return ctx->fail(FB_E_HIP, "sort sizing", (hipError_t)rc);
+  RC(ensure_tmp(ctx, bytes));
+  bytes = ctx->d_tmp.cap;
+  return ctx->launch("sort_triplets", [&] {
+    return fbk_sort_pairs(ctx->d_tpair_orig.as<int>(), sorted, ctx->d_perm_in.as<int>(), ctx->d_perm.as<int>(), T,
+                          end_bit, ctx->d_tmp.p, &bytes, st);
+  });
+}
+
+// Triplets, segments and tiles from the list order by a sort: for atoms with
+// more neighbours than k_targets holds, and lattices with coincident images.
+static int triplets_by_sort(fb_ctx *ctx) {
+  const int N = ctx->natoms;
+  const int64_t P = ctx->npairs;
+  hipStream_t st = ctx->stream;
+  ctx->order_gen = -1;
+  RC(list_order(ctx));
+  const int64_t T = ctx->order_ntrip;
+  ctx->ntrip = T;
+  ctx->nseg = 0;
+  FB_HIP(hipMemcpyAsync(ctx->h_toff.data(), ctx->d_toff.p, sizeof(int64_t) * (N + 1), hipMemcpyDeviceToHost, st));
+  FB_HIP(hipStreamSynchronize(st));
+  for (int k = 0; k < 3; k++) ctx->ntiles[k] = 0;
+  RC(ctx->launch("clear_targets", [&] { return fbk_fill_i32(ctx->d_pair_tgt.as<int>(), P, 0, st); }));
+  if (T == 0) return FB_OK;
+  RC(ensure_triplets(ctx, T));
+  FB_HIP(ctx->d_flag.ensure(sizeof(int) * T));
+  FB_HIP(ctx->d_segincl.ensure(sizeof(int) * T));
+  FB_HIP(ctx->d_seg_off.ensure(sizeof(int64_t) * (T + 1)));
+  FB_HIP(ctx->d_seg_pair.ensure(sizeof(int) * T));
+  RC(sort_by_target(ctx, ctx->d_tpair.as<int>()));
+  RC(ctx->launch("seg_mark", [&] { return fbk_seg_mark(T, ctx->d_tpair.as<int>(), ctx->d_flag.as<int>(), st); }));
+  size_t b2 = 0;
+  int rc = fbk_scan_incl_i32(ctx->d_flag.as<int>(), ctx->d_segincl.as<int>(), T, nullptr, &b2, st);
+  if (rc) return ctx->fail(FB_E_HIP, "scan sizing", (hipError_t)rc);
+  RC(ensure_tmp(ctx, b2));
+  b2 = ctx->d_tmp.cap;
+  RC(ctx->launch("seg_scan", [&] {
+    return fbk_scan_incl_i32(ctx->d_flag.as<int>(), ctx->d_segincl.as<int>(), T, ctx->d_tmp.p, &b2, st);
+  }));
+  int nseg = 0;
+  FB_HIP(hipMemcpyAsync(&nseg, ctx->d_segincl.as<int>() + (T - 1), sizeof(int), hipMemcpyDeviceToHost, st));
+  RC(ctx->launch("seg_fill", [&] {
+    return fbk_seg_fill(T, ctx->d_tpair.as<int>(), ctx->d_segincl.as<int>(), ctx->d_seg_off.as<int64_t>(),
+                        ctx->d_seg_pair.as<int>(), ctx->d_trip_seg.as<int>(), ctx->d_pair_tgt.as<int>(), st);
+  }));
+  RC(ctx->launch("gather_triplets", [&] {
+    return fbk_gather_trip(T, ctx->d_perm.as<int>(), ctx->d_trip_orig.as<int4>(), ctx->d_trip.as<int4>(), st);
+  }));
+  FB_HIP(hipStreamSynchronize(st));
+  ctx->nseg = nseg;
+  // per-triplet group and structure (list properties: species and order only)
+  DView v = ctx->view();
+  RC(ctx->launch("trip_aux", [&] { return fbk_trip_aux(v, ctx->d_trip_aux.as<int>(), st); }));
+  // tiles: whole segments, at most one chunk of triplets per tile unless a
+  // single segment is longer, so that a workgroup makes one pass over its
+  // triplets
+  const int chs[3] = {64, 128, 256};
+  for (int k = 0; k < 3; k++)
+    RC(build_tiles(ctx, ctx->d_noff.as<int64_t>(), ctx->d_seg_off.as<int64_t>(), ctx->d_seg_pair.as<int>(), nseg,
+                   chs[k], ctx->d_tiles[k], &ctx->ntiles[k]));
+  return FB_OK;
+}
+
 int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
   if (!ctx) return FB_E_ARG;
   if (!ctx->tables_ok) return ctx->fail(FB_E_ORDER, "build_lists before commit_tables");
@@ -1450,6 +1633,8 @@ int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
   }));
   RC(ctx->launch("neigh_back", [&] { return fbk_neigh_back(v, ctx->d_neigh_back.as<int>(), v.status, st); }));
   FB_HIP(ctx->d_pair_disp.ensure(sizeof(double) * 3 * std::max<int64_t>(P, 1)));
+  FB_HIP(ctx->d_pair_tgt.ensure(sizeof(int) * std::max<int64_t>(P, 1)));
+  ctx->h_toff.resize(N + 1);
   v = ctx->view();
   RC(ctx->launch("pair_disp", [&] { return fbk_pair_disp(v, ctx->d_pair_disp.as<double>(), st); }));
   {
@@ -1459,85 +1644,12 @@ int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
     for (int i = 0; i < N; i++)
       if (self[i] == -999) return ctx->fail(FB_E_NEIGH_SELF, "find_neighbors: neigh_self missing");
   }
-  // common neighbours
-  FB_HIP(ctx->d_ncommon.ensure(sizeof(int) * N));
-  FB_HIP(ctx->d_toff.ensure(sizeof(int64_t) * (N + 1)));
-  RC(ctx->launch("common_count", [&] { return fbk_common_count(v, ctx->d_ncommon.as<int>(), v.status, st); }));
-  RC(scan_i32(ctx, ctx->d_ncommon.as<int>(), ctx->d_toff.as<int64_t>(), N));
-  ctx->h_toff.resize(N + 1);
-  FB_HIP(hipMemcpyAsync(ctx->h_toff.data(), ctx->d_toff.p, sizeof(int64_t) * (N + 1), hipMemcpyDeviceToHost, st));
-  RC(ctx->check_status("find_common_neighbors"));
-  ctx->ntrip = ctx->h_toff[N];
+  int nmax = 0;
+  for (int i = 0; i < N; i++) nmax = std::max<int64_t>(nmax, ctx->h_noff[i + 1] - ctx->h_noff[i]);
+  if (P >= (1ll << 31)) return ctx->fail(FB_E_CAPACITY, "more than 2^31 pairs or triplets");
+  const bool general = nmax > fbk_targets_nmax() || any_coincident(ctx);
+  RC(general ? triplets_by_sort(ctx) : triplets_by_target(ctx, nmax));
   const int64_t T = ctx->ntrip;
-  if (P >= (1ll << 31) || T >= (1ll << 31)) return ctx->fail(FB_E_CAPACITY, "more than 2^31 pairs or triplets");
-  FB_HIP(ctx->d_trip_orig.ensure(sizeof(int4) * T));
-  FB_HIP(ctx->d_tpair_orig.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_trip.ensure(sizeof(int4) * T));
-  FB_HIP(ctx->d_tpair.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_perm_in.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_perm.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_flag.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_segincl.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_seg_off.ensure(sizeof(int64_t) * (T + 1)));
-  FB_HIP(ctx->d_seg_pair.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_trip_seg.ensure(sizeof(int) * T));
-  FB_HIP(ctx->d_pair_tgt.ensure(sizeof(int) * std::max<int64_t>(P, 1)));
-  RC(ctx->launch("clear_targets", [&] { return fbk_fill_i32(ctx->d_pair_tgt.as<int>(), P, 0, st); }));
-  RC(ctx->launch("common_fill", [&] {
-    return fbk_common_fill(v, ctx->d_toff.as<int64_t>(), ctx->d_trip_orig.as<int4>(), ctx->d_tpair_orig.as<int>(),
-                           v.status, st);
-  }));
-  ctx->nseg = 0;
-  for (int k = 0; k < 3; k++) ctx->ntiles[k] = 0;
-  if (T > 0) {
-    // stable radix sort of triplet ids by target pair
-    int end_bit = 1;
-    while ((1ll << end_bit) <= P) end_bit++;
-    RC(ctx->launch("iota", [&] { return fbk_iota(ctx->d_perm_in.as<int>(), T, st); }));
-    size_t bytes = 0;
-    int rc = fbk_sort_pairs(ctx->d_tpair_orig.as<int>(), ctx->d_tpair.as<int>(), ctx->d_perm_in.as<int>(),
-                            ctx->d_perm.as<int>(), T, end_bit, nullptr, &bytes, st);
-    if (rc) return ctx->fail(FB_E_HIP, "sort sizing", (hipError_t)rc);
-    size_t b2 = 0;
-    rc = fbk_scan_incl_i32(ctx->d_flag.as<int>(), ctx->d_segincl.as<int>(), T, nullptr, &b2, st);
-    if (rc) return ctx->fail(FB_E_HIP, "scan sizing", (hipError_t)rc);
-    RC(ensure_tmp(ctx, std::max(bytes, b2)));
-    bytes = ctx->d_tmp.cap;
-    RC(ctx->launch("sort_triplets", [&] {
-      return fbk_sort_pairs(ctx->d_tpair_orig.as<int>(), ctx->d_tpair.as<int>(), ctx->d_perm_in.as<int>(),
-                            ctx->d_perm.as<int>(), T, end_bit, ctx->d_tmp.p, &bytes, st);
-    }));
-    RC(ctx->launch("seg_mark", [&] { return fbk_seg_mark(T, ctx->d_tpair.as<int>(), ctx->d_flag.as<int>(), st); }));
-    b2 = ctx->d_tmp.cap;
-    RC(ctx->launch("seg_scan", [&] {
-      return fbk_scan_incl_i32(ctx->d_flag.as<int>(), ctx->d_segincl.as<int>(), T, ctx->d_tmp.p, &b2, st);
-    }));
-    int nseg = 0;
-    FB_HIP(hipMemcpyAsync(&nseg, ctx->d_segincl.as<int>() + (T - 1), sizeof(int), hipMemcpyDeviceToHost, st));
-    RC(ctx->launch("seg_fill", [&] {
-      return fbk_seg_fill(T, ctx->d_tpair.as<int>(), ctx->d_segincl.as<int>(), ctx->d_seg_off.as<int64_t>(),
-                          ctx->d_seg_pair.as<int>(), ctx->d_trip_seg.as<int>(), ctx->d_pair_tgt.as<int>(), st);
-    }));
-    RC(ctx->launch("gather_triplets", [&] {
-      return fbk_gather_trip(T, ctx->d_perm.as<int>(), ctx->d_trip_orig.as<int4>(), ctx->d_trip.as<int4>(), st);
-    }));
-    FB_HIP(hipStreamSynchronize(st));
-    ctx->nseg = nseg;
-    // per-triplet group and structure, per-tile segment ownership (list
-    // properties: species and triplet order only)
-    FB_HIP(ctx->d_trip_aux.ensure(sizeof(int) * T));
-    v = ctx->view();
-    v.ntrip = T;
-    v.nseg = nseg;
-    RC(ctx->launch("trip_aux", [&] { return fbk_trip_aux(v, ctx->d_trip_aux.as<int>(), st); }));
-    // mixed-kernel tiles: whole segments, at most one chunk of triplets per
-    // tile unless a single segment is longer, so that a workgroup makes one
-    // pass over its triplets
-    const int chs[3] = {64, 128, 256};
-    for (int k = 0; k < 3; k++)
-      RC(build_tiles(ctx, ctx->d_noff.as<int64_t>(), ctx->d_seg_off.as<int64_t>(), ctx->d_seg_pair.as<int>(), nseg,
-                     chs[k], ctx->d_tiles[k], &ctx->ntiles[k]));
-  }
   // block offsets
   v = ctx->view();
   RC(ctx->launch("block_sizes", [&] {
@@ -1583,6 +1695,7 @@ int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
   }
   ctx->lists_ok = true;
   ctx->lists_gen++;
+  if (general) ctx->order_gen = ctx->lists_gen;   // triplets_by_sort formed it
   if (npairs_total) *npairs_total = P;
   if (ntrip_total) *ntrip_total = T;
   return FB_OK;
@@ -1623,6 +1736,8 @@ int fb_get_common(fb_ctx *ctx, int is, int *ncommon, int *iatom_j, int *iatom_b,
                   int *neigh_common) {
   if (!ctx || !ctx->lists_ok) return ctx ? ctx->fail(FB_E_ORDER, "lists not built") : FB_E_ARG;
   if (is < 0 || is >= (int)ctx->structs.size()) return ctx->fail(FB_E_ARG, "structure index");
+  FB_HIP(hipSetDevice(ctx->device));
+  RC(list_order(ctx));
   FB_HIP(hipStreamSynchronize(ctx->stream));
   const DStruct &d = ctx->h_st[is];
   int64_t t0 = ctx->h_toff[d.atom_off], t1 = ctx->h_toff[d.atom_off + d.natoms];
@@ -2851,6 +2966,7 @@ int fb_get_pp_blocks(fb_ctx *ctx, int is, int which, double *out) {
 static int prep_forces(fb_ctx *ctx) {
   if (ctx->forces_gen == ctx->lists_gen) return FB_OK;
   hipStream_t st = ctx->stream;
+  RC(list_order(ctx));
   const int64_t P = ctx->npairs, T = ctx->ntrip, B = ctx->blen;
   const int N = ctx->natoms;
   auto one = [](int64_t n) { return (size_t)std::max<int64_t>(n, 1); };
@@ -2885,7 +3001,9 @@ static int prep_forces(fb_ctx *ctx) {
       return fbk_sort_pairs(ctx->d_jkey.as<int>(), ctx->d_jkey_s.as<int>(), ctx->d_iota_t.as<int>(),
                             ctx->d_perm_j.as<int>(), T, end_bit, ctx->d_tmp.p, &bytes, st);
     }));
-    // the inverse orders: where each triplet's iatom / jatom record goes
+    // the inverse orders: where each triplet's iatom / jatom record goes (the
+    // sorted targets themselves are at hand, d_iota_t takes them)
+    RC(sort_by_target(ctx, ctx->d_iota_t.as<int>()));
     RC(ctx->launch("invert_perm", [&] { return fbk_invert_perm(T, ctx->d_perm.as<int>(), ctx->d_inv_perm.as<int>(), st); }));
     RC(ctx->launch("invert_perm", [&] {
       return fbk_invert_perm(T, ctx->d_perm_j.as<int>(), ctx->d_inv_perm_j.as<int>(), st);

@@ -108,6 +108,21 @@ struct DStruct {
   int cn[3], cell_off;
 };
 
+// Totals of one atom's targets (triplets, segments, tiles per 3c chunk), or
+// their exclusive prefix over the atoms; and what the target-order triplet
+// kernel writes (DView holds the same arrays)
+struct TgtSum {
+  int64_t trip;
+  int seg, tile[3];
+};
+struct TgtOut {
+  int4 *trip;
+  int *trip_pair, *trip_seg, *trip_aux;
+  int64_t *seg_off;
+  int *seg_pair, *pair_tgt;
+  int4 *tiles[3];
+};
+
 // all device pointers of a context, passed by value to kernels
 struct DView {
   DSpecies sp;

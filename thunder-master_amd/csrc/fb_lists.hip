@@ -181,12 +181,270 @@ __global__ void k_neigh_back(DView v, int *neigh_back, int *status) {
   neigh_back[p] = found;
 }
 
-// common neighbours of ialpha.  FILL = false counts (find_common_max plus the
-// drop rule of find_common_neighbors, so the counts are exact); FILL = true
-// writes the triplet and its target pair.
+// ------------------------------------------------ triplets in target order
+// Every assembler sums triplets per target block, in the reference's order
+// (ialpha ascending, then the common-pair order).  A target pair (iatom,
+// jatom at image mbeta) receives a triplet from every other neighbour of
+// iatom, an atom ialpha at image b, that has jatom among its own neighbours;
+// seen from ialpha, iatom lies at image ib = -b and jatom at jb = ib + mbeta.
+// So the neighbours of iatom, sorted by (ialpha, ib), give the segment of a
+// target directly and in order: no list-order pass, no search for mneigh (the
+// target is the pair at hand) and no sort.  The conditions are those of
+// find_common_neighbors (M_neighbors.f90:681-812) in ialpha's frame, with the
+// same binary64 expressions: jatom in ialpha's list, |r2 - r1| below the
+// range, and the pair's displacement within 1e-4 of r2 - r1.
+//
+// One workgroup per atom, one wavefront per target, lanes over the sorted
+// neighbours.  k_targets<false> tests the candidates and keeps the ballot
+// masks (one word per target and 64 neighbours), the targets' counts and the
+// atom's totals, with its tiles of whole segments (greedy, at most 64, 128 or
+// 256 triplets); k_targets<true> writes triplets, segments and tiles at the
+// scanned offsets from the masks alone.
+// LDS per neighbour: home position, iatom at image ib and cutoff (tests only),
+// atom, image, ib, count, prefix, segment, order
+#define TGT_LDS(FILL) (((FILL) ? 0 : 56) + 20 + 4)
+#define TGT_NMAX 768      // neighbours per atom: 61 KB
+
 template <bool FILL>
+__global__ __launch_bounds__(LWG) void k_targets(DView v, TgtSum *sum, unsigned long long *mask, int nword, int *pcnt,
+                                                 TgtOut out) {
+  extern __shared__ __align__(16) unsigned char s_mem[];
+  __shared__ int s_wave[LWG / 64];
+  const int ia = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int s = v.atom_struct[ia];
+  const DStruct S = v.st[s];
+  const double *xls = v.xl + (int64_t)s * FB_NIMG * 3;
+  const int64_t o = v.noff[ia];
+  const int n = (int)(v.noff[ia + 1] - o);
+  double *sRa = reinterpret_cast<double *>(s_mem), *sR1 = sRa + 3 * n, *sRc = sR1 + 3 * n;
+  int *sAt = reinterpret_cast<int *>(s_mem + (FILL ? 0 : 56 * (size_t)n));
+  int *sImg = sAt + n, *sIb = sImg + n, *sCnt = sIb + n, *sPre = sCnt + n;
+  unsigned short *sSeg = reinterpret_cast<unsigned short *>(sPre + n), *sOrd = sSeg + n;
+  const int in1 = v.imass[ia];
+  const double rc1 = v.sp.rcmax[in1 - 1];
+  for (int k = tid; k < n; k += LWG) {
+    const int at = S.atom_off + v.neigh_j[o + k] - 1, b = v.neigh_b[o + k];
+    int c[3];
+    image_coords(b, c);
+    const int ib = image_of(-c[0], -c[1], -c[2]);
+    sAt[k] = at;
+    sImg[k] = (c[0] + 4) | (c[1] + 4) << 4 | (c[2] + 4) << 8;
+    sIb[k] = ib;
+    if (FILL) {
+      sCnt[k] = pcnt[o + k];
+    } else {
+      sRc[k] = v.sp.rcmax[v.imass[at] - 1];
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        sRa[3 * k + q] = v.ratom[3 * at + q];
+        sR1[3 * k + q] = v.ratom[3 * ia + q] + xls[3 * ib + q];
+      }
+    }
+  }
+  __syncthreads();
+  // order of the neighbours by (ialpha, ib); the entries are distinct
+  for (int k = tid; k < n; k += LWG) {
+    const int at = sAt[k], ib = sIb[k];
+    int rank = 0;
+    for (int j = 0; j < n; j++) rank += (sAt[j] < at || (sAt[j] == at && sIb[j] < ib)) ? 1 : 0;
+    sOrd[rank] = (unsigned short)k;
+  }
+  TgtSum base = {0, 0, {0, 0, 0}};
+  if (FILL) {
+    base = sum[ia];
+    // first triplet and segment of every target
+    int run = 0, srun = 0;
+    for (int k0 = 0; k0 < n; k0 += LWG) {
+      const int k = k0 + tid, c = k < n ? sCnt[k] : 0;
+      int tot, stot;
+      const int pos = run + block_scan_count(c, s_wave, &tot);
+      const int sg = srun + block_rank(c > 0, s_wave, &stot);
+      if (k < n) {
+        sPre[k] = pos;
+        sSeg[k] = (unsigned short)sg;
+        out.pair_tgt[o + k] = c > 0;
+        if (c > 0) {
+          out.seg_off[base.seg + sg] = base.trip + pos;
+          out.seg_pair[base.seg + sg] = (int)(o + k);
+        }
+      }
+      run += tot;
+      srun += stot;
+    }
+    if (ia == v.natoms - 1 && tid == 0) out.seg_off[base.seg + srun] = base.trip + run;
+  }
+  __syncthreads();
+  for (int p = wave; p < n; p += LWG / 64) {
+    const int ja = sAt[p], cp = sImg[p];
+    const int px = (cp & 15) - 4, py = (cp >> 4 & 15) - 4, pz = (cp >> 8 & 15) - 4;
+    const bool target = !(ja == ia && px == 0 && py == 0 && pz == 0);   // not the self entry
+    if (FILL && sCnt[p] == 0) continue;
+    double rj[3] = {0.0, 0.0, 0.0}, dp[3] = {0.0, 0.0, 0.0}, rc2 = 0.0, range = 0.0;
+    if (!FILL) {
+      rc2 = sRc[p];
+      range = rc1 + rc2 - 0.01;
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        rj[q] = sRa[3 * p + q];
+        dp[q] = v.pair_disp[3 * (o + p) + q];
+      }
+    }
+    int count = 0;
+    for (int k0 = 0; k0 < n; k0 += 64) {
+      unsigned long long m = FILL ? mask[(o + p) * nword + (k0 >> 6)] : 0ull;
+      int ial = 0, ib = 0, jb = 0;
+      bool pass = FILL ? (m >> lane & 1ull) : (target && k0 + lane < n);
+      if (pass) {
+        const int k = sOrd[k0 + lane], ck = sImg[k];
+        ial = sAt[k];
+        ib = sIb[k];
+        const int x = px - (ck & 15) + 4, y = py - (ck >> 4 & 15) + 4, z = pz - (ck >> 8 & 15) + 4;
+        if (FILL) {
+          jb = image_of(x, y, z);
+        } else {
+          pass = abs(x) <= 4 && abs(y) <= 4 && abs(z) <= 4 && !(ial == ia && ib == 0);
+          if (pass) {
+            jb = image_of(x, y, z);
+            double r1[3], r2[3], ra[3];
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+              r1[q] = sR1[3 * k + q];
+              r2[q] = rj[q] + xls[3 * jb + q];
+              ra[q] = sRa[3 * k + q];
+            }
+            pass = !(ja == ial && jb == 0) && d_distance(ra, r2) < sRc[k] + rc2 - 0.01 &&
+                   d_distance(r1, r2) < range && fabs(dp[0] - r2[0] + r1[0]) < 1.0e-4 &&
+                   fabs(dp[1] - r2[1] + r1[1]) < 1.0e-4 && fabs(dp[2] - r2[2] + r1[2]) < 1.0e-4;
+          }
+        }
+      }
+      if (!FILL) {
+        m = __ballot(pass);
+        if (lane == 0) mask[(o + p) * nword + (k0 >> 6)] = m;
+      } else if (pass) {
+        const int64_t t = base.trip + sPre[p] + count + __popcll(m & ((1ull << lane) - 1ull));
+        out.trip[t] = make_int4(ial, ia, ja, (ib & 0xffff) | (jb << 16));
+        out.trip_pair[t] = (int)(o + p);
+        out.trip_seg[t] = base.seg + sSeg[p];
+        const int gid = v.idx3c[(((in1 - 1) * v.sp.ns + (v.imass[ja] - 1)) * v.sp.ns + (v.imass[ial] - 1)) *
+                                FB_MAXSUB3];
+        out.trip_aux[t] = (gid < 0 ? 0xffff : gid) | (s << 16);
+      }
+      count += __popcll(m);
+    }
+    if (!FILL && lane == 0) {
+      pcnt[o + p] = count;
+      sCnt[p] = count;
+    }
+  }
+  __syncthreads();
+  // tiles of whole segments: thread c packs greedily for 64 << c triplets (a
+  // longer segment alone), the rule of k_tiles_atom
+  if (tid < 3) {
+    const int ch = 64 << tid;
+    int4 *tl = out.tiles[tid];
+    int cur = 0, nt = 0, seg = 0, t = 0, s0 = 0, f0 = 0;
+    for (int k = 0; k < n; k++) {
+      const int c = sCnt[k];
+      if (c == 0) continue;
+      if (cur > 0 && cur + c > ch) {
+        if (FILL)
+          tl[base.tile[tid] + nt] =
+              make_int4(base.seg + s0, base.seg + seg - 1, (int)base.trip + f0, (int)base.trip + t);
+        nt++;
+        cur = 0;
+        s0 = seg;
+        f0 = t;
+      }
+      cur += c;
+      t += c;
+      seg++;
+    }
+    if (cur > 0) {
+      if (FILL)
+        tl[base.tile[tid] + nt] = make_int4(base.seg + s0, base.seg + seg - 1, (int)base.trip + f0, (int)base.trip + t);
+      nt++;
+    }
+    if (!FILL) {
+      sum[ia].tile[tid] = nt;
+      if (tid == 0) {
+        sum[ia].trip = t;
+        sum[ia].seg = seg;
+      }
+    }
+  }
+}
+
+// exclusive prefix of the atoms' totals in place (entry natoms: the totals);
+// one workgroup, four atoms per thread and pass
+__global__ __launch_bounds__(1024) void k_target_scan(int natoms, TgtSum *sum) {
+  __shared__ int64_t s_t[16];
+  __shared__ int s_i[16][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  TgtSum run = {0, 0, {0, 0, 0}};
+  for (int a0 = 0; a0 < natoms; a0 += 4096) {
+    const int a = a0 + 4 * tid;
+    TgtSum e[4], mine = {0, 0, {0, 0, 0}};
+    for (int u = 0; u < 4; u++) {
+      e[u] = (a + u < natoms) ? sum[a + u] : TgtSum{0, 0, {0, 0, 0}};
+      mine.trip += e[u].trip;
+      mine.seg += e[u].seg;
+      for (int c = 0; c < 3; c++) mine.tile[c] += e[u].tile[c];
+    }
+    TgtSum inc = mine;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t yt = __shfl_up(inc.trip, d);
+      const int ys = __shfl_up(inc.seg, d);
+      int yc[3];
+      for (int c = 0; c < 3; c++) yc[c] = __shfl_up(inc.tile[c], d);
+      if (lane >= d) {
+        inc.trip += yt;
+        inc.seg += ys;
+        for (int c = 0; c < 3; c++) inc.tile[c] += yc[c];
+      }
+    }
+    if (lane == 63) {
+      s_t[wave] = inc.trip;
+      s_i[wave][0] = inc.seg;
+      for (int c = 0; c < 3; c++) s_i[wave][1 + c] = inc.tile[c];
+    }
+    __syncthreads();
+    TgtSum off = run;
+    for (int w = 0; w < 16; w++) {
+      if (w < wave) {
+        off.trip += s_t[w];
+        off.seg += s_i[w][0];
+        for (int c = 0; c < 3; c++) off.tile[c] += s_i[w][1 + c];
+      }
+      run.trip += s_t[w];
+      run.seg += s_i[w][0];
+      for (int c = 0; c < 3; c++) run.tile[c] += s_i[w][1 + c];
+    }
+    __syncthreads();
+    off.trip += inc.trip - mine.trip;
+    off.seg += inc.seg - mine.seg;
+    for (int c = 0; c < 3; c++) off.tile[c] += inc.tile[c] - mine.tile[c];
+    for (int u = 0; u < 4; u++) {
+      if (a + u < natoms) sum[a + u] = off;
+      off.trip += e[u].trip;
+      off.seg += e[u].seg;
+      for (int c = 0; c < 3; c++) off.tile[c] += e[u].tile[c];
+    }
+  }
+  if (tid == 0) sum[natoms] = run;
+}
+
+// common neighbours of ialpha in the reference's list order (fb_get_common,
+// the force assemblers).  FILL = false counts (find_common_max plus the drop
+// rule of find_common_neighbors, so the counts are exact); FILL = true writes
+// the triplet and its target pair.  mneigh is the first entry of iatom whose
+// displacement matches r2 - r1 within 1e-4.  A list is sorted by (mbeta,
+// jatom) and names (jatom, jbeta - ibeta) at most once, so a binary search
+// finds it; SCAN tests the entries in order instead, for lattices in which
+// two images coincide and the difference may go by another image's number.
+template <bool FILL, bool SCAN>
 __global__ __launch_bounds__(LWG) void k_common(DView v, int *ncommon_out, const int64_t *toff,
-                                                int4 *trip, int *trip_pair, int *status) {
+                                                int4 *trip, int *trip_pair) {
   __shared__ int s_wave[LWG / 64];
   const int ial = blockIdx.x;
   const int s = v.atom_struct[ial];
@@ -219,23 +477,31 @@ __global__ __launch_bounds__(LWG) void k_common(DView v, int *ncommon_out, const
         double z = d_distance(r1, r2);
         double range_max = v.sp.rcmax[v.imass[gia] - 1] + v.sp.rcmax[v.imass[gja] - 1] - 0.01;
         if (z < range_max) {
-          // mneigh: the first kneigh of iatom whose displacement r3 = xl(kbeta)
-          // + r_k - r_i matches r2 - r1 within 1e-4 per component; eight
-          // displacements loaded at a time, tested in order
           const double *dp = v.pair_disp + 3 * v.noff[gia];
+          auto match = [&](int k) {
+            return fabs(dp[3 * k] - r2[0] + r1[0]) < 1.0e-4 && fabs(dp[3 * k + 1] - r2[1] + r1[1]) < 1.0e-4 &&
+                   fabs(dp[3 * k + 2] - r2[2] + r1[2]) < 1.0e-4;
+          };
           const int ni = v.neighn[gia];
-          for (int k0 = 0; k0 < ni && m == -9999; k0 += 8) {
-            double r3[8][3];
-#pragma unroll
-            for (int u = 0; u < 8; u++)
-              if (k0 + u < ni)
-#pragma unroll
-                for (int k = 0; k < 3; k++) r3[u][k] = dp[3 * (k0 + u) + k];
-#pragma unroll
-            for (int u = 0; u < 8; u++)
-              if (m == -9999 && k0 + u < ni && fabs(r3[u][0] - r2[0] + r1[0]) < 1.0e-4 &&
-                  fabs(r3[u][1] - r2[1] + r1[1]) < 1.0e-4 && fabs(r3[u][2] - r2[2] + r1[2]) < 1.0e-4)
-                m = k0 + u + 1;
+          if (SCAN) {
+            for (int k = 0; k < ni && m == -9999; k++)
+              if (match(k)) m = k + 1;
+          } else {
+            int ci[3], cj[3];
+            image_coords(ib, ci);
+            image_coords(jb, cj);
+            const int x = cj[0] - ci[0], y = cj[1] - ci[1], w = cj[2] - ci[2];
+            if (abs(x) <= 4 && abs(y) <= 4 && abs(w) <= 4) {
+              const int kb = image_of(x, y, w);
+              const int *lj = v.neigh_j + v.noff[gia], *lb = v.neigh_b + v.noff[gia];
+              int lo = 0, hi = ni;
+              while (lo < hi) {
+                const int mid = (lo + hi) >> 1, b = lb[mid];
+                if (b < kb || (b == kb && lj[mid] < ja)) lo = mid + 1;
+                else hi = mid;
+              }
+              if (lo < ni && lb[lo] == kb && lj[lo] == ja && match(lo)) m = lo + 1;
+            }
           }
           pass = (m != -9999);
         }
@@ -403,16 +669,42 @@ int fbk_neigh_back(const DView &v, int *neigh_back, int *status, hipStream_t st)
   return (int)hipGetLastError();
 }
 
-int fbk_common_count(const DView &v, int *ncommon, int *status, hipStream_t st) {
-  hipLaunchKernelGGL(k_common<false>, dim3(v.natoms), dim3(LWG), 0, st, v, ncommon, (const int64_t *)nullptr,
-                     (int4 *)nullptr, (int *)nullptr, status);
+int fbk_common_count(const DView &v, int scan, int *ncommon, hipStream_t st) {
+  const dim3 g((unsigned)v.natoms);
+  if (scan)
+    hipLaunchKernelGGL((k_common<false, true>), g, dim3(LWG), 0, st, v, ncommon, (const int64_t *)nullptr,
+                       (int4 *)nullptr, (int *)nullptr);
+  else
+    hipLaunchKernelGGL((k_common<false, false>), g, dim3(LWG), 0, st, v, ncommon, (const int64_t *)nullptr,
+                       (int4 *)nullptr, (int *)nullptr);
   return (int)hipGetLastError();
 }
 
-int fbk_common_fill(const DView &v, const int64_t *toff, int4 *trip, int *trip_pair, int *status,
-                    hipStream_t st) {
-  hipLaunchKernelGGL(k_common<true>, dim3(v.natoms), dim3(LWG), 0, st, v, (int *)nullptr, toff, trip, trip_pair,
-                     status);
+int fbk_common_fill(const DView &v, int scan, const int64_t *toff, int4 *trip, int *trip_pair, hipStream_t st) {
+  const dim3 g((unsigned)v.natoms);
+  if (scan)
+    hipLaunchKernelGGL((k_common<true, true>), g, dim3(LWG), 0, st, v, (int *)nullptr, toff, trip, trip_pair);
+  else
+    hipLaunchKernelGGL((k_common<true, false>), g, dim3(LWG), 0, st, v, (int *)nullptr, toff, trip, trip_pair);
+  return (int)hipGetLastError();
+}
+
+// most neighbours per atom that the target-order kernels take
+int fbk_targets_nmax(void) { return TGT_NMAX; }
+
+int fbk_targets_count(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, hipStream_t st) {
+  if (nmax > TGT_NMAX) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_targets<false>, dim3((unsigned)v.natoms), dim3(LWG), TGT_LDS(false) * (size_t)nmax, st, v, sum,
+                     mask, (nmax + 63) / 64, pcnt, TgtOut{});
+  hipLaunchKernelGGL(k_target_scan, dim3(1), dim3(1024), 0, st, v.natoms, sum);
+  return (int)hipGetLastError();
+}
+
+int fbk_targets_fill(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, const TgtOut &out,
+                     hipStream_t st) {
+  if (nmax > TGT_NMAX) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_targets<true>, dim3((unsigned)v.natoms), dim3(LWG), TGT_LDS(true) * (size_t)nmax, st, v, sum,
+                     mask, (nmax + 63) / 64, pcnt, out);
   return (int)hipGetLastError();
 }
 

@@ -134,3 +134,19 @@ __device__ __forceinline__ int hit_images(const DStruct &S, const double *xls, c
   __syncthreads();
   return n;
 }
+
+// make_cells order of the images (c.SYSTEM/make_cells.f90:130-144): iz outer,
+// iy, ix inner over -4..4 without the origin, which is image 0
+__device__ __forceinline__ void image_coords(int mb, int *c) {
+  if (mb == 0) { c[0] = c[1] = c[2] = 0; return; }
+  const int L = (mb <= 364) ? mb - 1 : mb;
+  c[0] = L % 9 - 4;
+  c[1] = (L / 9) % 9 - 4;
+  c[2] = L / 81 - 4;
+}
+
+// image of coordinates within -4..4
+__device__ __forceinline__ int image_of(int x, int y, int z) {
+  const int L = (z + 4) * 81 + (y + 4) * 9 + (x + 4);
+  return L < 364 ? L + 1 : (L > 364 ? L : 0);
+}

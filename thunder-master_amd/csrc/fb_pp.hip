@@ -125,16 +125,6 @@ __global__ __launch_bounds__(LWG) void k_pp_neighbors(DView v, DPP q, int list) 
   if (!FILL && threadIdx.x == 0) q.n[list][ia] = count;
 }
 
-// make_cells order of the images (c.SYSTEM/make_cells.f90:130-144): iz outer,
-// iy, ix inner over -4..4 without the origin, which is image 0
-__device__ __forceinline__ void image_coords(int mb, int *c) {
-  if (mb == 0) { c[0] = c[1] = c[2] = 0; return; }
-  const int L = (mb <= 364) ? mb - 1 : mb;
-  c[0] = L % 9 - 4;
-  c[1] = (L / 9) % 9 - 4;
-  c[2] = L / 81 - 4;
-}
-
 // the first image mbeta with |xl(mbeta) - (xl(jbeta) + xl(ibeta))| < 1e-4 in
 // make_cells order, mbeta_max + 1 when none (find_neighbors_PPp,
 // M_neighbors_PP.f90:983-990).  The integer sum of the two image coordinates
@@ -150,11 +140,7 @@ __device__ inline int image_of_sum(const DStruct &S, const double *xls, int ib, 
     image_coords(jb, c);
     const int x = a[0] + c[0], y = a[1] + c[1], z = a[2] + c[2];
     if (abs(x) <= 4 && abs(y) <= 4 && abs(z) <= 4) {
-      int m = 0;
-      if (x || y || z) {
-        const int L = (z + 4) * 81 + (y + 4) * 9 + (x + 4);
-        m = (L < 364) ? L + 1 : L;
-      }
+      const int m = image_of(x, y, z);
       // two images within 1e-4 of one point would need a lattice vector below 2e-4 A
       if (d_distance(xls + 3 * m, r3) < 1.0e-4) return m;
     }

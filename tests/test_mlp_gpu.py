@@ -180,3 +180,21 @@ def test_network_against_table_path():
     assert seen == ntrip
     assert 0.0 < frac <= 1.0
     assert err <= 1e-4
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 2048, 2049, 4133])
+def test_gradients_at_ragged_batches(n):
+    """Batches around a 16-row tile, around the largest count of partial
+    gradients (128 tiles, one or more per workgroup) and of one row.  FP32
+    products summed over n rows: the error of a sum is at most about
+    sqrt(n) 2^-24 of its terms, 2e-5 of the largest gradient here."""
+    rng = np.random.default_rng(n)
+    p = rng.normal(0, 0.25, mo.NP).astype(np.float32)
+    X = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    T = rng.normal(0, 1, (n, 64)).astype(np.float32)
+    loss, g = _asm(_si_tables()).mlp_gradients(10, p, X, T)
+    lref, gref = mo.loss_and_grads(p.astype(np.float64), X, T, 10)
+    assert abs(loss - lref) <= 1e-5 * lref
+    for s, e in ((mo.P_W1, mo.P_B1), (mo.P_B1, mo.P_W2), (mo.P_W2, mo.P_B2), (mo.P_B2, mo.P_W3),
+                 (mo.P_W3, mo.P_B3), (mo.P_B3, mo.NP)):
+        assert np.max(np.abs(g[s:e] - gref[s:e])) <= 2e-5 * np.max(np.abs(gref[s:e])), s

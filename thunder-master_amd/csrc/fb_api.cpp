@@ -74,16 +74,11 @@ int fbk_mlp_rowmax(int64_t n, const float *T, float *M, hipStream_t st);
 int fbk_mlp_unenvelope(int64_t n, const float *X, float *T, float c, float kx, float ky, float xh, float yh,
                        hipStream_t st);
 int fbk_mlp_scale_cols(int64_t n, int ncol, float *A, const float *inv, hipStream_t st);
-int fbk_mlp_gemm(int M, int N, int K, const float *A, int64_t sai, int64_t sak, const float *B, int64_t sbk,
-                 int64_t sbj, float *C, int64_t sci, int64_t scj, int nz, float *partial, hipStream_t st);
-int fbk_mlp_bias_act(int64_t n, float *Z, float *A, const float *b, hipStream_t st);
-int fbk_mlp_out(int64_t n, int nme, float *Y, const float *b3, const float *T, float *dY, float *rowloss,
-                float inv_count, hipStream_t st);
-int fbk_mlp_act_back(int64_t n, const float *dA, const float *Z, float *dZ, hipStream_t st);
 int fbk_mlp_adam(int np, float *p, const float *g, float *m, float *v, float lr, float b1, float b2, float c1,
                  float c2, float eps, hipStream_t st);
 int fbk_mlp_infer(const DMlp *w, int64_t n, const float *X, float *Y, hipStream_t st);
-int fbk_mlp_loss(int64_t n, const float *rowloss, float scale, float *loss, hipStream_t st);
+int fbk_mlp_pass(int64_t n, int nme, float inv_count, const float *P, const float *X, const float *T, float *part,
+                 float *rowloss, float *grads, float loss_scale, float *loss, hipStream_t st);
 int fbk_mlp_calib(const DView &v, int gid, const DMlp *w, int64_t n, unsigned long long seed, unsigned *err,
                   hipStream_t st);
 }
@@ -212,7 +207,8 @@ bool same_list(const MeList &a, const std::vector<int> &mu, const std::vector<in
 
 struct fb_ctx {
   int device = 0;
-  float *scratch = nullptr;   // this device's scratch array (fb_mlp_gradients_noalloc)
+  float *scratch = nullptr;   // this context's part of the device's scratch array (fb_mlp_gradients_noalloc)
+  int scratch_slot = -1;
   int ncu = 256;              // compute units of the device
   int fused = 0;              // FB_TUNE_FUSED: 0 separate 2c/3c launches, 3 or 4 one launch (waves per SIMD)
   int persist = 0;            // FB_TUNE_PERSIST: the one launch's 3c waves take tiles from a queue
@@ -650,28 +646,26 @@ extern "C" {
 // why the last fb_create of this thread failed (fb_last_error(NULL) returns it)
 // ---------------------------------------------- scratch of the allocation-free entry point
 // fb_mlp_gradients_noalloc keeps the work arrays of one training batch (the
-// MlpWork arrays for FB_MLP_NOALLOC_MAX_BATCH samples, laid out at fixed
+// partial gradients and the losses of FB_MLP_NOALLOC_MAX_BATCH rows, at fixed
 // offsets) in this file-scope device array instead of allocating them.  Each
-// GPU holds its own copy until the process ends.  The host never passes the
-// array's name to a kernel: fb_create looks up its device address once per
-// device (with that device current) and every use goes through that address.
+// GPU holds its own copy until the process ends, in NA_SLOTS parts: a context
+// takes the least used part for its lifetime, so that up to NA_SLOTS contexts
+// of a GPU do not share one.  The host never passes the array's name to a
+// kernel: fb_create looks up its device address once per device (with that
+// device current) and every use goes through that address.
 namespace {
-constexpr int64_t NA_B = FB_MLP_NOALLOC_MAX_BATCH;
-constexpr int64_t NA_HID = NA_B * MLP_H;            // floats of one [B][64] array
-constexpr int64_t NA_OFF_Y = 7 * NA_HID;            // Z1, A1, Z2, A2, dA, dZ2, dZ1 first
-constexpr int64_t NA_OFF_DY = NA_OFF_Y + NA_B * MLP_O;
-constexpr int64_t NA_OFF_ROW = NA_OFF_DY + NA_B * MLP_O;
-constexpr int64_t NA_OFF_PART = NA_OFF_ROW + NA_B;
-constexpr int64_t NA_OFF_ONES = NA_OFF_PART + 64LL * MLP_H * MLP_O;
-constexpr int64_t NA_FLOATS = NA_OFF_ONES + 64;     // ones[1], padded to 256 bytes
+constexpr int64_t NA_OFF_ROW = (int64_t)MLP_PARTS * MLP_NP;
+constexpr int64_t NA_FLOATS = NA_OFF_ROW + FB_MLP_NOALLOC_MAX_BATCH;
+constexpr int NA_SLOTS = 4;
 constexpr int NA_MAXDEV = 64;
 std::mutex g_scratch_mu;
 float *g_scratch_dev[NA_MAXDEV] = {};
+int g_scratch_use[NA_MAXDEV][NA_SLOTS] = {};
 }  // namespace
-static __device__ __align__(256) float scratch[NA_FLOATS];
+static __device__ __align__(256) float scratch[NA_SLOTS * NA_FLOATS];
 
-// device address of this GPU's scratch array; the device must be current
-static hipError_t scratch_address(int device, float **out) {
+// a part of this GPU's scratch array for a context; the device must be current
+static hipError_t scratch_take(int device, int *slot, float **out) {
   if (device < 0 || device >= NA_MAXDEV) return hipErrorInvalidDevice;
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   if (!g_scratch_dev[device]) {
@@ -680,13 +674,22 @@ static hipError_t scratch_address(int device, float **out) {
     if (e != hipSuccess) return e;
     g_scratch_dev[device] = static_cast<float *>(ptr);
   }
-  *out = g_scratch_dev[device];
+  int *const use = g_scratch_use[device];
+  *slot = (int)(std::min_element(use, use + NA_SLOTS) - use);
+  use[*slot]++;
+  *out = g_scratch_dev[device] + *slot * NA_FLOATS;
   return hipSuccess;
+}
+
+static void scratch_give(int device, int slot) {
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  g_scratch_use[device][slot]--;
 }
 
 static thread_local std::string g_create_err = "null context";
 
 static int create_failed(fb_ctx *ctx, const char *what, hipError_t e) {
+  if (ctx->scratch_slot >= 0) scratch_give(ctx->device, ctx->scratch_slot);
   delete ctx;
   g_create_err = std::string("fb_create: ") + what + ": " + hipGetErrorString(e);
   return FB_E_HIP;
@@ -704,7 +707,7 @@ int fb_create(fb_ctx **out, int device) {
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming);
   if (e != hipSuccess) return create_failed(ctx, "streams", e);
-  e = scratch_address(device, &ctx->scratch);
+  e = scratch_take(device, &ctx->scratch_slot, &ctx->scratch);
   if (e != hipSuccess) return create_failed(ctx, "scratch address", e);
   e = hipDeviceGetAttribute(&ctx->ncu, hipDeviceAttributeMultiprocessorCount, device);
   if (e != hipSuccess) return create_failed(ctx, "device attributes", e);
@@ -722,6 +725,7 @@ int fb_destroy(fb_ctx *ctx) {
   if (!ctx) return FB_E_ARG;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  scratch_give(ctx->device, ctx->scratch_slot);
   delete ctx;
   return FB_OK;
 }
@@ -2032,24 +2036,12 @@ int fb_gamma_eigenvalues(fb_ctx *ctx, int is, int which, double *w, int64_t nw, 
 // ------------------------------------------------------- learned 3c surrogate
 namespace {
 
-// work arrays of one forward + backward pass over a batch of B samples:
-// Z1, A1, Z2, A2, dA, dZ2, dZ1 [B][64], Y, dY [B][64], rowloss [B], part
-// [64][64][64] (split-K partial products), ones [1] = 1.0f
-struct MlpWork {
-  float *Z1, *A1, *Z2, *A2, *Y, *dY, *dA, *dZ2, *dZ1, *rowloss, *part;
-  const float *ones;
-};
-
+// buffers of training and of fb_mlp_gradients; rowloss [B] and part
+// [MLP_PARTS][MLP_NP] are the work arrays of a pass
 struct MlpBufs {
-  DevBuf X, T, osc, inv, Z1, A1, Z2, A2, Y, dY, dA, dZ2, dZ1, rowloss, P, G, M, V, part, ones;
-  MlpWork work() {
-    return MlpWork{Z1.as<float>(), A1.as<float>(), Z2.as<float>(), A2.as<float>(), Y.as<float>(), dY.as<float>(),
-                   dA.as<float>(), dZ2.as<float>(), dZ1.as<float>(), rowloss.as<float>(), part.as<float>(),
-                   ones.as<float>()};
-  }
+  DevBuf X, T, osc, inv, rowloss, P, G, M, V, part;
   ~MlpBufs() {
-    DevBuf *b[] = {&X, &T, &osc, &inv, &Z1, &A1, &Z2, &A2, &Y, &dY, &dA, &dZ2, &dZ1, &rowloss, &P, &G, &M, &V, &part,
-                   &ones};
+    DevBuf *b[] = {&X, &T, &osc, &inv, &rowloss, &P, &G, &M, &V, &part};
     for (DevBuf *x : b) x->release();
   }
 };
@@ -2061,58 +2053,27 @@ struct MlpBufs {
   } while (0)
 
 int mlp_alloc_batch(fb_ctx *ctx, MlpBufs &b, int64_t B) {
-  const size_t h = sizeof(float) * (size_t)B * MLP_H, o = sizeof(float) * (size_t)B * MLP_O;
-  hipError_t e = hipSuccess;
-  DevBuf *hb[] = {&b.Z1, &b.A1, &b.Z2, &b.A2, &b.dA, &b.dZ2, &b.dZ1};
-  for (DevBuf *x : hb)
-    if (e == hipSuccess) e = x->ensure(h);
-  if (e == hipSuccess) e = b.Y.ensure(o);
-  if (e == hipSuccess) e = b.dY.ensure(o);
-  if (e == hipSuccess) e = b.rowloss.ensure(sizeof(float) * (size_t)B);
+  hipError_t e = b.rowloss.ensure(sizeof(float) * (size_t)B);
   if (e == hipSuccess) e = b.P.ensure(sizeof(float) * MLP_NP);
   if (e == hipSuccess) e = b.G.ensure(sizeof(float) * MLP_NP);
-  if (e == hipSuccess) e = b.part.ensure(sizeof(float) * 64 * MLP_H * MLP_O);
-  if (e == hipSuccess) e = b.ones.ensure(sizeof(float));
+  if (e == hipSuccess) e = b.part.ensure(sizeof(float) * MLP_PARTS * MLP_NP);
   if (e != hipSuccess) return ctx->fail(FB_E_HIP, "network buffers", e);
-  const float one = 1.0f;
-  FB_HIP(hipMemcpyAsync(b.ones.p, &one, sizeof(float), hipMemcpyHostToDevice, ctx->stream));
   return FB_OK;
 }
 
 // forward + backward of one batch (X [B][3], T [B][64]) with parameters P;
-// gradients into G, per-row losses into w.rowloss.  Every array of w is
-// written before it is read, so the work area needs no clearing.
-int mlp_fwd_bwd(fb_ctx *ctx, const MlpWork &w, const float *P, float *G, int nme, int64_t B, const float *X,
-                const float *T) {
-  hipStream_t st = ctx->stream;
-  float *Z1 = w.Z1, *A1 = w.A1, *Z2 = w.Z2, *A2 = w.A2, *Y = w.Y, *dY = w.dY, *dA = w.dA;
-  float *dZ2 = w.dZ2, *dZ1 = w.dZ1, *part = w.part;
-  const float *ones = w.ones;
-  const int Bi = (int)B;
-  const int nz = (int)std::min<int64_t>(64, std::max<int64_t>(1, B / 256));
+// gradients into G, per-row losses into rowloss and, unless null, the mean
+// batch loss into loss.  The work arrays are written before they are read, so
+// they need no clearing.
+int mlp_fwd_bwd(fb_ctx *ctx, float *part, float *rowloss, const float *P, float *G, int nme, int64_t B, const float *X,
+                const float *T, float *loss = nullptr) {
   int nvalid = 0;
   for (int o = 0; o < MLP_O; o++) {
     int th, m;
     nvalid += mlp_slot(o, nme, &th, &m) ? 1 : 0;
   }
-  // forward
-  MLP_RC(fbk_mlp_gemm(Bi, MLP_H, MLP_IN, X, MLP_IN, 1, P + MLP_P_W1, 1, MLP_IN, Z1, MLP_H, 1, 1, nullptr, st));
-  MLP_RC(fbk_mlp_bias_act(B, Z1, A1, P + MLP_P_B1, st));
-  MLP_RC(fbk_mlp_gemm(Bi, MLP_H, MLP_H, A1, MLP_H, 1, P + MLP_P_W2, 1, MLP_H, Z2, MLP_H, 1, 1, nullptr, st));
-  MLP_RC(fbk_mlp_bias_act(B, Z2, A2, P + MLP_P_B2, st));
-  MLP_RC(fbk_mlp_gemm(Bi, MLP_O, MLP_H, A2, MLP_H, 1, P + MLP_P_W3, 1, MLP_H, Y, MLP_O, 1, 1, nullptr, st));
-  MLP_RC(fbk_mlp_out(B, nme, Y, P + MLP_P_B3, T, dY, w.rowloss, 1.0f / ((float)B * (float)nvalid), st));
-  // backward
-  MLP_RC(fbk_mlp_gemm(MLP_O, MLP_H, Bi, dY, 1, MLP_O, A2, MLP_H, 1, G + MLP_P_W3, MLP_H, 1, nz, part, st));
-  MLP_RC(fbk_mlp_gemm(1, MLP_O, Bi, ones, 0, 0, dY, MLP_O, 1, G + MLP_P_B3, MLP_O, 1, nz, part, st));
-  MLP_RC(fbk_mlp_gemm(Bi, MLP_H, MLP_O, dY, MLP_O, 1, P + MLP_P_W3, MLP_H, 1, dA, MLP_H, 1, 1, nullptr, st));
-  MLP_RC(fbk_mlp_act_back(B, dA, Z2, dZ2, st));
-  MLP_RC(fbk_mlp_gemm(MLP_H, MLP_H, Bi, dZ2, 1, MLP_H, A1, MLP_H, 1, G + MLP_P_W2, MLP_H, 1, nz, part, st));
-  MLP_RC(fbk_mlp_gemm(1, MLP_H, Bi, ones, 0, 0, dZ2, MLP_H, 1, G + MLP_P_B2, MLP_H, 1, nz, part, st));
-  MLP_RC(fbk_mlp_gemm(Bi, MLP_H, MLP_H, dZ2, MLP_H, 1, P + MLP_P_W2, MLP_H, 1, dA, MLP_H, 1, 1, nullptr, st));
-  MLP_RC(fbk_mlp_act_back(B, dA, Z1, dZ1, st));
-  MLP_RC(fbk_mlp_gemm(MLP_H, MLP_IN, Bi, dZ1, 1, MLP_H, X, MLP_IN, 1, G + MLP_P_W1, MLP_IN, 1, nz, part, st));
-  MLP_RC(fbk_mlp_gemm(1, MLP_H, Bi, ones, 0, 0, dZ1, MLP_H, 1, G + MLP_P_B1, MLP_H, 1, nz, part, st));
+  const float inv = 1.0f / ((float)B * (float)nvalid);
+  MLP_RC(fbk_mlp_pass(B, nme, inv, P, X, T, part, rowloss, G, inv, loss, ctx->stream));
   return FB_OK;
 }
 
@@ -2291,7 +2252,7 @@ int fb_mlp_train(fb_ctx *ctx, int64_t nsamples, int nsteps, int batch, double lr
     double loss0 = -1.0, loss = -1.0;
     for (int step = 0; step < nsteps; step++) {
       const int64_t off = (step % nb) * batch;
-      RC(mlp_fwd_bwd(ctx, b.work(), b.P.as<float>(), b.G.as<float>(), g.nME, batch, b.X.as<float>() + off * MLP_IN,
+      RC(mlp_fwd_bwd(ctx, b.part.as<float>(), b.rowloss.as<float>(), b.P.as<float>(), b.G.as<float>(), g.nME, batch, b.X.as<float>() + off * MLP_IN,
                      b.T.as<float>() + off * MLP_O));
       if (step == 0) loss0 = mlp_batch_loss(ctx, b, g.nME, batch);
       const double lr_t = lr * (0.01 + 0.99 * 0.5 * (1.0 + std::cos(M_PI * step / nsteps)));
@@ -2300,7 +2261,7 @@ int fb_mlp_train(fb_ctx *ctx, int64_t nsamples, int nsteps, int batch, double lr
                           (float)b1, (float)b2, (float)c1, (float)c2, 1e-8f, ctx->stream));
     }
     // loss of the trained network on the first batch
-    RC(mlp_fwd_bwd(ctx, b.work(), b.P.as<float>(), b.G.as<float>(), g.nME, batch, b.X.as<float>(), b.T.as<float>()));
+    RC(mlp_fwd_bwd(ctx, b.part.as<float>(), b.rowloss.as<float>(), b.P.as<float>(), b.G.as<float>(), g.nME, batch, b.X.as<float>(), b.T.as<float>()));
     loss = mlp_batch_loss(ctx, b, g.nME, batch);
     FB_HIP(hipMemcpy(p.data(), b.P.p, sizeof(float) * MLP_NP, hipMemcpyDeviceToHost));
     ctx->h_mlp_params[gid] = p;
@@ -2437,7 +2398,7 @@ int fb_mlp_gradients(fb_ctx *ctx, int nme, const float *params, int n, const flo
   FB_HIP(hipMemcpyAsync(b.P.p, params, sizeof(float) * MLP_NP, hipMemcpyHostToDevice, ctx->stream));
   FB_HIP(hipMemcpyAsync(b.X.p, X, sizeof(float) * (size_t)n * MLP_IN, hipMemcpyHostToDevice, ctx->stream));
   FB_HIP(hipMemcpyAsync(b.T.p, T, sizeof(float) * (size_t)n * MLP_O, hipMemcpyHostToDevice, ctx->stream));
-  RC(mlp_fwd_bwd(ctx, b.work(), b.P.as<float>(), b.G.as<float>(), nme, n, b.X.as<float>(), b.T.as<float>()));
+  RC(mlp_fwd_bwd(ctx, b.part.as<float>(), b.rowloss.as<float>(), b.P.as<float>(), b.G.as<float>(), nme, n, b.X.as<float>(), b.T.as<float>()));
   const double l = mlp_batch_loss(ctx, b, nme, n);
   if (loss) *loss = l;
   FB_HIP(hipMemcpy(grads, b.G.p, sizeof(float) * MLP_NP, hipMemcpyDeviceToHost));
@@ -2456,21 +2417,7 @@ int fb_mlp_gradients_noalloc(fb_ctx *ctx, int nme, const float *params, int n, c
     return ctx->fail(FB_E_CAPACITY, "mlp_gradients_noalloc: batch larger than FB_MLP_NOALLOC_MAX_BATCH (2048)");
   FB_HIP(hipSetDevice(ctx->device));
   float *const sc = ctx->scratch;
-  const MlpWork w{sc, sc + NA_HID, sc + 2 * NA_HID, sc + 3 * NA_HID, sc + NA_OFF_Y, sc + NA_OFF_DY,
-                  sc + 4 * NA_HID, sc + 5 * NA_HID, sc + 6 * NA_HID, sc + NA_OFF_ROW, sc + NA_OFF_PART,
-                  sc + NA_OFF_ONES};
-  // 1.0f, written by a kernel (no host copy, nothing a graph replays wrongly)
-  int rc = fbk_fill_i32(reinterpret_cast<int *>(sc + NA_OFF_ONES), 1, 0x3f800000, ctx->stream);
-  if (rc) return ctx->fail(FB_E_HIP, "mlp_gradients_noalloc fill", (hipError_t)rc);
-  RC(mlp_fwd_bwd(ctx, w, params, grads, nme, n, X, T));
-  int nvalid = 0;
-  for (int o = 0; o < MLP_O; o++) {
-    int th, m;
-    nvalid += mlp_slot(o, nme, &th, &m) ? 1 : 0;
-  }
-  rc = fbk_mlp_loss(n, w.rowloss, 1.0f / ((float)n * (float)nvalid), loss, ctx->stream);
-  if (rc) return ctx->fail(FB_E_HIP, "mlp_gradients_noalloc loss", (hipError_t)rc);
-  return FB_OK;
+  return mlp_fwd_bwd(ctx, sc, sc + NA_OFF_ROW, params, grads, nme, n, X, T, loss);
 }
 
 int fb_mlp_forward(fb_ctx *ctx, int nme, const float *params, const float *oscale, int n, const float *X, float *Y) {

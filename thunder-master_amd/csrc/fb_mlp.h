@@ -49,6 +49,7 @@
 #define MLP_P_W3 (MLP_P_B2 + MLP_H)
 #define MLP_P_B3 (MLP_P_W3 + MLP_O * MLP_H)
 #define MLP_NP (MLP_P_B3 + MLP_O)   // 8576 FP32 parameters
+#define MLP_PARTS 128               // partial gradients of a training pass, at most
 #define MLP_CSUB 4                  // calibration sub-cells per table cell and direction
 
 typedef short mlp_s4 __attribute__((ext_vector_type(4)));

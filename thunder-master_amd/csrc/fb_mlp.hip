@@ -8,6 +8,8 @@
 // of theta cell 1 is below 1e-6, bicubic otherwise).
 #include "fb_mlp.h"
 
+#include <algorithm>
+
 // ---------------------------------------------------------------- samples
 __device__ inline unsigned long long mlp_mix(unsigned long long z) {
   z += 0x9e3779b97f4a7c15ull;
@@ -135,95 +137,191 @@ __global__ __launch_bounds__(256) void k_scale_cols(int64_t n, int ncol, float *
     A[e] *= inv[e % ncol];
 }
 
-// ---------------------------------------------------------------- FP32 GEMM
-// C(i, j) = sum_k A(i, k) B(k, j) over the k range of split z; strides in
-// elements; split z writes C + z*scz.  32x32 tiles, 256 threads, 2x2 each.
-struct MlpGemm {
-  int M, N, K, kchunk;
-  const float *A;
-  int64_t sai, sak;
-  const float *B;
-  int64_t sbk, sbj;
-  float *C;
-  int64_t sci, scj, scz;
-};
+// ---------------------------------------------------------------- FP32 training pass
+// Forward and backward of one batch.  A workgroup takes tiles of 16 rows
+// through the whole network: both 64 x 64 weight matrices and the rows'
+// activations stay in LDS, every product runs on v_mfma_f32_16x16x4_f32
+// (FP32 operands and sums), and the weight gradients of its tiles add up in
+// accumulator registers.  It writes one partial gradient; k_mlp_sum adds the
+// partials in workgroup order, so the result is the same run to run.
+//
+// The work is 105 MFLOP for 2048 rows: the bound is the chain of launches and,
+// within them, of LDS round trips.  As 24 launches (one per product, bias,
+// activation and split sum) the pass took 82 us with passes in flight and
+// 241 us alone; as these two it takes 7.4 us and 25 us.  Tiles of 16 rows, the
+// smallest of the instruction, give 2048 rows 128 workgroups.
+//
+// Lane layout (l = lane, r = l % 16, g = l / 16, wave w): a wavefront owns
+// units 16w .. 16w + 15 of every layer.  An accumulator holds rows 4g + j of
+// unit 16w + r; as the A operand of a weight gradient the same registers are
+// (unit r, row index g), so the row gradients feed it in place.  A contraction
+// index is free, so step j of a group of four takes k = 4g + j of 16: one
+// 16-byte LDS read feeds four instructions.
+#define MLP_ROWS 16
+#define MLP_LD 68   // LDS row of 64 units: 16-byte reads stay aligned, columns do not share banks
 
-__global__ __launch_bounds__(256) void k_mlp_gemm(MlpGemm g) {
-  __shared__ float As[32][33], Bs[32][33];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32;
-  const int kb = blockIdx.z * g.kchunk, ke = min(g.K, kb + g.kchunk);
-  float c00 = 0.f, c01 = 0.f, c10 = 0.f, c11 = 0.f;
-  for (int k = kb; k < ke; k += 32) {
-    for (int e = tid; e < 1024; e += 256) {
-      const int r = e >> 5, cc = e & 31;
-      As[r][cc] = (i0 + r < g.M && k + cc < ke) ? g.A[(int64_t)(i0 + r) * g.sai + (int64_t)(k + cc) * g.sak] : 0.f;
-      Bs[r][cc] = (k + r < ke && j0 + cc < g.N) ? g.B[(int64_t)(k + r) * g.sbk + (int64_t)(j0 + cc) * g.sbj] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (int kk = 0; kk < 32; kk++) {
-      const float a0 = As[2 * ty][kk], a1 = As[2 * ty + 1][kk];
-      const float b0 = Bs[kk][2 * tx], b1 = Bs[kk][2 * tx + 1];
-      c00 = __builtin_fmaf(a0, b0, c00);
-      c01 = __builtin_fmaf(a0, b1, c01);
-      c10 = __builtin_fmaf(a1, b0, c10);
-      c11 = __builtin_fmaf(a1, b1, c11);
-    }
-    __syncthreads();
+typedef float mlp_v4 __attribute__((ext_vector_type(4)));
+
+// c += A[16 rows][64] (rows of s) times the 64 x 16 operand whose element
+// (k, unit r) is b(k)
+template <typename B>
+__device__ __forceinline__ mlp_v4 mlp_rows64(const float (*s)[MLP_LD], int r, int g, B b) {
+  mlp_v4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const mlp_v4 a = *reinterpret_cast<const mlp_v4 *>(&s[r][16 * q + 4 * g]);
+    const mlp_v4 x = b(16 * q + 4 * g);
+#pragma unroll
+    for (int j = 0; j < 4; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], x[j], c, 0, 0, 0);
   }
-  float *C = g.C + (int64_t)blockIdx.z * g.scz;
-  const int i = i0 + 2 * ty, j = j0 + 2 * tx;
-  if (i < g.M && j < g.N) C[i * g.sci + j * g.scj] = c00;
-  if (i < g.M && j + 1 < g.N) C[i * g.sci + (j + 1) * g.scj] = c01;
-  if (i + 1 < g.M && j < g.N) C[(i + 1) * g.sci + j * g.scj] = c10;
-  if (i + 1 < g.M && j + 1 < g.N) C[(i + 1) * g.sci + (j + 1) * g.scj] = c11;
+  return c;
 }
 
-// out[e] = sum_z P[z*n + e], z in order (deterministic split-K reduction)
-__global__ __launch_bounds__(256) void k_mlp_sumz(int64_t n, int nz, const float *P, float *out) {
-  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  float s = 0.f;
-  for (int z = 0; z < nz; z++) s += P[(int64_t)z * n + e];
-  out[e] = s;
+__global__ __launch_bounds__(256) void k_mlp_pass(int64_t n, int nme, const float *P, const float *X, const float *T,
+                                                  float inv_count, float *part, float *rowloss) {
+  __shared__ __align__(16) float sW2[MLP_H][MLP_LD], sW3[MLP_O][MLP_LD];
+  __shared__ __align__(16) float sA1[MLP_ROWS][MLP_LD], sA2[MLP_ROWS][MLP_LD], sD[MLP_ROWS][MLP_LD];
+  __shared__ float sX[MLP_ROWS][4], sL[4][MLP_ROWS];
+  const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, r = l & 15, g = l >> 4;
+  const int u = 16 * w + r;   // this lane's unit
+  for (int e = tid; e < MLP_H * MLP_H; e += 256) {
+    sW2[e >> 6][e & 63] = P[MLP_P_W2 + e];
+    sW3[e >> 6][e & 63] = P[MLP_P_W3 + e];
+  }
+  const float w1[3] = {P[MLP_P_W1 + 3 * u], P[MLP_P_W1 + 3 * u + 1], P[MLP_P_W1 + 3 * u + 2]};
+  const float b1 = P[MLP_P_B1 + u], b2 = P[MLP_P_B2 + u], b3 = P[MLP_P_B3 + u];
+  int th, me;
+  const bool valid = mlp_slot(u, nme, &th, &me);
+  mlp_v4 g3[4] = {}, g2[4] = {};
+  float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, g1[3] = {0.f, 0.f, 0.f};
+  const int64_t ntile = (n + MLP_ROWS - 1) / MLP_ROWS;
+  for (int64_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+    const int64_t row0 = tile * MLP_ROWS;
+    __syncthreads();   // the previous tile's reads
+    if (tid < 3 * MLP_ROWS) sX[tid / 3][tid % 3] = row0 + tid / 3 < n ? X[row0 * MLP_IN + tid] : 0.f;
+    float t[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) t[j] = row0 + 4 * g + j < n ? T[(row0 + 4 * g + j) * MLP_O + u] : 0.f;
+    __syncthreads();
+    mlp_v4 z1, z2, d, c;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float *x = sX[4 * g + j];
+      z1[j] = __builtin_fmaf(x[2], w1[2], __builtin_fmaf(x[1], w1[1], x[0] * w1[0])) + b1;
+      sA1[4 * g + j][u] = mlp_act(z1[j]);
+    }
+    __syncthreads();
+    z2 = mlp_rows64(sA1, r, g, [&](int k) { return *reinterpret_cast<const mlp_v4 *>(&sW2[u][k]); });
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      z2[j] += b2;
+      sA2[4 * g + j][u] = mlp_act(z2[j]);
+    }
+    __syncthreads();
+    c = mlp_rows64(sA2, r, g, [&](int k) { return *reinterpret_cast<const mlp_v4 *>(&sW3[u][k]); });
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float e = (valid && row0 + 4 * g + j < n) ? c[j] + b3 - t[j] : 0.f;
+      d[j] = 2.0f * e * inv_count;
+      sD[4 * g + j][u] = d[j];
+      float s = e * e;
+#pragma unroll
+      for (int x = 1; x < 16; x <<= 1) s += __shfl_xor(s, x);
+      if (r == 0) sL[w][4 * g + j] = s;
+    }
+    __syncthreads();
+    if (tid < MLP_ROWS && row0 + tid < n) rowloss[row0 + tid] = ((sL[0][tid] + sL[1][tid]) + sL[2][tid]) + sL[3][tid];
+    // output layer
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      gb3 += d[j];
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        g3[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[j], sA2[4 * g + j][16 * q + r], g3[q], 0, 0, 0);
+    }
+    c = mlp_rows64(sD, r, g, [&](int k) { return mlp_v4{sW3[k][u], sW3[k + 1][u], sW3[k + 2][u], sW3[k + 3][u]}; });
+#pragma unroll
+    for (int j = 0; j < 4; j++) d[j] = c[j] * mlp_dact(z2[j]);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++) sD[4 * g + j][u] = d[j];
+    __syncthreads();
+    // second layer
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      gb2 += d[j];
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        g2[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[j], sA1[4 * g + j][16 * q + r], g2[q], 0, 0, 0);
+    }
+    c = mlp_rows64(sD, r, g, [&](int k) { return mlp_v4{sW2[k][u], sW2[k + 1][u], sW2[k + 2][u], sW2[k + 3][u]}; });
+    // first layer
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float e = c[j] * mlp_dact(z1[j]);
+      gb1 += e;
+#pragma unroll
+      for (int k = 0; k < 3; k++) g1[k] = __builtin_fmaf(e, sX[4 * g + j][k], g1[k]);
+    }
+  }
+  float *out = part + (int64_t)blockIdx.x * MLP_NP;
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      out[MLP_P_W3 + (16 * w + 4 * g + j) * MLP_H + 16 * q + r] = g3[q][j];
+      out[MLP_P_W2 + (16 * w + 4 * g + j) * MLP_H + 16 * q + r] = g2[q][j];
+    }
+  // the row groups g of a unit
+  auto rows = [&](float x) {
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+  };
+  gb1 = rows(gb1);
+  gb2 = rows(gb2);
+  gb3 = rows(gb3);
+#pragma unroll
+  for (int k = 0; k < 3; k++) g1[k] = rows(g1[k]);
+  if (g == 0) {
+    out[MLP_P_B1 + u] = gb1;
+    out[MLP_P_B2 + u] = gb2;
+    out[MLP_P_B3 + u] = gb3;
+#pragma unroll
+    for (int k = 0; k < 3; k++) out[MLP_P_W1 + 3 * u + k] = g1[k];
+  }
 }
+
+// grads[e] = sum over the partial gradients (four ranges of them side by
+// side, added in order); the last workgroup, when asked, the mean batch loss
+// from the row losses (lane-strided sums, then a fixed tree)
+__global__ __launch_bounds__(256) void k_mlp_sum(int npart, const float *part, float *grads, int64_t n,
+                                                 const float *rowloss, float scale, float *loss) {
+  __shared__ float s[256];
+  const int tid = threadIdx.x;
+  if (blockIdx.x == MLP_NP / 64) {
+    float a = 0.f;
+    for (int64_t i = tid; i < n; i += 256) a += rowloss[i];
+    s[tid] = a;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+      if (tid < h) s[tid] += s[tid + h];
+      __syncthreads();
+    }
+    if (tid == 0) loss[0] = s[0] * scale;
+    return;
+  }
+  const int e = blockIdx.x * 64 + (tid & 63), q = tid >> 6, per = (npart + 3) / 4;
+  const int z1 = min(npart, (q + 1) * per);
+  float a = 0.f;
+#pragma unroll 8
+  for (int z = q * per; z < z1; z++) a += part[(int64_t)z * MLP_NP + e];
+  s[tid] = a;
+  __syncthreads();
+  if (q == 0) grads[e] = ((s[tid] + s[64 + tid]) + s[128 + tid]) + s[192 + tid];
+}
+static_assert(MLP_NP % 64 == 0, "k_mlp_sum covers the gradient in whole workgroups");
 
 // ---------------------------------------------------------------- elementwise
-// Z[i][h] += b[h]; A = a(Z)
-__global__ __launch_bounds__(256) void k_mlp_bias_act(int64_t n, float *Z, float *A, const float *b) {
-  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e >= n * MLP_H) return;
-  const float z = Z[e] + b[e % MLP_H];
-  Z[e] = z;
-  A[e] = mlp_act(z);
-}
-
-// Y += b3; dY = 2 mask (Y - T) / (n nvalid); rowloss[i] = sum mask (Y - T)^2
-__global__ __launch_bounds__(256) void k_mlp_out(int64_t n, int nme, float *Y, const float *b3, const float *T,
-                                                 float *dY, float *rowloss, float inv_count) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float l = 0.f;
-  for (int o = 0; o < MLP_O; o++) {
-    int th, m;
-    const bool valid = mlp_slot(o, nme, &th, &m);
-    const float y = Y[i * MLP_O + o] + b3[o];
-    Y[i * MLP_O + o] = y;
-    const float d = valid ? y - T[i * MLP_O + o] : 0.f;
-    l = __builtin_fmaf(d, d, l);
-    dY[i * MLP_O + o] = 2.0f * d * inv_count;
-  }
-  rowloss[i] = l;
-}
-
-// dZ = dA * a'(Z)
-__global__ __launch_bounds__(256) void k_mlp_act_back(int64_t n, const float *dA, const float *Z, float *dZ) {
-  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e >= n * MLP_H) return;
-  dZ[e] = dA[e] * mlp_dact(Z[e]);
-}
-
 // Adam (bias-corrected), lr given per step by the host schedule
 __global__ __launch_bounds__(256) void k_mlp_adam(int np, float *p, const float *g, float *m, float *v, float lr,
                                                   float b1, float b2, float c1, float c2, float eps) {
@@ -302,27 +400,17 @@ __global__ __launch_bounds__(256) void k_mlp_calib(DView v, int gid, const DMlp 
   atomicMax(&err[mlp_subcell(x, y, g.xmax, g.ymax, g.nx, g.ny)], __float_as_uint((float)sqrt(e2)));
 }
 
-// Mean batch loss: one workgroup sums the per-row losses in a fixed order
-// (lane-strided partial sums, then a fixed tree), so the value is the same
-// run to run.
-__global__ __launch_bounds__(256) void k_mlp_loss(int64_t n, const float *rowloss, float scale, float *loss) {
-  __shared__ float part[256];
-  float a = 0.f;
-  for (int64_t i = threadIdx.x; i < n; i += 256) a += rowloss[i];
-  part[threadIdx.x] = a;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) loss[0] = part[0] * scale;
-}
-
 // ---------------------------------------------------------------- launchers
 extern "C" {
 
-int fbk_mlp_loss(int64_t n, const float *rowloss, float scale, float *loss, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_loss, dim3(1), dim3(256), 0, st, n, rowloss, scale, loss);
+// gradients of one batch into grads (part: MLP_PARTS partial gradients), the
+// rows' squared errors into rowloss and, unless null, their mean into loss
+int fbk_mlp_pass(int64_t n, int nme, float inv_count, const float *P, const float *X, const float *T, float *part,
+                 float *rowloss, float *grads, float loss_scale, float *loss, hipStream_t st) {
+  const int npart = (int)std::min<int64_t>((n + MLP_ROWS - 1) / MLP_ROWS, MLP_PARTS);
+  hipLaunchKernelGGL(k_mlp_pass, dim3(npart), dim3(256), 0, st, n, nme, P, X, T, inv_count, part, rowloss);
+  hipLaunchKernelGGL(k_mlp_sum, dim3(MLP_NP / 64 + (loss ? 1 : 0)), dim3(256), 0, st, npart, part, grads, n, rowloss,
+                     loss_scale, loss);
   return (int)hipGetLastError();
 }
 
@@ -350,47 +438,6 @@ int fbk_mlp_colmaxabs(int64_t n, int ncol, const float *A, float *out, hipStream
 
 int fbk_mlp_scale_cols(int64_t n, int ncol, float *A, const float *inv, hipStream_t st) {
   hipLaunchKernelGGL(k_scale_cols, dim3(4096), dim3(256), 0, st, n, ncol, A, inv);
-  return (int)hipGetLastError();
-}
-
-// C = A*B (M x N, inner K); nz > 1 splits K into partial products reduced in order
-int fbk_mlp_gemm(int M, int N, int K, const float *A, int64_t sai, int64_t sak, const float *B, int64_t sbk,
-                 int64_t sbj, float *C, int64_t sci, int64_t scj, int nz, float *partial, hipStream_t st) {
-  MlpGemm g{M, N, K, K, A, sai, sak, B, sbk, sbj, C, sci, scj, 0};
-  dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), 1);
-  // split partials are [z][M][N]: the reduced output must be row-major M x N
-  if (nz > 1 && (sci != N || scj != 1 || !partial)) return (int)hipErrorInvalidValue;
-  if (nz > 1) {
-    g.kchunk = ((K + nz - 1) / nz + 31) / 32 * 32;
-    nz = (K + g.kchunk - 1) / g.kchunk;
-    g.C = partial;
-    g.sci = N;
-    g.scj = 1;
-    g.scz = (int64_t)M * N;
-    grid.z = (unsigned)nz;
-    hipLaunchKernelGGL(k_mlp_gemm, grid, dim3(256), 0, st, g);
-    const int64_t n = (int64_t)M * N;
-    hipLaunchKernelGGL(k_mlp_sumz, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, nz, partial, C);
-  } else {
-    hipLaunchKernelGGL(k_mlp_gemm, grid, dim3(256), 0, st, g);
-  }
-  return (int)hipGetLastError();
-}
-
-int fbk_mlp_bias_act(int64_t n, float *Z, float *A, const float *b, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_bias_act, dim3((unsigned)((n * MLP_H + 255) / 256)), dim3(256), 0, st, n, Z, A, b);
-  return (int)hipGetLastError();
-}
-
-int fbk_mlp_out(int64_t n, int nme, float *Y, const float *b3, const float *T, float *dY, float *rowloss,
-                float inv_count, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_out, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, nme, Y, b3, T, dY, rowloss,
-                     inv_count);
-  return (int)hipGetLastError();
-}
-
-int fbk_mlp_act_back(int64_t n, const float *dA, const float *Z, float *dZ, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_act_back, dim3((unsigned)((n * MLP_H + 255) / 256)), dim3(256), 0, st, n, dA, Z, dZ);
   return (int)hipGetLastError();
 }
 

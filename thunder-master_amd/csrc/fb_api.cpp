@@ -967,6 +967,13 @@ int fb_commit_tables(fb_ctx *ctx) {
   };
   std::vector<double> tab3;
   std::vector<float> tab3f, tab3q;
+  // FP64 slab [iy][ix][ME][theta]: the theta cells arrive as [iy][ix][ME] each
+  auto append_theta = [](std::vector<double> &slab, const HCell3c *const *th) {
+    const size_t n = th[0]->data.size(), o = slab.size();
+    slab.resize(o + n * FB_NTHETA);
+    for (int t = 0; t < FB_NTHETA; t++)
+      for (size_t e = 0; e < n; e++) slab[o + e * FB_NTHETA + t] = th[t]->data[e];
+  };
   for (auto &kv : groups) {
     const HCell3c *th[FB_NTHETA] = {nullptr};
     for (auto *c : kv.second) th[c->itheta - 1] = c;
@@ -1005,7 +1012,7 @@ int fb_commit_tables(fb_ctx *ctx) {
     mu.insert(mu.end(), cl->mu.begin(), cl->mu.end());
     nu.insert(nu.end(), cl->nu.begin(), cl->nu.end());
     mv.insert(mv.end(), cl->mv.begin(), cl->mv.end());
-    for (int t = 0; t < FB_NTHETA; t++) tab3.insert(tab3.end(), th[t]->data.begin(), th[t]->data.end());
+    append_theta(tab3, th);
     method_table(g, th[0]->data.data());
     // FP32 slab [iy][ix][ME][theta]: the five values of one (point, ME) are
     // contiguous and load as one float4 + one float
@@ -1080,7 +1087,7 @@ int fb_commit_tables(fb_ctx *ctx) {
     mu.insert(mu.end(), cl->mu.begin(), cl->mu.end());
     nu.insert(nu.end(), cl->nu.begin(), cl->nu.end());
     mv.insert(mv.end(), cl->mv.begin(), cl->mv.end());
-    for (int t = 0; t < FB_NTHETA; t++) tab3.insert(tab3.end(), th[t]->data.begin(), th[t]->data.end());
+    append_theta(tab3, th);
     idx3r[((((size_t)(is - 1) * ns + (js - 1)) * ns + (ks - 1)) * 2 + (itype - 1)) * FB_MAXSUB3 + isub] =
         (int)grps.size();
     grps.push_back(g);

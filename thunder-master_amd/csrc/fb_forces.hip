@@ -478,8 +478,7 @@ __device__ inline int d_getD3c(const DView &v, int gid, double x, double y, doub
   if (iy > ny - 2) iy = ny - 2;
   const double px = x / dx - ix + 1.0, py = y / dy - iy + 1.0;
   const double *tab = v.tab3c + g.off;
-  const int64_t tstride = (int64_t)ny * nx * nME;
-#define T3F(th, i, j, m) tab[(th) * tstride + ((int64_t)((j) - 1) * nx + ((i) - 1)) * nME + (m)]
+#define T3F(th, i, j, m) tab[FB_T64(th, i, j, m, nx, nME)]
   const double gx = (T3F(0, ix + 1, iy, 0) - T3F(0, ix, iy, 0)) / dx;
   const double gy = (T3F(0, ix, iy + 1, 0) - T3F(0, ix, iy, 0)) / dy;
   const double gg = gx * gx + gy * gy;
@@ -1325,8 +1324,7 @@ __device__ __forceinline__ int dgetD3c_sp(const DView &v, int gid, double x, dou
   if (iy > ny - 2) iy = ny - 2;
   const double px = x / dx - ix + 1.0, py = y / dy - iy + 1.0;
   const double *tab = v.tab3c + g.off;
-  const int64_t tstride = (int64_t)ny * nx * NME;
-#define T3S(th, i, j, m) tab[(th) * tstride + ((int64_t)((j) - 1) * nx + ((i) - 1)) * NME + (m)]
+#define T3S(th, i, j, m) tab[FB_T64(th, i, j, m, nx, NME)]
   const double gx = (T3S(0, ix + 1, iy, 0) - T3S(0, ix, iy, 0)) / dx;
   const double gy = (T3S(0, ix, iy + 1, 0) - T3S(0, ix, iy, 0)) / dy;
   const bool three = (gx * gx + gy * gy) < 1.0e-6;
@@ -1526,8 +1524,7 @@ __device__ inline int stage_q(const DView &v, int gid, int nme, double x, double
   if (iy > ny - 2) iy = ny - 2;
   const double px = x / dx - ix + 1.0, py = y / dy - iy + 1.0;
   const double *tab = v.tab3c + g.off;
-  const int64_t tstride = (int64_t)ny * nx * nme;
-#define T3Q_(th, i, j, m) tab[(th) * tstride + ((int64_t)((j) - 1) * nx + ((i) - 1)) * nme + (m)]
+#define T3Q_(th, i, j, m) tab[FB_T64(th, i, j, m, nx, nme)]
   const double gx = (T3Q_(0, ix + 1, iy, 0) - T3Q_(0, ix, iy, 0)) / dx;
   const double gy = (T3Q_(0, ix, iy + 1, 0) - T3Q_(0, ix, iy, 0)) / dy;
   const bool three = (gx * gx + gy * gy) < 1.0e-6;
@@ -1714,7 +1711,7 @@ __device__ inline int stage_q_mx(const DView &v, int gid, int nme, double x, dou
   if (three) {
     // the 3-point rule's slopes come from ME 1 of theta cell 1 (binary64 table)
     const double *tab = v.tab3c + g.off;
-#define T3X(i, j) tab[((int64_t)((j) - 1) * nx + ((i) - 1)) * nme]
+#define T3X(i, j) tab[FB_T64(0, i, j, 0, nx, nme)]
     const double gx = (T3X(ix + 1, iy) - T3X(ix, iy)) / dx;
     const double gy = (T3X(ix, iy + 1) - T3X(ix, iy)) / dy;
 #undef T3X

@@ -90,7 +90,7 @@ struct DGroup3c {
   int nq;            // ME quads of the FP32 quad slab, ceil(nME / 4)
   double xmax, ymax, dx, dy;
   double rdx, rdy;   // 1/dx, 1/dy
-  int64_t off;       // FP64 slab, layout [theta][ny][nx][nME]
+  int64_t off;       // FP64 slab, layout [ny][nx][nME][theta] (FB_T64)
   int64_t off32;     // FP32 slab, layout [ny][nx][ME][theta], FB_TH32 values per (point, ME)
   int64_t off32q;    // FP32 quad slab, layout [ny][nx][theta][4 nq] (MEs zero-padded to whole quads)
   int64_t moff;      // method table [ny][nx] (uint8, 1 = 3-point rule), e.FDATA/M_Fdata_3c.f90:383-385
@@ -122,6 +122,11 @@ struct TgtOut {
   int *seg_pair, *pair_tgt;
   int4 *tiles[3];
 };
+
+// value of (theta th, ix = i, iy = j, ME m) of a group in the FP64 slab; i and
+// j count from 1, th and m from 0
+#define FB_T64(th, i, j, m, nx, nME) \
+  ((((int64_t)((j) - 1) * (nx) + ((i) - 1)) * (nME) + (m)) * FB_NTHETA + (th))
 
 // all device pointers of a context, passed by value to kernels
 struct DView {

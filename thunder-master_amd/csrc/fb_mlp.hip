@@ -38,8 +38,7 @@ __device__ inline void mlp_interim(const DView &v, const DGroup3c &g, double x, 
   *piy = iy;
   const double px = x / dx - ix + 1.0, py = y / dy - iy + 1.0;
   const double *tab = v.tab3c + g.off;
-  const int64_t tstride = (int64_t)ny * nx * nME;
-#define T3D(th, i, j, m) tab[(th) * tstride + ((int64_t)((j) - 1) * nx + ((i) - 1)) * nME + (m)]
+#define T3D(th, i, j, m) tab[FB_T64(th, i, j, m, nx, nME)]
   const double gx = (T3D(0, ix + 1, iy, 0) - T3D(0, ix, iy, 0)) / dx;
   const double gy = (T3D(0, ix, iy + 1, 0) - T3D(0, ix, iy, 0)) / dy;
   const double gg = gx * gx + gy * gy;

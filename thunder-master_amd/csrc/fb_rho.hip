@@ -16,6 +16,7 @@
 // Binary64 throughout; no atomics, deterministic.
 #include "fb_device.h"
 #include "fb_3c_dev.h"
+#include "fb_3c_wave.h"
 
 #define NBR 16    // elements of one orbital or shell block of s/p species (at most 4 x 4)
 
@@ -471,264 +472,6 @@ __global__ __launch_bounds__(WRS, 2) void k_rho_2c_sp(DView v, int stride) {
   if (status) atomicOr(v.status, status);
 }
 
-// assemble_rho_3c / assemble_rho_weighted_3c for s/p species with canonical
-// density tables.  A workgroup of RW lanes owns whole target segments, packed
-// at list build into tiles of at most RT triplets (the mixed kernel's 64-triplet
-// tiles), and works through them in four phases:
-//   A  one lane per triplet: binary64 geometry (rho_geo), Legendre P0..P4 and
-//      sin(theta), and per shell isorp of the third atom the group, the grid
-//      cell, px, py, the method of the cell and Qin, into LDS.
-//   B  one lane per (triplet, isorp, matrix element): the interpolation of
-//      getMEs_3c_sp for that element -- the five theta cells in order, each
-//      with the 16-point form or the 3-point rule, summed with P_theta --
-//      times sin(theta) where mvalue = 1.
-//   C  one lane per (triplet, isorp): rotation (or the shell-block reorder of
-//      the weighted density) times Qin into the triplet's LDS row.
-//   D  one lane per (owned segment, block element): the rows added onto the
-//      two-centre block in list order, isorp inner, as the reference does.
-// Every element goes through the same binary64 operations in the same order
-// as the one-lane-per-triplet form, so the blocks are bit-identical to it.
-#define RT 64           // triplets per tile
-#define RW 256          // lanes per workgroup
-#define RSO 2           // shells of an s/p third atom
-
-struct RTri {           // per triplet
-  double p[5], sint, pm[9];
-  int cls, nsorp;
-};
-struct RShell {         // per (triplet, isorp)
-  double px, py, q;
-  int64_t base;         // FP64 slab index of stencil corner (ix-1, iy-1), theta cell 1, ME 1
-  int rs, ts, nme, m1;  // row and theta strides (elements), ME count (0: no table), 3-point rule
-};
-
-// the unweighted density at three waves per SIMD (140 VGPRs): at four its
-// binary64 rotation spills 48 bytes per lane, whose scratch traffic doubles
-// the kernel's HBM bytes for a 5 % shorter run; the weighted one fits four
-template <bool W>
-__global__ __launch_bounds__(RW) __attribute__((amdgpu_waves_per_eu(W ? 4 : 3))) void k_rho_3c_ph(DView v) {
-  constexpr int NMX = W ? 4 : 10;          // matrix elements per (triplet, isorp)
-  constexpr int NBX = W ? 4 : 16;          // block elements
-  constexpr int ROW = NBX + 1;             // LDS row stride (doubles)
-  constexpr size_t SZ_A = sizeof(RTri) * RT + sizeof(RShell) * RT * RSO + sizeof(double) * RT * RSO * NMX;
-  constexpr size_t SZ_R = sizeof(double) * RT * RSO * ROW;
-  __shared__ __align__(16) unsigned char sbuf[SZ_A > SZ_R ? SZ_A : SZ_R];
-  __shared__ int64_t sSeg[RT + 1], sBo[RT];
-  __shared__ int sNb[RT], sNs[RT];
-  RTri *sT = reinterpret_cast<RTri *>(sbuf);
-  RShell *sS = reinterpret_cast<RShell *>(sbuf + sizeof(RTri) * RT);
-  double *sF = reinterpret_cast<double *>(sbuf + sizeof(RTri) * RT + sizeof(RShell) * RT * RSO);
-  double *sR = reinterpret_cast<double *>(sbuf);   // rows, after phase C has read A and B
-  const int tid = threadIdx.x;
-  const int4 td = v.tiles[0][xcd_tile(blockIdx.x, gridDim.x)];
-  const int64_t first = td.x, last = td.y, r0 = td.z, r1 = td.w;
-  if (first > last) return;
-  const int nown = (int)(last - first + 1);
-  double *const out = v.mat[W ? FB_MAT_RHOW_IN : FB_MAT_RHO_IN];
-  const int64_t *const off = W ? v.wboff : v.boff;
-  for (int k = tid; k <= nown; k += RW) sSeg[k] = v.seg_off[first + k];
-  for (int k = tid; k < nown; k += RW) {
-    const int p = v.seg_pair[first + k];
-    const int64_t b0 = off[p];
-    sBo[k] = b0;
-    sNb[k] = (int)(off[p + 1] - b0);
-  }
-  int status = 0;
-  for (int64_t c0 = r0; c0 < r1; c0 += RT) {
-    const int nt = (int)min((int64_t)RT, r1 - c0);
-    // ---------------- phase A
-    if (tid < nt) {
-      const int4 tr = v.trip[c0 + tid];
-      const int in1 = v.imass[tr.y], in2 = v.imass[tr.z], indna = v.imass[tr.x];
-      RTri &T = sT[tid];
-      double x, z, cost;
-      rho_geo(v, tr, x, z, cost, T.pm);
-      d_legendre(cost, T.p, &T.sint);
-      T.cls = (v.sp.norb[in1 - 1] == 4 ? 2 : 0) + (v.sp.norb[in2 - 1] == 4 ? 1 : 0);
-      int nsorp = v.sp.nssh[indna - 1];
-      if (nsorp > RSO) {
-        status |= ST_NO_TABLE;
-        nsorp = RSO;
-      }
-      T.nsorp = nsorp;
-      sNs[tid] = nsorp;
-      for (int so = 0; so < nsorp; so++) {
-        RShell &S = sS[tid * RSO + so];
-        const int gid = group3c_r(v, in1, in2, indna, W ? 1 : 0, so + 1);
-        S.q = v.qin[tr.x * FB_MAXSH + so];
-        if (gid < 0) {
-          status |= ST_NO_TABLE;
-          S.nme = 0;
-          continue;
-        }
-        const DGroup3c g = v.grp3c[gid];
-        const int nx = g.nx, ny = g.ny;
-        // e.FDATA/M_Fdata_3c.f90:367-381, as getMEs_3c_sp
-        const double dx = g.xmax / (nx - 1.0), dy = g.ymax / (ny - 1.0);
-        int ix = (int)(x / dx) + 1, iy = (int)(z / dy) + 1;
-        if (ix < 2) ix = 2;
-        if (iy < 2) iy = 2;
-        if (ix > nx - 2) ix = nx - 2;
-        if (iy > ny - 2) iy = ny - 2;
-        S.px = x / dx - ix + 1.0;
-        S.py = z / dy - iy + 1.0;
-        S.nme = g.nME;
-        S.rs = nx * g.nME;
-        S.ts = ny * nx * g.nME;
-        S.base = g.off + ((int64_t)(iy - 2) * nx + (ix - 2)) * g.nME;
-        S.m1 = v.meth3c[g.moff + (int64_t)(iy - 1) * nx + (ix - 1)];
-      }
-    }
-    __syncthreads();
-    // ---------------- phase B
-    for (int it = tid; it < nt * RSO * NMX; it += RW) {
-      const int t = it / (RSO * NMX), r = it - t * (RSO * NMX), so = r / NMX, m = r - so * NMX;
-      const RTri &T = sT[t];
-      const RShell &S = sS[t * RSO + so];
-      if (so >= T.nsorp || m >= S.nme) continue;
-      const double px = S.px, py = S.py;
-      const int rs = S.rs, nm = S.nme;
-      const double *tab = v.tab3c + S.base + m;
-      double F = 0.0;
-#pragma unroll 1
-      for (int th = 0; th < FB_NTHETA; th++) {
-        const double *tt = tab + (int64_t)th * S.ts;
-        double interim;
-        if (S.m1) {
-          interim = ((1.0 - px - py) * tt[rs + nm] + px * tt[rs + 2 * nm]) + py * tt[2 * rs + nm];
-        } else {
-          double gk[4];
-#pragma unroll
-          for (int k = 0; k < 4; k++) {
-            const double *col = tt + k * nm;
-            double f1m1 = col[0];
-            double f1m2 = 2.0 * f1m1, f1m3 = 3.0 * f1m1;
-            double f0p3 = 3.0 * col[rs], f0p6 = 2.0 * f0p3;
-            double f1p3 = 3.0 * col[2 * rs], f1p6 = 2.0 * f1p3;
-            double f2p1 = col[3 * rs];
-            double bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-            double bb2 = f1m3 - f0p6 + f1p3;
-            double bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-            double bb0 = f0p6;
-            gk[k] = ((bb3 * py + bb2) * py + bb1) * py + bb0;
-          }
-          double f1m1 = gk[0], f1m2 = 2.0 * f1m1, f1m3 = 3.0 * f1m1;
-          double f0p3 = 3.0 * gk[1], f0p6 = 2.0 * f0p3;
-          double f1p3 = 3.0 * gk[2], f1p6 = 2.0 * f1p3;
-          double f2p1 = gk[3];
-          double bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-          double bb2 = f1m3 - f0p6 + f1p3;
-          double bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-          double bb0 = f0p6;
-          interim = (((bb3 * px + bb2) * px + bb1) * px + bb0) / 36.0;
-        }
-        F = F + T.p[th] * interim;
-      }
-      // sin(theta) on the mvalue = 1 elements: all but the leading 6 / 2 / 1
-      // of the canonical order (none in the weighted shell blocks)
-      if (!W && m >= (nm == 10 ? 6 : (nm == 3 ? 2 : 1))) F = F * T.sint;
-      sF[(t * RSO + so) * NMX + m] = F;
-    }
-    __syncthreads();
-    // ---------------- phase C
-    if (W) {
-      // shell blocks: one lane per (triplet, isorp)
-      double X[NBX];
-      int nbc = 0;
-      double q = 0.0;
-      const int tc = tid / RSO, soc = tid - tc * RSO;
-      if (tc < nt && soc < sT[tc].nsorp) {
-        const RShell &S = sS[tc * RSO + soc];
-        double F[NMX];
-#pragma unroll
-        for (int m = 0; m < NMX; m++) F[m] = (m < S.nme) ? sF[(tc * RSO + soc) * NMX + m] : 0.0;
-        q = S.q;
-        switch (sT[tc].cls) {
-          case 3: shell_block<2, 2>(F, X); nbc = 4; break;
-          case 2: shell_block<2, 1>(F, X); nbc = 2; break;
-          case 1: shell_block<1, 2>(F, X); nbc = 2; break;
-          default: shell_block<1, 1>(F, X); nbc = 1; break;
-        }
-        if (S.nme == 0) nbc = 0;
-      }
-      __syncthreads();   // phase A and B data read; the rows overwrite them
-      if (tc < nt && soc < RSO) {
-        double *row = sR + (tc * RSO + soc) * ROW;
-#pragma unroll
-        for (int i = 0; i < NBX; i++) row[i] = (i < nbc) ? X[i] * q : 0.0;
-      }
-    } else {
-      // rotated blocks: one lane per (triplet, isorp, block column), the
-      // elements of rot3c_sp one at a time (rot3c_el: same terms, same order)
-      constexpr int NCI = (RT * RSO * 4 + RW - 1) / RW;
-      double Xc[NCI][4];
-      int dst[NCI], nr[NCI];
-#pragma unroll
-      for (int k = 0; k < NCI; k++) {
-        const int it = tid + k * RW, pr = it >> 2, col = it & 3, tc = pr / RSO, soc = pr - tc * RSO;
-        dst[k] = -1;
-        nr[k] = 0;
-        if (tc < nt && soc < sT[tc].nsorp) {
-          const RTri &T = sT[tc];
-          const RShell &S = sS[pr];
-          const int cls = T.cls, nmu = (cls & 2) ? 4 : 1, nnu = (cls & 1) ? 4 : 1;
-          if (S.nme > 0 && col < nnu) {
-            double F[NMX], pm[9];
-#pragma unroll
-            for (int m = 0; m < NMX; m++) F[m] = (m < S.nme) ? sF[pr * NMX + m] : 0.0;
-#pragma unroll
-            for (int e = 0; e < 9; e++) pm[e] = T.pm[e];
-            const double q = S.q;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-              double x = 0.0;
-              if (r < nmu) {
-                switch (cls) {
-                  case 3: x = rot3c_el<3>(r, col, pm, F); break;
-                  case 2: x = rot3c_el<2>(r, col, pm, F); break;
-                  case 1: x = rot3c_el<1>(r, col, pm, F); break;
-                  default: x = rot3c_el<0>(r, col, pm, F); break;
-                }
-              }
-              Xc[k][r] = x * q;
-            }
-            dst[k] = pr * ROW + nmu * col;
-            nr[k] = nmu;
-          }
-        }
-      }
-      __syncthreads();   // phase A and B data read; the rows overwrite them
-#pragma unroll
-      for (int k = 0; k < NCI; k++)
-        if (dst[k] >= 0)
-#pragma unroll
-          for (int r = 0; r < 4; r++)
-            if (r < nr[k]) sR[dst[k] + r] = Xc[k][r];
-    }
-    __syncthreads();
-    // ---------------- phase D
-#pragma unroll
-    for (int j = 0; j < (RT * NBX + RW - 1) / RW; j++) {
-      const int sl = tid + j * RW;
-      if (sl < nown * NBX) {
-        const int sg = sl / NBX, e = sl - sg * NBX;
-        const int64_t k0 = max(sSeg[sg], c0), k1 = min(sSeg[sg + 1], c0 + nt);
-        if (k0 < k1 && e < sNb[sg]) {
-          double *const o = out + sBo[sg] + e;
-          double a = *o;
-          for (int64_t k = k0; k < k1; k++) {
-            const int row = (int)(k - c0);
-            for (int so = 0; so < sNs[row]; so++) a = a + sR[(row * RSO + so) * ROW + e];
-          }
-          *o = a;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (status) atomicOr(v.status, status);
-}
-
 // per pair: nssh_mu * nssh_nu (sizes of the shell blocks)
 __global__ void k_shell_sizes(DView v, int64_t *sz) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -788,9 +531,9 @@ int fbk_rho_3c(const DView &v, int weighted, int maxsh, int sp, hipStream_t st) 
     if (v.ntiles[0] == 0) return 0;
     const dim3 g((unsigned)v.ntiles[0]);
     if (weighted)
-      hipLaunchKernelGGL(k_rho_3c_ph<true>, g, dim3(RW), 0, st, v);
+      hipLaunchKernelGGL(k_3c_wave<W3_RHOS>, g, dim3(64 * w3_terms(W3_RHOS)), 0, st, v);
     else
-      hipLaunchKernelGGL(k_rho_3c_ph<false>, g, dim3(RW), 0, st, v);
+      hipLaunchKernelGGL(k_3c_wave<W3_RHO>, g, dim3(64 * w3_terms(W3_RHO)), 0, st, v);
     return (int)hipGetLastError();
   }
   if (fb_wide_species(v.sp)) launch_rho_3c<FB_MOD>(v, weighted, maxsh, st);

@@ -266,8 +266,9 @@ struct fb_ctx {
 
   // forces (k.DASSEMBLERS): density matrix in, Dblocks and force pieces out
   DevBuf d_rho, d_dmat[3], d_fatom, d_fontop, d_f3a, d_f3b, d_f3c, d_f3, d_jkey, d_jkey_s, d_iota_t, d_perm_j,
-      d_inv_perm, d_inv_perm_j, d_ioff, d_joff;
-  long forces_gen = -1;          // lists_gen the force buffers and orderings belong to
+      d_inv_perm, d_inv_perm_j, d_ioff, d_joff, d_fseg, d_fpair, d_pq, d_trip_nb, d_aseg, d_afix;
+  long forces_gen = -1;          // lists_gen the force buffers belong to
+  long forces_order_gen[2] = {-1, -1};   // and the orderings of the generic and of the s/p 3c kernels
   // McWEDA densities: shell-block offsets, per-structure ranges, progress
   DevBuf d_wbsz, d_wboff;
   std::vector<int64_t> h_wboff_struct;
@@ -393,6 +394,12 @@ struct fb_ctx {
     f.ioff = d_ioff.as<int64_t>();
     f.inv_perm_j = d_inv_perm_j.as<int>();
     f.joff = d_joff.as<int64_t>();
+    f.fseg = d_fseg.as<double>();
+    f.fpair = d_fpair.as<double>();
+    f.pq = d_pq.as<double>();
+    f.trip_nb = d_trip_nb.as<int>();
+    f.aseg = d_aseg.as<int>();
+    f.afix = d_afix.as<int>();
     return f;
   }
 
@@ -577,7 +584,8 @@ struct fb_ctx {
     for (int l = 0; l < 3; l++)
       for (DevBuf *b : {&d_ppn[l], &d_ppoff[l], &d_ppj[l], &d_ppb[l], &d_ppatom[l], &d_ppself[l]}) b->release();
     DevBuf *fbufs[] = {&d_rho, &d_dmat[0], &d_dmat[1], &d_dmat[2], &d_fatom, &d_fontop, &d_f3a, &d_f3b, &d_f3c,
-                       &d_f3, &d_jkey, &d_jkey_s, &d_iota_t, &d_perm_j, &d_inv_perm, &d_inv_perm_j, &d_ioff, &d_joff};
+                       &d_f3, &d_jkey, &d_jkey_s, &d_iota_t, &d_perm_j, &d_inv_perm, &d_inv_perm_j, &d_ioff, &d_joff,
+                       &d_fseg, &d_fpair, &d_pq, &d_trip_nb, &d_aseg, &d_afix};
     for (DevBuf *b : fbufs) b->release();
     reset_events();
     for (auto e : pool) (void)hipEventDestroy(e);
@@ -2914,26 +2922,57 @@ int fb_get_pp_blocks(fb_ctx *ctx, int is, int which, double *out) {
 }
 
 // ------------------------------------------------------------------ forces
-// Buffers of the force assemblers and the two triplet orderings of the
-// per-atom sums (iatom: the target-pair order of the lists; jatom: a stable
-// radix sort of the list order by jatom), built once per list generation.
+// Buffers of the force assemblers, once per list generation.
 static int prep_forces(fb_ctx *ctx) {
   if (ctx->forces_gen == ctx->lists_gen) return FB_OK;
-  hipStream_t st = ctx->stream;
-  RC(list_order(ctx));
-  const int64_t P = ctx->npairs, T = ctx->ntrip, B = ctx->blen;
-  const int N = ctx->natoms;
+  const int64_t P = ctx->npairs, B = ctx->blen;
   auto one = [](int64_t n) { return (size_t)std::max<int64_t>(n, 1); };
   FB_HIP(ctx->d_rho.ensure(sizeof(double) * one(B)));
   for (int i = 0; i < 3; i++) FB_HIP(ctx->d_dmat[i].ensure(sizeof(double) * one(3 * B)));
   FB_HIP(ctx->d_fatom.ensure(sizeof(double) * one(3 * P)));
   FB_HIP(ctx->d_fontop.ensure(sizeof(double) * one(3 * P)));
-  FB_HIP(ctx->d_f3a.ensure(sizeof(double) * one(3 * T)));
+  FB_HIP(ctx->d_f3a.ensure(sizeof(double) * one(3 * ctx->ntrip)));
+  FB_HIP(ctx->d_f3.ensure(sizeof(double) * one(9 * (int64_t)ctx->natoms)));
+  ctx->rho_ok.assign(ctx->structs.size(), 0);
+  for (int i = 0; i < 5; i++) ctx->ddone[i] = 0;
+  ctx->forces_gen = ctx->lists_gen;
+  return FB_OK;
+}
+
+// s/p species with canonical tables take the register-resident force kernels
+static bool sp_forces(const fb_ctx *ctx) { return ctx->canon_sp && ctx->force_kernel == 1; }
+
+// What the 3c force kernels need of the lists, once per list generation.  The
+// generic kernels: the triplets in list order and the two orderings of the
+// per-atom sums (iatom: the target-pair order; jatom: a stable radix sort of
+// the list order by jatom).  The s/p kernels work in target order.
+static int prep_d3c(fb_ctx *ctx) {
+  const bool sp = sp_forces(ctx);
+  if (ctx->forces_order_gen[sp] == ctx->lists_gen) return FB_OK;
+  hipStream_t st = ctx->stream;
+  const int64_t P = ctx->npairs, T = ctx->ntrip;
+  const int N = ctx->natoms;
+  auto one = [](int64_t n) { return (size_t)std::max<int64_t>(n, 1); };
+  DView v = ctx->view();
+  if (sp) {
+    FB_HIP(ctx->d_fseg.ensure(sizeof(double) * one(6 * P)));
+    FB_HIP(ctx->d_fpair.ensure(sizeof(double) * one(3 * P)));
+    FB_HIP(ctx->d_pq.ensure(sizeof(double) * one(8 * P)));
+    FB_HIP(ctx->d_trip_nb.ensure(sizeof(int) * one(T)));
+    FB_HIP(ctx->d_aseg.ensure(sizeof(int) * (N + 1)));
+    FB_HIP(ctx->d_afix.ensure(sizeof(int) * N));
+    RC(ctx->launch("d3c_clear", [&] { return fbk_fill_i32(ctx->d_afix.as<int>(), N, 0, st); }));
+    RC(ctx->launch("d3c_lists", [&] {
+      return fbk_d3c_sp_lists(v, ctx->d_trip_nb.as<int>(), ctx->d_aseg.as<int>(), st);
+    }));
+    ctx->forces_order_gen[sp] = ctx->lists_gen;
+    return FB_OK;
+  }
+  RC(list_order(ctx));
   FB_HIP(ctx->d_f3b.ensure(sizeof(double) * one(3 * T)));
   FB_HIP(ctx->d_f3c.ensure(sizeof(double) * one(3 * T)));
   FB_HIP(ctx->d_inv_perm.ensure(sizeof(int) * one(T)));
   FB_HIP(ctx->d_inv_perm_j.ensure(sizeof(int) * one(T)));
-  FB_HIP(ctx->d_f3.ensure(sizeof(double) * one(9 * (int64_t)N)));
   FB_HIP(ctx->d_ioff.ensure(sizeof(int64_t) * (N + 1)));
   FB_HIP(ctx->d_joff.ensure(sizeof(int64_t) * (N + 1)));
   FB_HIP(ctx->d_jkey.ensure(sizeof(int) * one(T)));
@@ -2967,10 +3006,7 @@ static int prep_forces(fb_ctx *ctx) {
     return fbk_f3_offsets(N, T, ctx->d_noff.as<int64_t>(), ctx->d_tpair.as<int>(), ctx->d_jkey_s.as<int>(),
                           ctx->d_ioff.as<int64_t>(), ctx->d_joff.as<int64_t>(), st);
   }));
-  FB_HIP(hipStreamSynchronize(st));
-  ctx->rho_ok.assign(ctx->structs.size(), 0);
-  for (int i = 0; i < 5; i++) ctx->ddone[i] = 0;
-  ctx->forces_gen = ctx->lists_gen;
+  ctx->forces_order_gen[sp] = ctx->lists_gen;
   return FB_OK;
 }
 
@@ -3002,11 +3038,10 @@ static bool all_rho(const fb_ctx *ctx) {
   return !ctx->rho_ok.empty();
 }
 
-// s/p species with canonical tables take the register-resident kernels
 static int launch_d2c(fb_ctx *ctx, int mask, const char *what) {
   DView v = ctx->view();
   DForce f = ctx->fview();
-  if (ctx->canon_sp && ctx->force_kernel == 1)
+  if (sp_forces(ctx))
     return ctx->launch(what, [&] { return fbk_d2c_sp(v, f, mask, ctx->stream); });
   return ctx->launch(what, [&] { return fbk_d2c(v, f, mask, ctx->stream); });
 }
@@ -3036,14 +3071,17 @@ int fb_dassemble_vna_2c(fb_ctx *ctx) {
 }
 
 static int run_d3c(fb_ctx *ctx) {
+  RC(prep_d3c(ctx));
   DView v = ctx->view();
   DForce f = ctx->fview();
-  if (ctx->canon_sp && ctx->force_kernel == 1)
+  if (sp_forces(ctx)) {
     RC(ctx->launch("Dassemble_vna_3c", [&] {
       return fbk_d3c_sp(v, f, any_charge(ctx), ctx->precision == FB_PREC_MIXED, ctx->stream);
     }));
-  else
-    RC(ctx->launch("Dassemble_vna_3c", [&] { return fbk_d3c(v, f, ctx->stream); }));
+    RC(ctx->launch("forces_3c_sum", [&] { return fbk_d3c_sp_sum(v, f, ctx->stream); }));
+    return FB_OK;
+  }
+  RC(ctx->launch("Dassemble_vna_3c", [&] { return fbk_d3c(v, f, ctx->stream); }));
   RC(ctx->launch("forces_3c_sum", [&] { return fbk_f3_reduce(v, f, ctx->stream); }));
   return FB_OK;
 }

@@ -868,61 +868,6 @@ __device__ __forceinline__ void drot2c_sp(const double *pm, const double *dpm, c
   }
 }
 
-// Drotate of a 3c block, canonical ME order
-// {ss, s-pz, pz-s, py-py, pz-pz, px-px, s-px, px-s, px-pz, pz-px} (s-sp: {ss, s-pz, s-px}; sp-s: {ss, pz-s, px-s})
-template <int CLS>
-__device__ __forceinline__ void drot3c_sp(const double *pm, const double *dpm, const double *F, const double *DM,
-                                          double *X) {
-  X[0] = DM[0];
-  if (CLS == CLS_SPSP) {
-#pragma unroll
-    for (int l = 0; l < 3; l++) {
-      double x = DD_(l, 1) * F[1];
-      x = x + PP_(l, 1) * DM[1];
-      x = x + DD_(l, 2) * F[6];
-      x = x + PP_(l, 2) * DM[6];
-      X[(1 + l) * 4] = x;
-    }
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      double x = DD_(k, 1) * F[2];
-      x = x + PP_(k, 1) * DM[2];
-      x = x + DD_(k, 2) * F[7];
-      x = x + PP_(k, 2) * DM[7];
-      X[1 + k] = x;
-    }
-#pragma unroll
-    for (int l = 0; l < 3; l++)
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        double x = 0.0;
-        x = drot_pp_term(x, pm, dpm, k, l, 0, 0, F[3], DM[3]);
-        x = drot_pp_term(x, pm, dpm, k, l, 1, 1, F[4], DM[4]);
-        x = drot_pp_term(x, pm, dpm, k, l, 2, 1, F[8], DM[8]);
-        x = drot_pp_term(x, pm, dpm, k, l, 1, 2, F[9], DM[9]);
-        x = drot_pp_term(x, pm, dpm, k, l, 2, 2, F[5], DM[5]);
-        X[(1 + l) * 4 + 1 + k] = x;
-      }
-  } else if (CLS == CLS_SSP) {
-#pragma unroll
-    for (int l = 0; l < 3; l++) {
-      double x = DD_(l, 1) * F[1];
-      x = x + PP_(l, 1) * DM[1];
-      x = x + DD_(l, 2) * F[2];
-      x = x + PP_(l, 2) * DM[2];
-      X[1 + l] = x;
-    }
-  } else if (CLS == CLS_SPS) {
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      double x = DD_(k, 1) * F[1];
-      x = x + PP_(k, 1) * DM[1];
-      x = x + DD_(k, 2) * F[2];
-      x = x + PP_(k, 2) * DM[2];
-      X[1 + k] = x;
-    }
-  }
-}
 #undef PP_
 #undef DD_
 
@@ -1226,792 +1171,7 @@ __global__ __launch_bounds__(WD2S) void k_d2c_sp(DView v, DForce Fo, int mask) {
 }
 
 // ---------------------------------------------------------------- 3c, s/p
-
-// Depsilon_3c restricted to one Cartesian component ix (1-based): the
-// (ix, :, :) slices of dera3 and der13 depend on that component only
-struct D3Scal {
-  double crossmag, r2mag2, r1mag2, ratmmag2, r1dotr2, r2dotratm, r1dotratm;
-  bool zero;
-};
-
-__device__ __forceinline__ void d3_scal(const double *r1, const double *r2, const double *r21, const double *ratm,
-                                        const double *rnabc, D3Scal &S) {
-  double ca0 = r21[1] * rnabc[2] - r21[2] * rnabc[1];
-  double ca1 = r21[2] * rnabc[0] - r21[0] * rnabc[2];
-  double ca2 = r21[0] * rnabc[1] - r21[1] * rnabc[0];
-  S.crossmag = sqrt(ca0 * ca0 + ca1 * ca1 + ca2 * ca2);
-  S.zero = fabs(S.crossmag) < 1.0e-3;
-  S.r2mag2 = r2[0] * r2[0] + r2[1] * r2[1] + r2[2] * r2[2];
-  S.r1mag2 = r1[0] * r1[0] + r1[1] * r1[1] + r1[2] * r1[2];
-  S.ratmmag2 = ratm[0] * ratm[0] + ratm[1] * ratm[1] + ratm[2] * ratm[2];
-  S.r1dotr2 = r1[0] * r2[0] + r1[1] * r2[1] + r1[2] * r2[2];
-  S.r2dotratm = r2[0] * ratm[0] + r2[1] * ratm[1] + r2[2] * ratm[2];
-  S.r1dotratm = r1[0] * ratm[0] + r1[1] * ratm[1] + r1[2] * ratm[2];
-}
-
-// dA[imu + 3*(k-1)] = dera3(ix, imu, k), dB = der13(ix, imu, k)
-__device__ __forceinline__ void d3_slice(const double *r1, const double *r2, double z, const double *ratm,
-                                         const double *eps3, const D3Scal &S, int ix, double *dA, double *dB) {
-#define E3(i, j) eps3[3 * ((j) - 1) + (i) - 1]
-#define SA(imu, k) dA[((imu) - 1) + 3 * ((k) - 1)]
-#define SB(imu, k) dB[((imu) - 1) + 3 * ((k) - 1)]
-#pragma unroll
-  for (int i = 0; i < 9; i++) { dA[i] = 0.0; dB[i] = 0.0; }
-  if (S.zero) return;
-  const double cm = S.crossmag;
-  const double ra = sel3(ratm, ix - 1), r1x = sel3(r1, ix - 1), r2x = sel3(r2, ix - 1);
-  const double e3x = ix == 1 ? E3(1, 3) : (ix == 2 ? E3(2, 3) : E3(3, 3));
-#pragma unroll
-  for (int imu = 1; imu <= 3; imu++) {
-    double sum = d_levi(ix, imu, 1) * (r2[0] - r1[0]) + d_levi(ix, imu, 2) * (r2[1] - r1[1]) +
-                 d_levi(ix, imu, 3) * (r2[2] - r1[2]);
-    SA(imu, 2) = (1.0 / cm) * (sum - (E3(imu, 2) / cm) *
-                                         ((S.r1mag2 + S.r2mag2 - 2.0 * S.r1dotr2) * ra +
-                                          (S.r1dotr2 - S.r1mag2 - S.r2dotratm + S.r1dotratm) * r2x +
-                                          (S.r1dotr2 - S.r2mag2 + S.r2dotratm - S.r1dotratm) * r1x));
-  }
-  SA(1, 1) = E3(3, 3) * SA(2, 2) - E3(2, 3) * SA(3, 2);
-  SA(2, 1) = E3(1, 3) * SA(3, 2) - E3(3, 3) * SA(1, 2);
-  SA(3, 1) = E3(2, 3) * SA(1, 2) - E3(1, 3) * SA(2, 2);
-#pragma unroll
-  for (int imu = 1; imu <= 3; imu++) {
-    SB(imu, 3) = (1.0 / z) * (E3(imu, 3) * e3x - d_delk(imu, ix));
-    double sum = d_levi(ix, imu, 1) * (ratm[0] - r2[0]) + d_levi(ix, imu, 2) * (ratm[1] - r2[1]) +
-                 d_levi(ix, imu, 3) * (ratm[2] - r2[2]);
-    SB(imu, 2) = (1.0 / cm) * (sum - (E3(imu, 2) / cm) *
-                                         ((S.r2dotratm - S.r1dotratm + S.r1dotr2 - S.r2mag2) * ra +
-                                          (S.r2dotratm + S.r1dotratm - S.r1dotr2 - S.ratmmag2) * r2x +
-                                          (S.ratmmag2 - 2.0 * S.r2dotratm + S.r2mag2) * r1x));
-  }
-  SB(1, 1) = E3(3, 3) * SB(2, 2) - E3(3, 2) * SB(2, 3) - E3(2, 3) * SB(3, 2) + E3(2, 2) * SB(3, 3);
-  SB(2, 1) = E3(1, 3) * SB(3, 2) - E3(1, 2) * SB(3, 3) - E3(3, 3) * SB(1, 2) + E3(3, 2) * SB(1, 3);
-  SB(3, 1) = E3(2, 3) * SB(1, 2) - E3(2, 2) * SB(1, 3) - E3(1, 3) * SB(2, 2) + E3(1, 2) * SB(2, 3);
-#undef E3
-#undef SA
-#undef SB
-}
-
-// Dtwister p part from a slice s[imu + 3*(k-1)] = deps(ix, imu, k)
-__device__ __forceinline__ void dpmat_slice(const double *s, double *dpm) {
-#define SL(imu, k) s[((imu) - 1) + 3 * ((k) - 1)]
-  dpm[0] = SL(2, 2); dpm[3] = SL(2, 3); dpm[6] = SL(2, 1);
-  dpm[1] = SL(3, 2); dpm[4] = SL(3, 3); dpm[7] = SL(3, 1);
-  dpm[2] = SL(1, 2); dpm[5] = SL(1, 3); dpm[8] = SL(1, 1);
-#undef SL
-}
-
-// getDMEs_Fdata_3c of one canonical group: values and d/dcos, d/dx, d/dy
-template <int NME>
-__device__ __forceinline__ int dgetD3c_sp(const DView &v, int gid, double x, double y, double cost, double *F,
-                                          double *DpF, double *DxF, double *DyF) {
-  if (gid < 0) return ST_NO_TABLE;
-  const DGroup3c g = v.grp3c[gid];
-  const int nx = g.nx, ny = g.ny;
-  // Legendre P0..P4 and derivatives, selected per theta below (no private array)
-  const double cost2 = cost * cost;
-  const double sint = sqrt(fmax(1.0e-5, 1.0 - cost2));
-  const double p2 = 0.5 * (3.0 * cost2 - 1.0);
-  const double p3 = 0.5 * cost * (5.0 * cost2 - 3.0);
-  const double p4 = 0.125 * (3.0 - cost2 * (30.0 - 35.0 * cost2));
-  const double dp2 = 3.0 * cost;
-  const double dp3 = (15.0 * cost2 - 3.0) / 2.0;
-  const double dp4 = 0.5 * cost * (35.0 * cost2 - 15.0);
-  const double dx = g.xmax / (nx - 1.0), dy = g.ymax / (ny - 1.0);
-  int ix = (int)(x / dx) + 1, iy = (int)(y / dy) + 1;
-  if (ix < 2) ix = 2;
-  if (iy < 2) iy = 2;
-  if (ix > nx - 2) ix = nx - 2;
-  if (iy > ny - 2) iy = ny - 2;
-  const double px = x / dx - ix + 1.0, py = y / dy - iy + 1.0;
-  const double *tab = v.tab3c + g.off;
-#define T3S(th, i, j, m) tab[FB_T64(th, i, j, m, nx, NME)]
-  const double gx = (T3S(0, ix + 1, iy, 0) - T3S(0, ix, iy, 0)) / dx;
-  const double gy = (T3S(0, ix, iy + 1, 0) - T3S(0, ix, iy, 0)) / dy;
-  const bool three = (gx * gx + gy * gy) < 1.0e-6;
-#pragma unroll
-  for (int m = 0; m < NME; m++) { F[m] = 0.0; DpF[m] = 0.0; DxF[m] = 0.0; DyF[m] = 0.0; }
-  for (int th = 0; th < FB_NTHETA; th++) {
-    const double pt = th == 0 ? 1.0 : (th == 1 ? cost : (th == 2 ? p2 : (th == 3 ? p3 : p4)));
-    const double dpt = th == 0 ? 0.0 : (th == 1 ? 1.0 : (th == 2 ? dp2 : (th == 3 ? dp3 : dp4)));
-#pragma unroll
-    for (int m = 0; m < NME; m++) {
-      if (three) {
-        const double interim =
-            ((1.0 - px - py) * T3S(th, ix, iy, m) + px * T3S(th, ix + 1, iy, m)) + py * T3S(th, ix, iy + 1, m);
-        F[m] = F[m] + pt * interim;
-        DpF[m] = DpF[m] + dpt * interim;
-        DxF[m] = DxF[m] + pt * gx;
-        DyF[m] = DyF[m] + pt * gy;
-      } else {
-        double gk[4], gp[4];
-#pragma unroll
-        for (int k = -1; k <= 2; k++) {
-          double f1m1 = T3S(th, ix + k, iy - 1, m);
-          double f1m2 = 2.0 * f1m1, f1m3 = 3.0 * f1m1;
-          double f0p3 = 3.0 * T3S(th, ix + k, iy, m), f0p6 = 2.0 * f0p3;
-          double f1p3 = 3.0 * T3S(th, ix + k, iy + 1, m), f1p6 = 2.0 * f1p3;
-          double f2p1 = T3S(th, ix + k, iy + 2, m);
-          double bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-          double bb2 = f1m3 - f0p6 + f1p3;
-          double bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-          double bb0 = f0p6;
-          gk[k + 1] = ((bb3 * py + bb2) * py + bb1) * py + bb0;
-          gp[k + 1] = ((3.0 * bb3 * py + 2.0 * bb2) * py + bb1);
-        }
-        double f1m1 = gk[0], f1m2 = 2.0 * f1m1, f1m3 = 3.0 * f1m1;
-        double f0p3 = 3.0 * gk[1], f0p6 = 2.0 * f0p3;
-        double f1p3 = 3.0 * gk[2], f1p6 = 2.0 * f1p3;
-        double f2p1 = gk[3];
-        double bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-        double bb2 = f1m3 - f0p6 + f1p3;
-        double bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-        double bb0 = f0p6;
-        const double interim = (((bb3 * px + bb2) * px + bb1) * px + bb0) / 36.0;
-        F[m] = F[m] + pt * interim;
-        DpF[m] = DpF[m] + dpt * interim;
-        DxF[m] = DxF[m] + pt * ((3.0 * bb3 * px + 2.0 * bb2) * px + bb1) / (36.0 * dx);
-        f1m1 = gp[0]; f1m2 = 2.0 * f1m1; f1m3 = 3.0 * f1m1;
-        f0p3 = 3.0 * gp[1]; f0p6 = 2.0 * f0p3;
-        f1p3 = 3.0 * gp[2]; f1p6 = 2.0 * f1p3;
-        f2p1 = gp[3];
-        bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-        bb2 = f1m3 - f0p6 + f1p3;
-        bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-        bb0 = f0p6;
-        DyF[m] = DyF[m] + pt * (((bb3 * px + bb2) * px + bb1) * px + bb0) / (36.0 * dy);
-      }
-    }
-  }
-#undef T3S
-  constexpr int NM0 = (NME == 10) ? 6 : (NME == 3 ? 2 : 1);
-#pragma unroll
-  for (int m = NM0; m < NME; m++) {
-    DpF[m] = DpF[m] * sint - cost * F[m] / sint;
-    F[m] = F[m] * sint;
-    DxF[m] = DxF[m] * sint;
-    DyF[m] = DyF[m] * sint;
-  }
-  return 0;
-}
-
-struct DGeo3s {
-  double r1[3], r2[3], rna[3], r21[3], rnabc[3], sighat[3], rhat[3], amt[3], bmt[3];
-  double z, x, cost, d13, d23;
-  double eps[9];
-};
-
-__device__ __forceinline__ void d_dgeo3s(const DView &v, int4 tr, bool charged, DGeo3s &G) {
-  const int ial = tr.x, gia = tr.y, gja = tr.z;
-  const int ib = tr.w & 0xffff, jb = (tr.w >> 16) & 0xffff;
-  const int s = v.atom_struct[ial];
-  const double *xls = v.xl + (int64_t)s * FB_NIMG * 3;
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    G.r1[k] = v.ratom[3 * gia + k] + xls[3 * ib + k];
-    G.r2[k] = v.ratom[3 * gja + k] + xls[3 * jb + k];
-    G.rna[k] = v.ratom[3 * ial + k];
-    G.r21[k] = G.r2[k] - G.r1[k];
-  }
-  G.z = d_distance(G.r1, G.r2);
-  if (G.z < 1.0e-5) { G.sighat[0] = 0.0; G.sighat[1] = 0.0; G.sighat[2] = 1.0; }
-  else {
-#pragma unroll
-    for (int k = 0; k < 3; k++) G.sighat[k] = G.r21[k] / G.z;
-  }
-#pragma unroll
-  for (int k = 0; k < 3; k++) G.rnabc[k] = G.rna[k] - (G.r1[k] + G.r21[k] / 2.0);
-  G.x = sqrt(G.rnabc[0] * G.rnabc[0] + G.rnabc[1] * G.rnabc[1] + G.rnabc[2] * G.rnabc[2]);
-  G.d13 = d_distance(G.rna, G.r1);
-  G.d23 = d_distance(G.rna, G.r2);
-  if (G.x < 1.0e-5) { G.rhat[0] = 0.0; G.rhat[1] = 0.0; G.rhat[2] = 0.0; }
-  else if (charged) {
-#pragma unroll
-    for (int k = 0; k < 3; k++) G.rhat[k] = (G.rna[k] - 0.5 * (G.r1[k] + G.r2[k])) / G.x;
-  } else {
-#pragma unroll
-    for (int k = 0; k < 3; k++) G.rhat[k] = G.rnabc[k] / G.x;
-  }
-  G.cost = G.sighat[0] * G.rhat[0] + G.sighat[1] * G.rhat[1] + G.sighat[2] * G.rhat[2];
-  d_epsilon(G.rhat, G.sighat, G.eps);
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    G.amt[k] = (G.x > 1.0e-5) ? (G.sighat[k] - G.cost * G.rhat[k]) / G.x : 0.0;
-    G.bmt[k] = (G.cost * G.sighat[k] - G.rhat[k]) / G.z;
-  }
-}
-
-// element (row, col) of the rotated derivative of a 3c block: drot3c_sp one
-// element at a time (same terms, same order), so that a triplet never holds a
-// whole rotated block
-template <int CLS>
-__device__ __forceinline__ double drot3c_el(int row, int col, const double *pm, const double *dpm, const double *F,
-                                            const double *DM) {
-#define PP_(k, m) pm[3 * (m) + (k)]
-#define DD_(k, m) dpm[3 * (m) + (k)]
-  if (row == 0 && col == 0) return DM[0];
-  if (CLS == CLS_SPSP) {
-    if (row == 0) {
-      const int l = col - 1;
-      double x = DD_(l, 1) * F[1];
-      x = x + PP_(l, 1) * DM[1];
-      x = x + DD_(l, 2) * F[6];
-      return x + PP_(l, 2) * DM[6];
-    }
-    if (col == 0) {
-      const int k = row - 1;
-      double x = DD_(k, 1) * F[2];
-      x = x + PP_(k, 1) * DM[2];
-      x = x + DD_(k, 2) * F[7];
-      return x + PP_(k, 2) * DM[7];
-    }
-    const int k = row - 1, l = col - 1;
-    double x = 0.0;
-    x = drot_pp_term(x, pm, dpm, k, l, 0, 0, F[3], DM[3]);
-    x = drot_pp_term(x, pm, dpm, k, l, 1, 1, F[4], DM[4]);
-    x = drot_pp_term(x, pm, dpm, k, l, 2, 1, F[8], DM[8]);
-    x = drot_pp_term(x, pm, dpm, k, l, 1, 2, F[9], DM[9]);
-    return drot_pp_term(x, pm, dpm, k, l, 2, 2, F[5], DM[5]);
-  }
-  if (CLS == CLS_SSP) {
-    const int l = col - 1;
-    double x = DD_(l, 1) * F[1];
-    x = x + PP_(l, 1) * DM[1];
-    x = x + DD_(l, 2) * F[2];
-    return x + PP_(l, 2) * DM[2];
-  }
-  if (CLS == CLS_SPS) {
-    const int k = row - 1;
-    double x = DD_(k, 1) * F[1];
-    x = x + PP_(k, 1) * DM[1];
-    x = x + DD_(k, 2) * F[2];
-    return x + PP_(k, 2) * DM[2];
-  }
-  return 0.0;
-}
-
-#undef PP_
-#undef DD_
-
-// ---------------------------------------------------------------------------
-// Four lanes per triplet.  Phase A: lane q interpolates matrix elements q, q+4,
-// q+8 of the group (value and its cos, x and y derivatives) into the
-// triplet's LDS row.  Phase B: lane q < 3 takes Cartesian component q: the
-// frame-derivative slices of that component, f3naMa / f3naMb, the two rotated
-// derivative blocks element by element, and the contraction with the density
-// block, so that no lane loops over components and every private value has a
-// compile-time index.  Lane 3 idles in phase B.
-#define T3Q 64                 // lanes per workgroup: 16 triplets
-#define SIROW (4 * NME3F + 1)  // LDS row per triplet (odd stride: no bank sharing)
-
-// getDMEs_Fdata_3c of elements q, q+4, q+8 of one canonical group into row
-__device__ inline int stage_q(const DView &v, int gid, int nme, double x, double y, double cost, double *row, int q) {
-  if (gid < 0) return ST_NO_TABLE;
-  const DGroup3c g = v.grp3c[gid];
-  const int nx = g.nx, ny = g.ny;
-  const double cost2 = cost * cost;
-  const double sint = sqrt(fmax(1.0e-5, 1.0 - cost2));
-  const double p2 = 0.5 * (3.0 * cost2 - 1.0);
-  const double p3 = 0.5 * cost * (5.0 * cost2 - 3.0);
-  const double p4 = 0.125 * (3.0 - cost2 * (30.0 - 35.0 * cost2));
-  const double dp2 = 3.0 * cost;
-  const double dp3 = (15.0 * cost2 - 3.0) / 2.0;
-  const double dp4 = 0.5 * cost * (35.0 * cost2 - 15.0);
-  const double dx = g.xmax / (nx - 1.0), dy = g.ymax / (ny - 1.0);
-  int ix = (int)(x / dx) + 1, iy = (int)(y / dy) + 1;
-  if (ix < 2) ix = 2;
-  if (iy < 2) iy = 2;
-  if (ix > nx - 2) ix = nx - 2;
-  if (iy > ny - 2) iy = ny - 2;
-  const double px = x / dx - ix + 1.0, py = y / dy - iy + 1.0;
-  const double *tab = v.tab3c + g.off;
-#define T3Q_(th, i, j, m) tab[FB_T64(th, i, j, m, nx, nme)]
-  const double gx = (T3Q_(0, ix + 1, iy, 0) - T3Q_(0, ix, iy, 0)) / dx;
-  const double gy = (T3Q_(0, ix, iy + 1, 0) - T3Q_(0, ix, iy, 0)) / dy;
-  const bool three = (gx * gx + gy * gy) < 1.0e-6;
-  const int nm0 = (nme == 10) ? 6 : (nme == 3 ? 2 : 1);   // canonical order: mvalue = 1 elements last
-  for (int m = q; m < nme; m += 4) {
-    double F = 0.0, DpF = 0.0, DxF = 0.0, DyF = 0.0;
-    for (int th = 0; th < FB_NTHETA; th++) {
-      const double pt = th == 0 ? 1.0 : (th == 1 ? cost : (th == 2 ? p2 : (th == 3 ? p3 : p4)));
-      const double dpt = th == 0 ? 0.0 : (th == 1 ? 1.0 : (th == 2 ? dp2 : (th == 3 ? dp3 : dp4)));
-      if (three) {
-        const double interim =
-            ((1.0 - px - py) * T3Q_(th, ix, iy, m) + px * T3Q_(th, ix + 1, iy, m)) + py * T3Q_(th, ix, iy + 1, m);
-        F = F + pt * interim;
-        DpF = DpF + dpt * interim;
-        DxF = DxF + pt * gx;
-        DyF = DyF + pt * gy;
-      } else {
-        double gk[4], gp[4];
-#pragma unroll
-        for (int k = -1; k <= 2; k++) {
-          double f1m1 = T3Q_(th, ix + k, iy - 1, m);
-          double f1m2 = 2.0 * f1m1, f1m3 = 3.0 * f1m1;
-          double f0p3 = 3.0 * T3Q_(th, ix + k, iy, m), f0p6 = 2.0 * f0p3;
-          double f1p3 = 3.0 * T3Q_(th, ix + k, iy + 1, m), f1p6 = 2.0 * f1p3;
-          double f2p1 = T3Q_(th, ix + k, iy + 2, m);
-          double bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-          double bb2 = f1m3 - f0p6 + f1p3;
-          double bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-          double bb0 = f0p6;
-          gk[k + 1] = ((bb3 * py + bb2) * py + bb1) * py + bb0;
-          gp[k + 1] = ((3.0 * bb3 * py + 2.0 * bb2) * py + bb1);
-        }
-        double f1m1 = gk[0], f1m2 = 2.0 * f1m1, f1m3 = 3.0 * f1m1;
-        double f0p3 = 3.0 * gk[1], f0p6 = 2.0 * f0p3;
-        double f1p3 = 3.0 * gk[2], f1p6 = 2.0 * f1p3;
-        double f2p1 = gk[3];
-        double bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-        double bb2 = f1m3 - f0p6 + f1p3;
-        double bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-        double bb0 = f0p6;
-        const double interim = (((bb3 * px + bb2) * px + bb1) * px + bb0) / 36.0;
-        F = F + pt * interim;
-        DpF = DpF + dpt * interim;
-        DxF = DxF + pt * ((3.0 * bb3 * px + 2.0 * bb2) * px + bb1) / (36.0 * dx);
-        f1m1 = gp[0]; f1m2 = 2.0 * f1m1; f1m3 = 3.0 * f1m1;
-        f0p3 = 3.0 * gp[1]; f0p6 = 2.0 * f0p3;
-        f1p3 = 3.0 * gp[2]; f1p6 = 2.0 * f1p3;
-        f2p1 = gp[3];
-        bb3 = -f1m1 + f0p3 - f1p3 + f2p1;
-        bb2 = f1m3 - f0p6 + f1p3;
-        bb1 = -f1m2 - f0p3 + f1p6 - f2p1;
-        bb0 = f0p6;
-        DyF = DyF + pt * (((bb3 * px + bb2) * px + bb1) * px + bb0) / (36.0 * dy);
-      }
-    }
-#undef T3Q_
-    if (m >= nm0) {
-      DpF = DpF * sint - cost * F / sint;
-      F = F * sint;
-      DxF = DxF * sint;
-      DyF = DyF * sint;
-    }
-    row[m] = F;
-    row[nme + m] = DpF;
-    row[2 * nme + m] = DxF;
-    row[3 * nme + m] = DyF;
-  }
-  return 0;
-}
-
-// (x, z, cos theta) of a triplet with the expressions of d_dgeo3s, without the
-// frame: what the interpolation needs
-__device__ __forceinline__ void xzc3(const DView &v, int4 tr, bool charged, double &x, double &z, double &cost) {
-  const int ial = tr.x, gia = tr.y, gja = tr.z;
-  const int ib = tr.w & 0xffff, jb = (tr.w >> 16) & 0xffff;
-  const int s = v.atom_struct[ial];
-  const double *xls = v.xl + (int64_t)s * FB_NIMG * 3;
-  double r1[3], r2[3], rna[3], r21[3], sighat[3], rnabc[3], rhat[3];
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    r1[k] = v.ratom[3 * gia + k] + xls[3 * ib + k];
-    r2[k] = v.ratom[3 * gja + k] + xls[3 * jb + k];
-    rna[k] = v.ratom[3 * ial + k];
-    r21[k] = r2[k] - r1[k];
-  }
-  z = d_distance(r1, r2);
-  if (z < 1.0e-5) { sighat[0] = 0.0; sighat[1] = 0.0; sighat[2] = 1.0; }
-  else {
-#pragma unroll
-    for (int k = 0; k < 3; k++) sighat[k] = r21[k] / z;
-  }
-#pragma unroll
-  for (int k = 0; k < 3; k++) rnabc[k] = rna[k] - (r1[k] + r21[k] / 2.0);
-  x = sqrt(rnabc[0] * rnabc[0] + rnabc[1] * rnabc[1] + rnabc[2] * rnabc[2]);
-  if (x < 1.0e-5) { rhat[0] = 0.0; rhat[1] = 0.0; rhat[2] = 0.0; }
-  else if (charged) {
-#pragma unroll
-    for (int k = 0; k < 3; k++) rhat[k] = (rna[k] - 0.5 * (r1[k] + r2[k])) / x;
-  } else {
-#pragma unroll
-    for (int k = 0; k < 3; k++) rhat[k] = rnabc[k] / x;
-  }
-  cost = sighat[0] * rhat[0] + sighat[1] * rhat[1] + sighat[2] * rhat[2];
-}
-
-// ---------------------------------------------------------------------------
-// Mixed precision (fb_set_precision FB_PREC_MIXED): the interpolation of phase
-// A in FP32 over the FP32 slab [iy][ix][ME][theta] -- cubic Lagrange weights in
-// x and y and their derivatives (the Horner form of M_Fdata_3c.f90:636-713 is
-// this polynomial times 36), the Legendre fold of the value and of its cos theta
-// derivative at every stencil point.  The cell, the method, the interpolation
-// arguments and everything of phase B stay binary64.
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t slab32(const float *tab, int64_t nfloats) {
-  return __builtin_amdgcn_make_buffer_rsrc((void *)tab, (short)0, (int)(nfloats * 4), 0x00020000);
-}
-
-// sum_theta P_theta T_theta and sum_theta dP_theta T_theta of one (point, ME); off in bytes
-__device__ __forceinline__ void fold2(__amdgpu_buffer_rsrc_t r, unsigned off, const float *P, const float *dP,
-                                      float &tv, float &tp) {
-  const float4 a = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
-  const float b = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(off + 16u), 0, 0));
-  float v = P[0] * a.x;
-  v = __builtin_fmaf(P[1], a.y, v);
-  v = __builtin_fmaf(P[2], a.z, v);
-  v = __builtin_fmaf(P[3], a.w, v);
-  tv = __builtin_fmaf(P[4], b, v);
-  float u = dP[1] * a.y;
-  u = __builtin_fmaf(dP[2], a.z, u);
-  u = __builtin_fmaf(dP[3], a.w, u);
-  tp = __builtin_fmaf(dP[4], b, u);
-}
-
-// weights of the 4-point cubic on nodes -1, 0, 1, 2 and their p-derivatives
-__device__ __forceinline__ void cubic_wd(float p, float *w, float *d) {
-  const float pm1 = p - 1.f, pm2 = p - 2.f, pp1 = p + 1.f, s6 = 1.f / 6.f, p2 = p * p;
-  w[0] = -p * pm1 * pm2 * s6;
-  w[1] = pp1 * pm1 * pm2 * 0.5f;
-  w[2] = -pp1 * p * pm2 * 0.5f;
-  w[3] = pp1 * p * pm1 * s6;
-  d[0] = -(3.f * p2 - 6.f * p + 2.f) * s6;
-  d[1] = (3.f * p2 - 4.f * p - 1.f) * 0.5f;
-  d[2] = -(3.f * p2 - 2.f * p - 2.f) * 0.5f;
-  d[3] = (3.f * p2 - 1.f) * s6;
-}
-
-// elements q, q+4, q+8 of one canonical group into row (binary64 values)
-__device__ inline int stage_q_mx(const DView &v, int gid, int nme, double x, double y, double cost, double *row,
-                                 int q) {
-  if (gid < 0) return ST_NO_TABLE;
-  const DGroup3c g = v.grp3c[gid];
-  const int nx = g.nx, ny = g.ny;
-  const double dx = g.xmax / (nx - 1.0), dy = g.ymax / (ny - 1.0);
-  int ix = (int)(x / dx) + 1, iy = (int)(y / dy) + 1;
-  if (ix < 2) ix = 2;
-  if (iy < 2) iy = 2;
-  if (ix > nx - 2) ix = nx - 2;
-  if (iy > ny - 2) iy = ny - 2;
-  const double px = x / dx - ix + 1.0, py = y / dy - iy + 1.0;
-  const int64_t icell = (int64_t)(iy - 1) * nx + (ix - 1);
-  const bool three = v.meth3c[g.moff + icell] != 0;
-  const double cost2 = cost * cost;
-  const float sint = (float)sqrt(fmax(1.0e-5, 1.0 - cost2)), cf = (float)cost;
-  float P[5], dP[5];
-  P[0] = 1.f;
-  P[1] = cf;
-  P[2] = (float)(0.5 * (3.0 * cost2 - 1.0));
-  P[3] = (float)(0.5 * cost * (5.0 * cost2 - 3.0));
-  P[4] = (float)(0.125 * (3.0 - cost2 * (30.0 - 35.0 * cost2)));
-  dP[0] = 0.f;
-  dP[1] = 1.f;
-  dP[2] = (float)(3.0 * cost);
-  dP[3] = (float)((15.0 * cost2 - 3.0) / 2.0);
-  dP[4] = (float)(0.5 * cost * (35.0 * cost2 - 15.0));
-  const __amdgpu_buffer_rsrc_t r = slab32(v.tab3c32, v.ntab3c32);
-  const unsigned PT = (unsigned)(nme * FB_TH32 * 4);            // bytes per ix step
-  const unsigned RB = (unsigned)(nx * nme * FB_TH32 * 4);       // bytes per iy step
-  const unsigned base = (unsigned)(g.off32 + ((int64_t)(iy - 2) * nx + (ix - 2)) * nme * FB_TH32) * 4u;
-  const int nm0 = (nme == 10) ? 6 : (nme == 3 ? 2 : 1);
-  float wx[4], wy[4], dwx[4], dwy[4];
-  cubic_wd((float)px, wx, dwx);
-  cubic_wd((float)py, wy, dwy);
-  float gxs = 0.f, gys = 0.f;
-  if (three) {
-    // the 3-point rule's slopes come from ME 1 of theta cell 1 (binary64 table)
-    const double *tab = v.tab3c + g.off;
-#define T3X(i, j) tab[FB_T64(0, i, j, 0, nx, nme)]
-    const double gx = (T3X(ix + 1, iy) - T3X(ix, iy)) / dx;
-    const double gy = (T3X(ix, iy + 1) - T3X(ix, iy)) / dy;
-#undef T3X
-    const float ps = (((P[0] + P[1]) + P[2]) + P[3]) + P[4];
-    gxs = (float)gx * ps;
-    gys = (float)gy * ps;
-  }
-  const float idx = (float)(1.0 / dx), idy = (float)(1.0 / dy);
-  for (int m = q; m < nme; m += 4) {
-    const unsigned o = base + (unsigned)(m * FB_TH32 * 4);
-    float fv, fp, fx, fy;
-    if (three) {
-      const unsigned c = o + RB + PT;   // (ix, iy)
-      float t0, p0, t1, p1, t2, p2;
-      fold2(r, c, P, dP, t0, p0);
-      fold2(r, c + PT, P, dP, t1, p1);
-      fold2(r, c + RB, P, dP, t2, p2);
-      const float w0 = (1.f - (float)px) - (float)py;
-      fv = __builtin_fmaf((float)py, t2, __builtin_fmaf((float)px, t1, w0 * t0));
-      fp = __builtin_fmaf((float)py, p2, __builtin_fmaf((float)px, p1, w0 * p0));
-      fx = gxs;
-      fy = gys;
-    } else {
-      fv = 0.f;
-      fp = 0.f;
-      fx = 0.f;
-      fy = 0.f;
-#pragma unroll
-      for (int l = 0; l < 4; l++) {
-        float gv = 0.f, gp = 0.f, gd = 0.f;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          float tv, tp;
-          fold2(r, o + (unsigned)l * RB + (unsigned)k * PT, P, dP, tv, tp);
-          gv = __builtin_fmaf(wx[k], tv, gv);
-          gp = __builtin_fmaf(wx[k], tp, gp);
-          gd = __builtin_fmaf(dwx[k], tv, gd);
-        }
-        fv = __builtin_fmaf(wy[l], gv, fv);
-        fp = __builtin_fmaf(wy[l], gp, fp);
-        fx = __builtin_fmaf(wy[l], gd, fx);
-        fy = __builtin_fmaf(dwy[l], gv, fy);
-      }
-      fx = fx * idx;
-      fy = fy * idy;
-    }
-    if (m >= nm0) {
-      fp = fp * sint - cf * fv / sint;
-      fv = fv * sint;
-      fx = fx * sint;
-      fy = fy * sint;
-    }
-    row[m] = fv;
-    row[nme + m] = fp;
-    row[2 * nme + m] = fx;
-    row[3 * nme + m] = fy;
-  }
-  return 0;
-}
-
-// the scalars of one Cartesian component q (0..2) of a triplet's geometry
-struct DGeoQ {
-  double rh, am, sg, bm;              // rhat, amt, sighat, bmt components
-  double r1q, r2q, raq, e3q;          // r1, r2, ratm components and eps(q+1, 3)
-  double rA1, rA2;                    // (rna - r1)/d13, (rna - r2)/d23 components (charged terms)
-};
-
-__device__ __forceinline__ double pick3(double a, double b, double c, int q) { return q == 0 ? a : (q == 1 ? b : c); }
-
-__device__ __forceinline__ void geo_q(const DGeo3s &G, int q, DGeoQ &Q) {
-  Q.rh = pick3(G.rhat[0], G.rhat[1], G.rhat[2], q);
-  Q.am = pick3(G.amt[0], G.amt[1], G.amt[2], q);
-  Q.sg = pick3(G.sighat[0], G.sighat[1], G.sighat[2], q);
-  Q.bm = pick3(G.bmt[0], G.bmt[1], G.bmt[2], q);
-  Q.r1q = pick3(G.r1[0], G.r1[1], G.r1[2], q);
-  Q.r2q = pick3(G.r2[0], G.r2[1], G.r2[2], q);
-  Q.raq = pick3(G.rna[0], G.rna[1], G.rna[2], q);
-  Q.e3q = pick3(G.eps[6], G.eps[7], G.eps[8], q);
-  const double a1x = G.d13 > 1.0e-5 ? (G.rna[0] - G.r1[0]) / G.d13 : 0.0;
-  const double a1y = G.d13 > 1.0e-5 ? (G.rna[1] - G.r1[1]) / G.d13 : 0.0;
-  const double a1z = G.d13 > 1.0e-5 ? (G.rna[2] - G.r1[2]) / G.d13 : 0.0;
-  const double a2x = G.d23 > 1.0e-5 ? (G.rna[0] - G.r2[0]) / G.d23 : 0.0;
-  const double a2y = G.d23 > 1.0e-5 ? (G.rna[1] - G.r2[1]) / G.d23 : 0.0;
-  const double a2z = G.d23 > 1.0e-5 ? (G.rna[2] - G.r2[2]) / G.d23 : 0.0;
-  Q.rA1 = pick3(a1x, a1y, a1z, q);
-  Q.rA2 = pick3(a2x, a2y, a2z, q);
-}
-
-// Depsilon_3c slices of component ix = q + 1 from component scalars
-__device__ __forceinline__ void d3_slice_q(const DGeo3s &G, const D3Scal &S, const DGeoQ &Q, int ix, double *dA,
-                                           double *dB) {
-#define E3(i, j) G.eps[3 * ((j) - 1) + (i) - 1]
-#define SA(imu, k) dA[((imu) - 1) + 3 * ((k) - 1)]
-#define SB(imu, k) dB[((imu) - 1) + 3 * ((k) - 1)]
-#pragma unroll
-  for (int i = 0; i < 9; i++) { dA[i] = 0.0; dB[i] = 0.0; }
-  if (S.zero) return;
-  const double cm = S.crossmag;
-#pragma unroll
-  for (int imu = 1; imu <= 3; imu++) {
-    double sum = d_levi(ix, imu, 1) * (G.r2[0] - G.r1[0]) + d_levi(ix, imu, 2) * (G.r2[1] - G.r1[1]) +
-                 d_levi(ix, imu, 3) * (G.r2[2] - G.r1[2]);
-    SA(imu, 2) = (1.0 / cm) * (sum - (E3(imu, 2) / cm) *
-                                         ((S.r1mag2 + S.r2mag2 - 2.0 * S.r1dotr2) * Q.raq +
-                                          (S.r1dotr2 - S.r1mag2 - S.r2dotratm + S.r1dotratm) * Q.r2q +
-                                          (S.r1dotr2 - S.r2mag2 + S.r2dotratm - S.r1dotratm) * Q.r1q));
-  }
-  SA(1, 1) = E3(3, 3) * SA(2, 2) - E3(2, 3) * SA(3, 2);
-  SA(2, 1) = E3(1, 3) * SA(3, 2) - E3(3, 3) * SA(1, 2);
-  SA(3, 1) = E3(2, 3) * SA(1, 2) - E3(1, 3) * SA(2, 2);
-#pragma unroll
-  for (int imu = 1; imu <= 3; imu++) {
-    SB(imu, 3) = (1.0 / G.z) * (E3(imu, 3) * Q.e3q - d_delk(imu, ix));
-    double sum = d_levi(ix, imu, 1) * (G.rna[0] - G.r2[0]) + d_levi(ix, imu, 2) * (G.rna[1] - G.r2[1]) +
-                 d_levi(ix, imu, 3) * (G.rna[2] - G.r2[2]);
-    SB(imu, 2) = (1.0 / cm) * (sum - (E3(imu, 2) / cm) *
-                                         ((S.r2dotratm - S.r1dotratm + S.r1dotr2 - S.r2mag2) * Q.raq +
-                                          (S.r2dotratm + S.r1dotratm - S.r1dotr2 - S.ratmmag2) * Q.r2q +
-                                          (S.ratmmag2 - 2.0 * S.r2dotratm + S.r2mag2) * Q.r1q));
-  }
-  SB(1, 1) = E3(3, 3) * SB(2, 2) - E3(3, 2) * SB(2, 3) - E3(2, 3) * SB(3, 2) + E3(2, 2) * SB(3, 3);
-  SB(2, 1) = E3(1, 3) * SB(3, 2) - E3(1, 2) * SB(3, 3) - E3(3, 3) * SB(1, 2) + E3(3, 2) * SB(1, 3);
-  SB(3, 1) = E3(2, 3) * SB(1, 2) - E3(2, 2) * SB(1, 3) - E3(1, 3) * SB(2, 2) + E3(1, 2) * SB(2, 3);
-#undef E3
-#undef SA
-#undef SB
-}
-
-// component q of the neutral (charged = false) or one charged shell's forces of
-// a triplet, continuing (a, b, c): f3naa, f3nab, f3nac sums
-template <int CLS, bool CHG>
-__device__ __forceinline__ void force3c_q(const DView &v, const DForce &Fo, const DGeo3s &G, const D3Scal &S,
-                                          const DGeoQ &Q, int q, int64_t bo, const double *row, double dQ,
-                                          double stinky, double dstA, double dstB, double dstC, double &a, double &b,
-                                          double &c) {
-  constexpr int NME = nme3c_of(CLS);
-  constexpr int NMU = (CLS & 2) ? 4 : 1, NNU = (CLS & 1) ? 4 : 1;
-  double pm[9], sA[9], sB[9], dpA[9], dpB[9], F[NME], Ma[NME], Mb[NME];
-  d_pmat<double>(G.eps, pm);
-  d3_slice_q(G, S, Q, q + 1, sA, sB);
-  dpmat_slice(sA, dpA);
-  dpmat_slice(sB, dpB);
-#pragma unroll
-  for (int m = 0; m < NME; m++) {
-    F[m] = row[m];
-    const double dp = row[NME + m];
-    Ma[m] = Q.rh * row[2 * NME + m] + Q.am * dp;
-    Mb[m] = -Q.sg * row[3 * NME + m] + Q.bm * dp - Ma[m] / 2.0;
-  }
-  const double *sb = v.mat[FB_MAT_S] + bo, *db = v.mat[FB_MAT_DIP] + bo;
-  const double *sD = Fo.dmat[0] + 3 * bo, *dD = Fo.dmat[2] + 3 * bo;
-  const double d13sq = G.d13 * G.d13, d23sq = G.d23 * G.d23;
-#pragma unroll
-  for (int col = 0; col < NNU; col++)
-#pragma unroll
-    for (int row_ = 0; row_ < NMU; row_++) {
-      const int i = row_ + NMU * col;
-      const double xa = drot3c_el<CLS>(row_, col, pm, dpA, F, Ma);
-      const double xb = drot3c_el<CLS>(row_, col, pm, dpB, F, Mb);
-      const double xc = -xa - xb;
-      if (!CHG) {
-        const double r = Fo.rho[bo + i];
-        a = a - r * xa * FB_P_EQ2;
-        b = b - r * xb * FB_P_EQ2;
-        c = c - r * xc * FB_P_EQ2;
-      } else {
-        const double bx = rot3c_el<CLS>(row_, col, pm, F);
-        const double sterm = sb[i] / 2.0, dterm = db[i] / G.z;
-        const double emnpl = (sterm - dterm) / G.d13 + (sterm + dterm) / G.d23;
-        const double spterm = sD[q + 3 * i] / 2.0;
-        double dpterm = dD[q + 3 * i] / G.z;
-        dpterm = dpterm + dterm * Q.sg / G.z;
-        const double dA = -((sterm - dterm) * Q.rA1 / d13sq) - (sterm + dterm) * Q.rA2 / d23sq;
-        const double dB = (sterm - dterm) * Q.rA1 / d13sq + (spterm - dpterm) / G.d13 + (spterm + dpterm) / G.d23;
-        const double dC = -dA - dB;
-        const double w = FB_P_EQ2 * dQ * Fo.rho[bo + i];
-        a = a - w * (stinky * xa + dstA * bx - dstA * emnpl + (1.0 - stinky) * dA);
-        b = b - w * (stinky * xb + dstB * bx - dstB * emnpl + (1.0 - stinky) * dB);
-        c = c - w * (stinky * xc + dstC * bx - dstC * emnpl + (1.0 - stinky) * dC);
-      }
-    }
-}
-
-template <bool CHG>
-__device__ __forceinline__ void force3c_dispatch(int cls, const DView &v, const DForce &Fo, const DGeo3s &G,
-                                                 const D3Scal &S, const DGeoQ &Q, int q, int64_t bo, const double *row,
-                                                 double dQ, double st, double dA, double dB, double dC, double &a,
-                                                 double &b, double &c) {
-  switch (cls) {
-    case 3: force3c_q<3, CHG>(v, Fo, G, S, Q, q, bo, row, dQ, st, dA, dB, dC, a, b, c); break;
-    case 2: force3c_q<2, CHG>(v, Fo, G, S, Q, q, bo, row, dQ, st, dA, dB, dC, a, b, c); break;
-    case 1: force3c_q<1, CHG>(v, Fo, G, S, Q, q, bo, row, dQ, st, dA, dB, dC, a, b, c); break;
-    default: force3c_q<0, CHG>(v, Fo, G, S, Q, q, bo, row, dQ, st, dA, dB, dC, a, b, c); break;
-  }
-}
-
-// The per-triplet forces go to three arrays in the order in which they are
-// summed per atom: f3a (on ialpha) in list order, f3b (on iatom) in target-pair
-// order, f3c (on jatom) in jatom order; component q of each.
-template <bool MX>
-__global__ __launch_bounds__(T3Q) void k_d3c_sp(DView v, DForce Fo) {
-  __shared__ double sI[T3Q / 4][SIROW];
-  const int slot = threadIdx.x >> 2, q = threadIdx.x & 3;
-  const int64_t t = xcd_tile(blockIdx.x, gridDim.x) * (T3Q / 4) + slot;
-  if (t >= v.ntrip) return;
-  const int4 tr = Fo.trip[t];
-  const int in1 = v.imass[tr.y], in2 = v.imass[tr.z], indna = v.imass[tr.x];
-  const int cls = (v.sp.norb[in1 - 1] == 4 ? 2 : 0) + (v.sp.norb[in2 - 1] == 4 ? 1 : 0);
-  const int nme = cls == 3 ? 10 : (cls == 0 ? 1 : 3);
-  double x, z, cost;
-  xzc3(v, tr, false, x, z, cost);
-  double *row = sI[slot];
-  const int gid0 = group3c_of(v, in1, in2, indna, 0);
-  int status = MX ? stage_q_mx(v, gid0, nme, x, z, cost, row, q) : stage_q(v, gid0, nme, x, z, cost, row, q);
-  // the four lanes of a triplet sit in one wavefront: a wavefront barrier
-  // orders phase A's LDS writes before phase B's reads
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  status |= __shfl_xor(status, 1, 4) | __shfl_xor(status, 2, 4);
-  if (q < 3) {
-    double a = 0.0, b = 0.0, c = 0.0;
-    if (!status) {
-      DGeo3s G;
-      d_dgeo3s(v, tr, false, G);
-      D3Scal S;
-      d3_scal(G.r1, G.r2, G.r21, G.rna, G.rnabc, S);
-      DGeoQ Q;
-      geo_q(G, q, Q);
-      force3c_dispatch<false>(cls, v, Fo, G, S, Q, q, v.boff[Fo.tpair[t]], row, 0.0, 0.0, 0.0, 0.0, 0.0, a, b, c);
-    }
-    Fo.f3a[3 * t + q] = a;
-    Fo.f3b[3 * (int64_t)Fo.inv_perm[t] + q] = b;
-    Fo.f3c[3 * (int64_t)Fo.inv_perm_j[t] + q] = c;
-  }
-  if (status && q == 0) atomicOr(v.status, status);
-}
-
-// charged shells (M_Dassemble_3c_DOGS.f90:460-776): continues each triplet's
-// neutral sums with every isorp whose dQ is not zero
-__global__ __launch_bounds__(T3Q) void k_d3c_sp_q(DView v, DForce Fo) {
-  __shared__ double sI[T3Q / 4][SIROW];
-  const int slot = threadIdx.x >> 2, q = threadIdx.x & 3;
-  const int64_t t = xcd_tile(blockIdx.x, gridDim.x) * (T3Q / 4) + slot;
-  if (t >= v.ntrip) return;
-  const int4 tr = Fo.trip[t];
-  const int indna = v.imass[tr.x];
-  bool charged = false;
-  for (int isorp = 1; isorp <= v.sp.nssh[indna - 1]; isorp++) charged |= (v.dQ[tr.x * FB_MAXSH + isorp - 1] != 0.0);
-  if (!charged) return;
-  const int in1 = v.imass[tr.y], in2 = v.imass[tr.z];
-  const int cls = (v.sp.norb[in1 - 1] == 4 ? 2 : 0) + (v.sp.norb[in2 - 1] == 4 ? 1 : 0);
-  const int nme = cls == 3 ? 10 : (cls == 0 ? 1 : 3);
-  const int64_t bo = v.boff[Fo.tpair[t]];
-  DGeo3s G;
-  d_dgeo3s(v, tr, true, G);
-  D3Scal S;
-  d3_scal(G.r1, G.r2, G.r21, G.rna, G.rnabc, S);
-  DGeoQ Q;
-  geo_q(G, q < 3 ? q : 0, Q);
-  const double rc3 = v.sp.rcmin[indna - 1];
-  const double rend1 = v.sp.rcmin[in1 - 1] + rc3, rend2 = v.sp.rcmin[in2 - 1] + rc3;
-  const double st13 = d_smoother(G.d13, rend1, 0.8), dst13 = d_Dsmoother(G.d13, rend1, 0.8);
-  const double st23 = d_smoother(G.d23, rend2, 0.8), dst23 = d_Dsmoother(G.d23, rend2, 0.8);
-  const double stinky = st13 * st23;
-  const double dstB = -dst13 * st23 * Q.rA1;
-  const double dstC = -st13 * dst23 * Q.rA2;
-  const double dstA = -dstB - dstC;
-  double *row = sI[slot];
-  double a = 0.0, b = 0.0, c = 0.0;
-  const int64_t ob = 3 * (int64_t)Fo.inv_perm[t] + q, oc = 3 * (int64_t)Fo.inv_perm_j[t] + q;
-  if (q < 3) {
-    a = Fo.f3a[3 * t + q];
-    b = Fo.f3b[ob];
-    c = Fo.f3c[oc];
-  }
-  int status = 0;
-  for (int isorp = 1; isorp <= v.sp.nssh[indna - 1]; isorp++) {
-    const double dQ = v.dQ[tr.x * FB_MAXSH + isorp - 1];
-    if (dQ == 0.0) continue;
-    int st = stage_q(v, group3c_of(v, in1, in2, indna, isorp), nme, G.x, G.z, G.cost, row, q);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    st |= __shfl_xor(st, 1, 4) | __shfl_xor(st, 2, 4);
-    status |= st;
-    if (!st && q < 3)
-      force3c_dispatch<true>(cls, v, Fo, G, S, Q, q, bo, row, dQ, stinky, dstA, dstB, dstC, a, b, c);
-    // the row is rewritten by the next shell: reads of this one complete first
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-  if (q < 3) {
-    Fo.f3a[3 * t + q] = a;
-    Fo.f3b[ob] = b;
-    Fo.f3c[oc] = c;
-  }
-  if (status && q == 0) atomicOr(v.status, status);
-}
+#include "fb_d3c_wave.h"
 
 extern "C" int fbk_d2c_sp(const DView &v, const DForce &f, int mask, hipStream_t st) {
   if (v.npairs == 0) return 0;
@@ -2025,13 +1185,37 @@ extern "C" int fbk_d2c_sp(const DView &v, const DForce &f, int mask, hipStream_t
   return (int)hipGetLastError();
 }
 
-// charged = 0: the neutral pass only (every shell charge of the batch is zero);
-// mixed = 1: the FP32 interpolation of the neutral pass
+// charged = 0: every shell charge of the batch is zero; mixed = 1: the FP32
+// interpolation of the neutral term
 extern "C" int fbk_d3c_sp(const DView &v, const DForce &f, int charged, int mixed, hipStream_t st) {
-  if (v.ntrip == 0) return 0;
-  const dim3 grid((unsigned)((v.ntrip + T3Q / 4 - 1) / (T3Q / 4)));
-  if (mixed) hipLaunchKernelGGL(k_d3c_sp<true>, grid, dim3(T3Q), 0, st, v, f);
-  else hipLaunchKernelGGL(k_d3c_sp<false>, grid, dim3(T3Q), 0, st, v, f);
-  if (charged) hipLaunchKernelGGL(k_d3c_sp_q, grid, dim3(T3Q), 0, st, v, f);
+  if (v.ntrip > 0) {
+    const dim3 grid((unsigned)v.ntiles[0]);
+    if (charged) {
+      hipLaunchKernelGGL(k_d3c_pair, dim3((unsigned)((v.npairs + 255) / 256)), dim3(256), 0, st, v, f);
+      if (mixed) hipLaunchKernelGGL((k_d3c_wave<true, true>), grid, dim3(64), 0, st, v, f);
+      else hipLaunchKernelGGL((k_d3c_wave<false, true>), grid, dim3(64), 0, st, v, f);
+    } else {
+      if (mixed) hipLaunchKernelGGL((k_d3c_wave<true, false>), grid, dim3(64), 0, st, v, f);
+      else hipLaunchKernelGGL((k_d3c_wave<false, false>), grid, dim3(64), 0, st, v, f);
+    }
+  }
+  return (int)hipGetLastError();
+}
+
+// per-atom sums of fbk_d3c_sp's forces
+extern "C" int fbk_d3c_sp_sum(const DView &v, const DForce &f, hipStream_t st) {
+  if (v.natoms == 0) return 0;
+  hipLaunchKernelGGL(k_d3c_fix, dim3((unsigned)((v.natoms + 63) / 64)), dim3(64), 0, st, v, f);
+  hipLaunchKernelGGL(k_d3c_atom, dim3(v.natoms), dim3(256), 0, st, v, f);
+  hipLaunchKernelGGL(k_d3c_back, dim3(v.natoms), dim3(64), 0, st, v, f);
+  return (int)hipGetLastError();
+}
+
+// what these sums need of the lists: each triplet's pair to its third atom,
+// each atom's first segment
+extern "C" int fbk_d3c_sp_lists(const DView &v, int *trip_nb, int *aseg, hipStream_t st) {
+  if (v.ntrip > 0)
+    hipLaunchKernelGGL(k_trip_nb, dim3((unsigned)((v.ntrip + 255) / 256)), dim3(256), 0, st, v, trip_nb);
+  hipLaunchKernelGGL(k_atom_seg, dim3((unsigned)((v.natoms + 256) / 256)), dim3(256), 0, st, v, aseg);
   return (int)hipGetLastError();
 }

@@ -66,3 +66,40 @@ def test_lattice_with_coincident_images():
     lat = np.array([[12.0, 0.0, 0.0], [-14.4, 0.0, 0.0], [0.0, 0.0, 12.0]])
     pos = np.array([[1.0, 0.3, 0.2], [1.0, 0.1, 0.9], [1.0, 1.4, 0.5]])   # apart across the repeat of 2.4 A only
     check([synth.H_SP], [synth.Structure(pos, np.ones(3, np.int32), lat, 0)])
+
+
+@pytest.mark.parametrize("n", [255, 256, 257])
+def test_neighbours_around_the_capacity_of_the_one_pass_search(n):
+    """Every atom sees every other, so the lists are known."""
+    g = 0.62 * np.array(np.meshgrid(*[np.arange(-5, 6)] * 3)).reshape(3, -1).T
+    pos = g[np.argsort(np.sum(g * g, axis=1), kind="stable")[:n]]
+    pos += np.random.default_rng(1).uniform(-0.03, 0.03, pos.shape)
+    asm = Assembler(synth.make_tables([synth.SI]), precision="fp64")
+    asm.add_structure(synth.Structure(pos + 20.0, np.ones(n, np.int32), np.diag([40.0] * 3), 1))
+    asm.build_lists()
+    r = asm.lists()
+    assert np.all(r["neighn"] == n) and np.all(r["neigh_b"] == 0)
+    assert np.array_equal(r["neigh_j"].reshape(n, n), np.tile(np.arange(1, n + 1), (n, 1)))
+    assert np.array_equal(r["neigh_back"].reshape(n, n), np.tile(np.arange(1, n + 1)[:, None], (1, n)))
+    assert np.array_equal(r["neigh_self"], np.arange(1, n + 1))
+    asm.close()
+
+
+def test_more_atoms_than_one_workgroup_bins():
+    spatial = pytest.importorskip("scipy.spatial")
+    st = synth.diamond_si((11, 11, 11), sigma=0.05, seed=4)
+    asm = Assembler(synth.make_tables([synth.SI]), precision="fp64")
+    asm.add_structure(st)
+    asm.build_lists()
+    r = asm.lists()
+    box = np.diag(st.lattice)
+    x = np.mod(st.ratom, box)
+    tree = spatial.cKDTree(x, boxsize=box)
+    rng = 2.0 * max(synth.SI.rcutoffA) - 0.01
+    count = np.array([len(q) for q in tree.query_ball_point(x, rng)])
+    assert np.array_equal(r["neighn"], count)
+    # neigh_back is an involution between the pairs
+    off = np.concatenate([[0], np.cumsum(r["neighn"])])
+    back = off[r["neigh_j"] - 1] + r["neigh_back"] - 1
+    assert np.array_equal(back[back], np.arange(len(back)))
+    asm.close()

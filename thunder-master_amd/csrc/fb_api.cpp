@@ -34,14 +34,20 @@ int fbk_tiles_atom(int natoms, const int64_t *pair_off, const int64_t *seg_off, 
                    int ch, int fill, int *cnt, const int64_t *tile_off, int4 *tiles, hipStream_t st);
 int fbk_gather_i64(int n, const int64_t *src, const int64_t *idx, int64_t *dst, hipStream_t st);
 int fbk_cell_count(const DView &v, int *cnt, int *atom_cell, hipStream_t st);
-int fbk_cell_fill(const DView &v, const int *atom_cell, int *cursor, int *cell_atoms, hipStream_t st);
+int fbk_cell_fill(const DView &v, const int *atom_cell, int *cursor, int *cell_atoms, CellAtom *cell_rec,
+                  hipStream_t st);
+int fbk_cells(const DView &v, int ncells, int64_t *cell_start, int *cell_atoms, CellAtom *cell_rec, hipStream_t st);
+int fbk_nb_find(const DView &v, const CellAtom *cell_rec, int *neighn, int *nblk, unsigned *keys, int *neigh_self,
+                int64_t *noff, int64_t *aboff, int64_t *h_off, int *h_status, hipStream_t st);
+int fbk_nb_place(const DView &v, const unsigned *keys, const int64_t *aboff, const NbOut &o, hipStream_t st);
 int fbk_neighbors_fill(const DView &v, const int64_t *noff, int *neigh_j, int *neigh_b, int *neigh_self,
                        int *pair_atom, int *status, hipStream_t st);
 int fbk_neigh_back(const DView &v, int *neigh_back, int *status, hipStream_t st);
 int fbk_common_count(const DView &v, int scan, int *ncommon, hipStream_t st);
 int fbk_common_fill(const DView &v, int scan, const int64_t *toff, int4 *trip, int *trip_pair, hipStream_t st);
 int fbk_targets_nmax(void);
-int fbk_targets_count(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, hipStream_t st);
+int fbk_targets_count(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, int64_t *h_toff,
+                      TgtSum *h_tot, int *h_status, hipStream_t st);
 int fbk_targets_fill(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, const TgtOut &out,
                      hipStream_t st);
 int fbk_block_sizes(const DView &v, int64_t *sz, int4 *rec, hipStream_t st);
@@ -107,6 +113,24 @@ struct DevBuf {
     cap = 0;
   }
   template <typename T> T *as() const { return (T *)p; }
+};
+
+// page-locked host memory that kernels write list sizes to
+struct HostBuf {
+  void *p = nullptr;
+  size_t cap = 0;
+  hipError_t ensure(size_t bytes) {
+    if (bytes <= cap) return hipSuccess;
+    release();
+    hipError_t e = hipHostMalloc(&p, bytes);
+    if (e == hipSuccess) cap = bytes;
+    return e;
+  }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    cap = 0;
+  }
 };
 
 struct HCell2c {
@@ -259,7 +283,14 @@ struct fb_ctx {
   DevBuf d_mat[FB_NMAT];
   int64_t npairs = 0, ntrip = 0, nseg = 0, blen = 0;
   std::vector<int64_t> h_noff, h_toff, h_boff_struct;
-  std::vector<TgtSum> h_tgt;
+  HostBuf h_list;   // natoms + 1 pair, block element and triplet offsets, then ListTail
+  struct ListTail {
+    TgtSum tgt;
+    int status;
+  };
+  int64_t *list_off(int which) const { return (int64_t *)h_list.p + (size_t)which * (natoms + 1); }
+  ListTail *list_tail() const { return (ListTail *)list_off(3); }
+  DevBuf d_cell_rec, d_nblk, d_nb_keys, d_aboff;   // neighbour search in one pass
   int64_t order_ntrip = 0;
   bool lists_ok = false;
   int done[5] = {0, 0, 0, 0, 0};
@@ -572,7 +603,7 @@ struct fb_ctx {
                       &d_mu, &d_nu, &d_mv, &d_grid2c, &d_pden, &d_wg2c, &d_cell_cnt, &d_cell_start, &d_cell_atoms, &d_atom_cell, &d_pair_disp, &d_tile_cnt, &d_tile_off, &d_gidx, &d_gout, &d_st, &d_xl, &d_ratom, &d_imass, &d_atom_struct, &d_dQ,
                       &d_neighn, &d_noff, &d_neigh_j, &d_neigh_b, &d_neigh_back, &d_neigh_self, &d_pair_atom, &d_pair_rec, &d_pair_perm,
                       &d_bsz, &d_boff, &d_ncommon, &d_toff, &d_trip_orig, &d_tpair_orig, &d_trip, &d_tpair,
-                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
+                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_cell_rec, &d_nblk, &d_nb_keys, &d_aboff, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
                       &d_mlp, &d_mlp_err, &d_mlp_count, &d_queue, &d_meth3c,
                       &d_status, &d_idx3r, &d_qin, &d_wbsz, &d_wboff, &d_pp_map, &d_px_map, &d_px_point,
                       &d_inv_pp, &d_inv_px, &d_cand_cnt, &d_cand_off, &d_cand_j, &d_cand_b, &d_pc_n, &d_pc_off,
@@ -589,6 +620,7 @@ struct fb_ctx {
     for (DevBuf *b : fbufs) b->release();
     reset_events();
     for (auto e : pool) (void)hipEventDestroy(e);
+    h_list.release();
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     if (h_status) (void)hipHostFree(h_status);
@@ -1454,6 +1486,31 @@ static int ensure_triplets(fb_ctx *ctx, int64_t T) {
   return FB_OK;
 }
 
+// 2c workgroups: whole atoms, at most 16 atoms and FB_2C_PCAP pairs each (an
+// atom with more neighbours gets a workgroup of its own, run in passes), and
+// the order of the pairs inside
+static int pair_order(fb_ctx *ctx) {
+  std::vector<int> wg;
+  wg.push_back(0);
+  int na = 0;
+  int64_t np = 0;
+  for (int a = 0; a < ctx->natoms; a++) {
+    int64_t n = ctx->h_noff[a + 1] - ctx->h_noff[a];
+    if (na > 0 && (na == 16 || np + n > FB_2C_PCAP)) {
+      wg.push_back(a);
+      na = 0;
+      np = 0;
+    }
+    na++;
+    np += n;
+  }
+  wg.push_back(ctx->natoms);
+  ctx->nwg2c = (int)wg.size() - 1;
+  RC(upload(ctx, ctx->d_wg2c, wg.data(), wg.size() * sizeof(int), "upload wg2c"));
+  DView v = ctx->view();
+  return ctx->launch("pair_perm", [&] { return fbk_pair_perm(v, ctx->d_pair_perm.as<unsigned char>(), ctx->stream); });
+}
+
 // Triplets, segments and tiles formed directly in target order (k_targets):
 // count, scan, fill.
 static int triplets_by_target(fb_ctx *ctx, int nmax) {
@@ -1467,11 +1524,16 @@ static int triplets_by_target(fb_ctx *ctx, int nmax) {
   unsigned long long *mask = ctx->d_tgt_mask.as<unsigned long long>();
   int *cnt = ctx->d_tgt_cnt.as<int>();
   DView v = ctx->view();
-  RC(ctx->launch("targets_count", [&] { return fbk_targets_count(v, nmax, sum, mask, cnt, st); }));
-  ctx->h_tgt.resize(N + 1);
-  FB_HIP(hipMemcpyAsync(ctx->h_tgt.data(), sum, sizeof(TgtSum) * (N + 1), hipMemcpyDeviceToHost, st));
-  FB_HIP(hipStreamSynchronize(st));
-  const TgtSum &tot = ctx->h_tgt[N];
+  fb_ctx::ListTail *tail = ctx->list_tail();
+  RC(ctx->launch("targets_count", [&] {
+    return fbk_targets_count(v, nmax, sum, mask, cnt, ctx->list_off(2), &tail->tgt, &tail->status, st);
+  }));
+  FB_HIP(hipEventRecord(ctx->ev_fork, st));
+  // the 2c kernel's pair order, while the host reads the sizes
+  RC(pair_order(ctx));
+  FB_HIP(hipEventSynchronize(ctx->ev_fork));
+  RC(ctx->decode_status(tail->status, "find_neighbors"));
+  const TgtSum tot = tail->tgt;
   const int64_t T = tot.trip;
   RC(ensure_triplets(ctx, T));
   FB_HIP(ctx->d_seg_off.ensure(sizeof(int64_t) * (tot.seg + 1)));
@@ -1488,7 +1550,7 @@ static int triplets_by_target(fb_ctx *ctx, int nmax) {
   }
   // of an atom's triplets only the structure's totals are kept on the host:
   // the same whether an atom owns the targets or is the third atom
-  for (int i = 0; i <= N; i++) ctx->h_toff[i] = ctx->h_tgt[i].trip;
+  ctx->h_toff.assign(ctx->list_off(2), ctx->list_off(2) + N + 1);
   return ctx->launch("targets_fill", [&] { return fbk_targets_fill(v, nmax, sum, mask, cnt, out, st); });
 }
 
@@ -1596,6 +1658,139 @@ static int triplets_by_sort(fb_ctx *ctx) {
   return FB_OK;
 }
 
+// atoms binned into their structure's cells (counting sort; order inside a
+// cell is free: the search orders its results)
+static int build_cells(fb_ctx *ctx) {
+  if (ctx->cell_bits == 0) return FB_OK;
+  hipStream_t st = ctx->stream;
+  const int N = ctx->natoms;
+  const int64_t C = ctx->ncells;
+  FB_HIP(ctx->d_cell_start.ensure(sizeof(int64_t) * (C + 1)));
+  FB_HIP(ctx->d_cell_atoms.ensure(sizeof(int) * std::max(N, 1)));
+  FB_HIP(ctx->d_cell_rec.ensure(sizeof(CellAtom) * std::max(N, 1)));
+  CellAtom *rec = ctx->d_cell_rec.as<CellAtom>();
+  DView v = ctx->view();
+  // one workgroup up to 8192 atoms: 14 us at 2048 atoms where the separate
+  // launches take 36, and 4 us more per further 1024
+  if (C <= FB_CELLS_ONE && N <= 8192)
+    return ctx->launch("cells", [&] {
+      return fbk_cells(v, (int)C, ctx->d_cell_start.as<int64_t>(), ctx->d_cell_atoms.as<int>(), rec, st);
+    });
+  FB_HIP(ctx->d_cell_cnt.ensure(sizeof(int) * C));
+  FB_HIP(ctx->d_atom_cell.ensure(sizeof(int) * std::max(N, 1)));
+  RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
+  RC(ctx->launch("cell_count", [&] {
+    return fbk_cell_count(v, ctx->d_cell_cnt.as<int>(), ctx->d_atom_cell.as<int>(), st);
+  }));
+  RC(scan_i32(ctx, ctx->d_cell_cnt.as<int>(), ctx->d_cell_start.as<int64_t>(), C));
+  RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
+  v = ctx->view();
+  return ctx->launch("cell_fill", [&] {
+    return fbk_cell_fill(v, ctx->d_atom_cell.as<int>(), ctx->d_cell_cnt.as<int>(), ctx->d_cell_atoms.as<int>(), rec,
+                         st);
+  });
+}
+
+static int ensure_pairs(fb_ctx *ctx) {
+  const int64_t P = ctx->npairs;
+  if (P >= (1ll << 31)) return ctx->fail(FB_E_CAPACITY, "more than 2^31 pairs or triplets");
+  FB_HIP(ctx->d_neigh_j.ensure(sizeof(int) * P));
+  FB_HIP(ctx->d_neigh_b.ensure(sizeof(int) * P));
+  FB_HIP(ctx->d_neigh_back.ensure(sizeof(int) * P));
+  FB_HIP(ctx->d_pair_atom.ensure(sizeof(int) * P));
+  FB_HIP(ctx->d_pair_rec.ensure(sizeof(int4) * std::max<int64_t>(P, 1)));
+  FB_HIP(ctx->d_pair_perm.ensure(std::max<int64_t>(P, 1)));
+  FB_HIP(ctx->d_boff.ensure(sizeof(int64_t) * (P + 1)));
+  FB_HIP(ctx->d_pair_disp.ensure(sizeof(double) * 3 * std::max<int64_t>(P, 1)));
+  FB_HIP(ctx->d_pair_tgt.ensure(sizeof(int) * std::max<int64_t>(P, 1)));
+  return FB_OK;
+}
+
+static int most_neighbors(const fb_ctx *ctx) {
+  int64_t n = 0;
+  for (int i = 0; i < ctx->natoms; i++) n = std::max(n, ctx->h_noff[i + 1] - ctx->h_noff[i]);
+  return (int)std::min<int64_t>(n, 1 << 30);
+}
+
+// The neighbour lists and all pair records from one search; *placed = false:
+// left to neighbors_two_pass (its conditions are above k_nb_find).  The status
+// of the placing kernel is read with the triplets' sizes.
+static int neighbors_one_pass(fb_ctx *ctx, int *nmax, bool *placed) {
+  const int N = ctx->natoms;
+  if (N == 0 || ctx->cell_bits == 0 || any_coincident(ctx)) return FB_OK;
+  hipStream_t st = ctx->stream;
+  FB_HIP(ctx->d_nblk.ensure(sizeof(int) * N));
+  FB_HIP(ctx->d_nb_keys.ensure(sizeof(unsigned) * (size_t)FB_NB_CAP * N));
+  FB_HIP(ctx->d_aboff.ensure(sizeof(int64_t) * (N + 1)));
+  DView v = ctx->view();
+  fb_ctx::ListTail *tail = ctx->list_tail();
+  RC(ctx->launch("neighbors", [&] {
+    return fbk_nb_find(v, ctx->d_cell_rec.as<CellAtom>(), ctx->d_neighn.as<int>(), ctx->d_nblk.as<int>(),
+                       ctx->d_nb_keys.as<unsigned>(), ctx->d_neigh_self.as<int>(), ctx->d_noff.as<int64_t>(),
+                       ctx->d_aboff.as<int64_t>(), ctx->list_off(0), &tail->status, st);
+  }));
+  FB_HIP(hipStreamSynchronize(st));
+  const int *status = &tail->status;
+  if (*status & ST_TOO_CLOSE) return ctx->decode_status(*status, "find_neighbors");
+  ctx->h_noff.assign(ctx->list_off(0), ctx->list_off(0) + N + 1);
+  ctx->npairs = ctx->h_noff[N];
+  *nmax = most_neighbors(ctx);
+  if (*nmax > FB_NB_CAP) return FB_OK;
+  RC(ensure_pairs(ctx));
+  const int64_t *aboff = ctx->list_off(1);
+  ctx->blen = aboff[N];
+  for (size_t k = 0; k < ctx->structs.size(); k++) ctx->h_boff_struct[k] = aboff[ctx->h_st[k].atom_off];
+  ctx->h_boff_struct[ctx->structs.size()] = ctx->blen;
+  NbOut o{ctx->d_neigh_j.as<int>(), ctx->d_neigh_b.as<int>(),    ctx->d_neigh_back.as<int>(), ctx->d_pair_atom.as<int>(),
+          ctx->d_pair_rec.as<int4>(), ctx->d_boff.as<int64_t>(), ctx->d_pair_disp.as<double>()};
+  v = ctx->view();
+  RC(ctx->launch("neighbors_place", [&] {
+    return fbk_nb_place(v, ctx->d_nb_keys.as<unsigned>(), ctx->d_aboff.as<int64_t>(), o, st);
+  }));
+  *placed = true;
+  return *status ? ctx->check_status("find_neighbors") : FB_OK;
+}
+
+// The general form: count, fill, then the pair records in launches of their own
+static int neighbors_two_pass(fb_ctx *ctx, int *nmax) {
+  const int N = ctx->natoms;
+  hipStream_t st = ctx->stream;
+  RC(ctx->clear_status());
+  DView v = ctx->view();
+  RC(ctx->launch("neighbors_count", [&] { return fbk_neighbors_count(v, ctx->d_neighn.as<int>(), v.status, st); }));
+  RC(scan_i32(ctx, ctx->d_neighn.as<int>(), ctx->d_noff.as<int64_t>(), N));
+  FB_HIP(hipMemcpyAsync(ctx->h_noff.data(), ctx->d_noff.p, sizeof(int64_t) * (N + 1), hipMemcpyDeviceToHost, st));
+  RC(ctx->check_status("find_neighbors"));
+  ctx->npairs = ctx->h_noff[N];
+  *nmax = most_neighbors(ctx);
+  const int64_t P = ctx->npairs;
+  RC(ensure_pairs(ctx));
+  FB_HIP(ctx->d_bsz.ensure(sizeof(int64_t) * P));
+  v = ctx->view();
+  RC(ctx->launch("fill_self", [&] { return fbk_fill_i32(ctx->d_neigh_self.as<int>(), N, -999, st); }));
+  RC(ctx->launch("neighbors_fill", [&] {
+    return fbk_neighbors_fill(v, ctx->d_noff.as<int64_t>(), ctx->d_neigh_j.as<int>(), ctx->d_neigh_b.as<int>(),
+                              ctx->d_neigh_self.as<int>(), ctx->d_pair_atom.as<int>(), v.status, st);
+  }));
+  RC(ctx->launch("neigh_back", [&] { return fbk_neigh_back(v, ctx->d_neigh_back.as<int>(), v.status, st); }));
+  RC(ctx->launch("pair_disp", [&] { return fbk_pair_disp(v, ctx->d_pair_disp.as<double>(), st); }));
+  RC(ctx->launch("block_sizes", [&] {
+    return fbk_block_sizes(v, ctx->d_bsz.as<int64_t>(), ctx->d_pair_rec.as<int4>(), st);
+  }));
+  RC(scan_i64(ctx, ctx->d_bsz.as<int64_t>(), ctx->d_boff.as<int64_t>(), P));
+  std::vector<int> self(N);
+  FB_HIP(hipMemcpyAsync(self.data(), ctx->d_neigh_self.p, sizeof(int) * N, hipMemcpyDeviceToHost, st));
+  FB_HIP(hipMemcpyAsync(&ctx->blen, ctx->d_boff.as<int64_t>() + P, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  RC(ctx->check_status("find_neighbors"));
+  for (int i = 0; i < N; i++)
+    if (self[i] == -999) return ctx->fail(FB_E_NEIGH_SELF, "find_neighbors: neigh_self missing");
+  std::vector<int64_t> idx(ctx->structs.size());
+  for (size_t k = 0; k < idx.size(); k++) idx[k] = ctx->h_noff[ctx->h_st[k].atom_off];
+  RC(gather_to_host(ctx, ctx->d_boff.as<int64_t>(), idx, ctx->h_boff_struct.data()));
+  ctx->h_boff_struct[ctx->structs.size()] = ctx->blen;
+  return FB_OK;
+}
+
 int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
   if (!ctx) return FB_E_ARG;
   if (!ctx->tables_ok) return ctx->fail(FB_E_ORDER, "build_lists before commit_tables");
@@ -1608,110 +1803,26 @@ int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
   FB_HIP(ctx->d_neighn.ensure(sizeof(int) * N));
   FB_HIP(ctx->d_noff.ensure(sizeof(int64_t) * (N + 1)));
   FB_HIP(ctx->d_neigh_self.ensure(sizeof(int) * N));
-  if (ctx->cell_bits > 0) {
-    // atoms binned into their structure's cells (counting sort; order inside a
-    // cell is free: the search orders its results through a bitmap)
-    const int64_t C = ctx->ncells;
-    FB_HIP(ctx->d_cell_cnt.ensure(sizeof(int) * C));
-    FB_HIP(ctx->d_cell_start.ensure(sizeof(int64_t) * (C + 1)));
-    FB_HIP(ctx->d_cell_atoms.ensure(sizeof(int) * std::max(N, 1)));
-    FB_HIP(ctx->d_atom_cell.ensure(sizeof(int) * std::max(N, 1)));
-    DView vb = ctx->view();
-    RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
-    RC(ctx->launch("cell_count", [&] {
-      return fbk_cell_count(vb, ctx->d_cell_cnt.as<int>(), ctx->d_atom_cell.as<int>(), st);
-    }));
-    RC(scan_i32(ctx, ctx->d_cell_cnt.as<int>(), ctx->d_cell_start.as<int64_t>(), C));
-    RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
-    vb = ctx->view();
-    RC(ctx->launch("cell_fill", [&] {
-      return fbk_cell_fill(vb, ctx->d_atom_cell.as<int>(), ctx->d_cell_cnt.as<int>(), ctx->d_cell_atoms.as<int>(), st);
-    }));
-  }
-  DView v = ctx->view();
-  RC(ctx->launch("neighbors_count", [&] { return fbk_neighbors_count(v, ctx->d_neighn.as<int>(), v.status, st); }));
-  RC(scan_i32(ctx, ctx->d_neighn.as<int>(), ctx->d_noff.as<int64_t>(), N));
-  ctx->h_noff.resize(N + 1);
-  FB_HIP(hipMemcpyAsync(ctx->h_noff.data(), ctx->d_noff.p, sizeof(int64_t) * (N + 1), hipMemcpyDeviceToHost, st));
-  RC(ctx->check_status("find_neighbors"));
-  ctx->npairs = ctx->h_noff[N];
-  const int64_t P = ctx->npairs;
-  FB_HIP(ctx->d_neigh_j.ensure(sizeof(int) * P));
-  FB_HIP(ctx->d_neigh_b.ensure(sizeof(int) * P));
-  FB_HIP(ctx->d_neigh_back.ensure(sizeof(int) * P));
-  FB_HIP(ctx->d_pair_atom.ensure(sizeof(int) * P));
-  FB_HIP(ctx->d_pair_rec.ensure(sizeof(int4) * std::max<int64_t>(P, 1)));
-  FB_HIP(ctx->d_pair_perm.ensure(std::max<int64_t>(P, 1)));
-  FB_HIP(ctx->d_bsz.ensure(sizeof(int64_t) * P));
-  FB_HIP(ctx->d_boff.ensure(sizeof(int64_t) * (P + 1)));
-  v = ctx->view();
-  RC(ctx->launch("fill_self", [&] { return fbk_fill_i32(ctx->d_neigh_self.as<int>(), N, -999, st); }));
-  RC(ctx->launch("neighbors_fill", [&] {
-    return fbk_neighbors_fill(v, ctx->d_noff.as<int64_t>(), ctx->d_neigh_j.as<int>(), ctx->d_neigh_b.as<int>(),
-                              ctx->d_neigh_self.as<int>(), ctx->d_pair_atom.as<int>(), v.status, st);
-  }));
-  RC(ctx->launch("neigh_back", [&] { return fbk_neigh_back(v, ctx->d_neigh_back.as<int>(), v.status, st); }));
-  FB_HIP(ctx->d_pair_disp.ensure(sizeof(double) * 3 * std::max<int64_t>(P, 1)));
-  FB_HIP(ctx->d_pair_tgt.ensure(sizeof(int) * std::max<int64_t>(P, 1)));
-  ctx->h_toff.resize(N + 1);
-  v = ctx->view();
-  RC(ctx->launch("pair_disp", [&] { return fbk_pair_disp(v, ctx->d_pair_disp.as<double>(), st); }));
-  {
-    std::vector<int> self(N);
-    FB_HIP(hipMemcpyAsync(self.data(), ctx->d_neigh_self.p, sizeof(int) * N, hipMemcpyDeviceToHost, st));
-    RC(ctx->check_status("find_neighbors"));
-    for (int i = 0; i < N; i++)
-      if (self[i] == -999) return ctx->fail(FB_E_NEIGH_SELF, "find_neighbors: neigh_self missing");
-  }
+  FB_HIP(ctx->h_list.ensure(sizeof(int64_t) * 3 * (N + 1) + sizeof(fb_ctx::ListTail)));
+  RC(build_cells(ctx));
   int nmax = 0;
-  for (int i = 0; i < N; i++) nmax = std::max<int64_t>(nmax, ctx->h_noff[i + 1] - ctx->h_noff[i]);
-  if (P >= (1ll << 31)) return ctx->fail(FB_E_CAPACITY, "more than 2^31 pairs or triplets");
+  ctx->h_noff.resize(N + 1);
+  ctx->h_toff.resize(N + 1);
+  ctx->h_boff_struct.resize(ctx->structs.size() + 1);
+  bool placed = false;
+  RC(neighbors_one_pass(ctx, &nmax, &placed));
+  if (!placed) RC(neighbors_two_pass(ctx, &nmax));
+  const int64_t P = ctx->npairs;
   const bool general = nmax > fbk_targets_nmax() || any_coincident(ctx);
+  if (general) RC(pair_order(ctx));
   RC(general ? triplets_by_sort(ctx) : triplets_by_target(ctx, nmax));
   const int64_t T = ctx->ntrip;
-  // block offsets
-  v = ctx->view();
-  RC(ctx->launch("block_sizes", [&] {
-    return fbk_block_sizes(v, ctx->d_bsz.as<int64_t>(), ctx->d_pair_rec.as<int4>(), st);
-  }));
-  RC(scan_i64(ctx, ctx->d_bsz.as<int64_t>(), ctx->d_boff.as<int64_t>(), P));
-  FB_HIP(hipMemcpyAsync(&ctx->blen, ctx->d_boff.as<int64_t>() + P, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  RC(ctx->check_status("find_common_neighbors"));
-  ctx->h_boff_struct.resize(ctx->structs.size() + 1);
-  {
-    std::vector<int64_t> idx(ctx->structs.size());
-    for (size_t k = 0; k < idx.size(); k++) idx[k] = ctx->h_noff[ctx->h_st[k].atom_off];
-    RC(gather_to_host(ctx, ctx->d_boff.as<int64_t>(), idx, ctx->h_boff_struct.data()));
-  }
-  ctx->h_boff_struct[ctx->structs.size()] = ctx->blen;
+  if (general) RC(ctx->check_status("find_common_neighbors"));
   for (int i = 0; i < 5; i++) {
     FB_HIP(ctx->d_mat[i].ensure(sizeof(double) * std::max<int64_t>(ctx->blen, 1)));
     ctx->done[i] = 0;
   }
-  // 2c workgroups: whole atoms, at most 16 atoms and FB_2C_PCAP pairs each (an
-  // atom with more neighbours gets a workgroup of its own, run in passes)
-  {
-    std::vector<int> wg;
-    wg.push_back(0);
-    int na = 0;
-    int64_t np = 0;
-    for (int a = 0; a < N; a++) {
-      int64_t n = ctx->h_noff[a + 1] - ctx->h_noff[a];
-      if (na > 0 && (na == 16 || np + n > FB_2C_PCAP)) {
-        wg.push_back(a);
-        na = 0;
-        np = 0;
-      }
-      na++;
-      np += n;
-    }
-    wg.push_back(N);
-    ctx->nwg2c = (int)wg.size() - 1;
-    RC(upload(ctx, ctx->d_wg2c, wg.data(), wg.size() * sizeof(int), "upload wg2c"));
-    v = ctx->view();
-    RC(ctx->launch("pair_perm", [&] { return fbk_pair_perm(v, ctx->d_pair_perm.as<unsigned char>(), st); }));
-    FB_HIP(hipStreamSynchronize(st));
-  }
+  FB_HIP(hipStreamSynchronize(st));
   ctx->lists_ok = true;
   ctx->lists_gen++;
   if (general) ctx->order_gen = ctx->lists_gen;   // triplets_by_sort formed it

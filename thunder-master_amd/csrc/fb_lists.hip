@@ -15,6 +15,12 @@
 #define LWG 256
 #include "fb_lists_dev.h"
 
+// Atoms up to which the list kernels of one workgroup per atom take 1024
+// threads instead of 256: two such workgroups fit a compute unit, so all run at
+// once.  Measured (targets counted / filled): 96 atoms 39 / 30 -> 30 / 23 us;
+// 1000 atoms, 256 threads 61 / 49, 1024 threads 57 / 60 us.
+#define LIST_WIDE 512
+
 // atoms binned by cell (counting sort of the neighbour search)
 __global__ void k_cell_count(DView v, int *cnt, int *atom_cell) {
   const int ia = blockIdx.x * blockDim.x + threadIdx.x;
@@ -26,12 +32,66 @@ __global__ void k_cell_count(DView v, int *cnt, int *atom_cell) {
   atomicAdd(&cnt[c], 1);
 }
 
-__global__ void k_cell_fill(DView v, const int *atom_cell, int *cursor, int *cell_atoms) {
+__device__ __forceinline__ CellAtom cell_record(const DView &v, int ia) {
+  return CellAtom{{v.ratom[3 * ia], v.ratom[3 * ia + 1], v.ratom[3 * ia + 2]}, v.sp.rcmax[v.imass[ia] - 1]};
+}
+
+__global__ void k_cell_fill(DView v, const int *atom_cell, int *cursor, int *cell_atoms, CellAtom *cell_rec) {
   const int ia = blockIdx.x * blockDim.x + threadIdx.x;
   if (ia >= v.natoms) return;
   const int c = atom_cell[ia];
   const int k = atomicAdd(&cursor[c], 1);
   cell_atoms[v.cell_start[c] + k] = ia - v.st[v.atom_struct[ia]].atom_off;
+  cell_rec[v.cell_start[c] + k] = cell_record(v, ia);
+}
+
+// The same in one launch of one workgroup, for few cells and atoms: clearing,
+// counting, scan and fill are six launches, 36 us at 96 atoms and at 2048
+// where this one takes 7 and 14 us.
+__global__ __launch_bounds__(1024) void k_cells(DView v, int ncells, int64_t *cell_start, int *cell_atoms,
+                                                CellAtom *cell_rec) {
+  __shared__ int s_cnt[FB_CELLS_ONE];
+  __shared__ int s_wave[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int c = tid; c < FB_CELLS_ONE; c += 1024) s_cnt[c] = 0;
+  __syncthreads();
+  auto cell = [&](int ia) {
+    const DStruct &S = v.st[v.atom_struct[ia]];
+    const double r[3] = {v.ratom[3 * ia], v.ratom[3 * ia + 1], v.ratom[3 * ia + 2]};
+    return S.cell_off + cell_of(S, r);
+  };
+  for (int ia = tid; ia < v.natoms; ia += 1024) atomicAdd(&s_cnt[cell(ia)], 1);
+  __syncthreads();
+  int own[FB_CELLS_ONE / 1024], sum = 0;
+#pragma unroll
+  for (int u = 0; u < FB_CELLS_ONE / 1024; u++) {
+    own[u] = s_cnt[tid * (FB_CELLS_ONE / 1024) + u];
+    sum += own[u];
+  }
+  int inc = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(inc, d);
+    if (lane >= d) inc += y;
+  }
+  if (lane == 63) s_wave[wave] = inc;
+  __syncthreads();
+  int at = inc - sum;
+  for (int w = 0; w < wave; w++) at += s_wave[w];
+#pragma unroll
+  for (int u = 0; u < FB_CELLS_ONE / 1024; u++) {
+    const int c = tid * (FB_CELLS_ONE / 1024) + u;
+    s_cnt[c] = at;
+    if (c <= ncells) cell_start[c] = at;
+    at += own[u];
+  }
+  if (tid == 0 && ncells == FB_CELLS_ONE) cell_start[ncells] = v.natoms;
+  __syncthreads();
+  for (int ia = tid; ia < v.natoms; ia += 1024) {
+    const int k = atomicAdd(&s_cnt[cell(ia)], 1);
+    cell_atoms[k] = ia - v.st[v.atom_struct[ia]].atom_off;
+    cell_rec[k] = cell_record(v, ia);
+  }
 }
 
 // FILL = false: count neighbours (find_neigh_max); FILL = true: write them.
@@ -139,6 +199,246 @@ __global__ __launch_bounds__(LWG) void k_neighbors(DView v, int *neighn_out, con
   if (!FILL && threadIdx.x == 0) neighn_out[ia] = count;
 }
 
+// ------------------------------------------------ neighbours in one search
+// The search once instead of twice (count, then fill): a workgroup per atom
+// tests the atoms of all cells of all images that may reach it, a wavefront
+// per cell, keeps the hits in LDS as image << 18 | jatom, and sorts them by
+// rank.  That key order is the reference's list order (mbeta outer, jatom
+// inner).  The sorted keys go to the atom's FB_NB_CAP entries of a scratch
+// array; k_list_scan turns counts into offsets, and k_nb_place writes the
+// lists with all that follows from a pair (displacement, block offset, record)
+// and finds neigh_back by binary search among the partner's keys.
+// k_neighbors and the kernels below serve what this form does not: atoms with
+// more neighbours than FB_NB_CAP, lattices with images within the reference's
+// tolerances of each other, structures without a cell list.
+// Latency-bound: 1024 threads per atom where there are fewer atoms than fill
+// the chip.  Measured with the scans and launches they replace, C/H/N/O of 96
+// atoms / carbon of 2048: 131 / 180 -> 25 / 59 us.
+#define NB_SHIFT 18       // jatom's bits in a key (cell lists are used up to 262,144 atoms)
+
+template <int W>
+__global__ __launch_bounds__(W) void k_nb_find(DView v, const CellAtom *cell_rec, int *neighn, int *nblk,
+                                               unsigned *keys, int *neigh_self, int *status) {
+  constexpr int NI = 64;   // images per round
+  __shared__ int s_img[FB_NIMG];
+  __shared__ int s_cell[NI * 27];
+  __shared__ short s_cimg[NI * 27];
+  __shared__ unsigned s_key[FB_NB_CAP];
+  __shared__ int s_nimg, s_ne, s_n, s_b;
+  const int ia = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int s = v.atom_struct[ia];
+  const DStruct &S = v.st[s];
+  const int li = ia - S.atom_off, in1 = v.imass[ia], norb1 = v.sp.norb[in1 - 1];
+  const double r1[3] = {v.ratom[3 * ia], v.ratom[3 * ia + 1], v.ratom[3 * ia + 2]};
+  const double rci = v.sp.rcmax[in1 - 1], reach = rci + S.rcmax_all + 1.0e-6;
+  const double *xls = v.xl + (int64_t)s * FB_NIMG * 3;
+  if (tid == 0) {
+    s_nimg = 0;
+    s_n = 0;
+    s_b = 0;
+  }
+  __syncthreads();
+  for (int mb = tid; mb <= S.mbeta_max; mb += W)
+    if (image_may_hit(S, xls + 3 * mb, r1, reach)) s_img[atomicAdd(&s_nimg, 1)] = mb;
+  __syncthreads();
+  const int nimg = s_nimg;
+  int blk = 0;
+  bool close = false;
+  for (int i0 = 0; i0 < nimg; i0 += NI) {
+    if (tid == 0) s_ne = 0;
+    __syncthreads();
+    if (tid < NI && i0 + tid < nimg) {
+      // the cells that overlap the box +- crange around r1 in this image (query_cells)
+      const int mb = s_img[i0 + tid];
+      int lo[3], n[3];
+      bool any = true;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        const double q = r1[a] - xls[3 * mb + a];
+        const double fl = floor((q - S.crange - S.clo[a]) / S.cw[a]);
+        const double fh = floor((q + S.crange - S.clo[a]) / S.cw[a]);
+        any = any && !(fh < 0.0 || fl > (double)(S.cn[a] - 1));
+        lo[a] = (int)fmin(fmax(fl, 0.0), (double)(S.cn[a] - 1));
+        n[a] = max(min((int)fmin(fh, (double)(S.cn[a] - 1)) - lo[a] + 1, 3), 0);
+      }
+      const int nc = any ? n[0] * n[1] * n[2] : 0;
+      const int at = atomicAdd(&s_ne, nc);
+      for (int t = 0; t < nc; t++) {
+        const int cx = lo[0] + t % n[0], cy = lo[1] + (t / n[0]) % n[1], cz = lo[2] + t / (n[0] * n[1]);
+        s_cell[at + t] = S.cell_off + (cz * S.cn[1] + cy) * S.cn[0] + cx;
+        s_cimg[at + t] = (short)mb;
+      }
+    }
+    __syncthreads();
+    const int ne = s_ne;
+    for (int e = wave; e < ne; e += W / 64) {
+      const int c = s_cell[e], mb = s_cimg[e];
+      const double x0 = xls[3 * mb], x1 = xls[3 * mb + 1], x2 = xls[3 * mb + 2];
+      const int64_t k1 = v.cell_start[c + 1];
+      for (int64_t k0 = v.cell_start[c]; k0 < k1; k0 += 64) {
+        const int64_t k = k0 + lane;
+        int lj = 0;
+        bool hit = false;
+        if (k < k1) {
+          lj = v.cell_atoms[k];
+          const CellAtom a = cell_rec[k];
+          const double r2[3] = {a.r[0] + x0, a.r[1] + x1, a.r[2] + x2};
+          const double z = d_distance(r1, r2);
+          close |= lj != li && z < 0.5;
+          hit = z < rci + a.rc - 0.01;
+          if (hit) blk += norb1 * v.sp.norb[v.imass[S.atom_off + lj] - 1];
+        }
+        const unsigned long long m = __ballot(hit);
+        if (m == 0) continue;
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&s_n, __popcll(m));
+        at = __builtin_amdgcn_readfirstlane(at) + __popcll(m & ((1ull << lane) - 1ull));
+        if (hit && at < FB_NB_CAP) s_key[at] = ((unsigned)mb << NB_SHIFT) | (unsigned)lj;
+      }
+    }
+    __syncthreads();
+  }
+  if (close) atomicOr(status, ST_TOO_CLOSE);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) blk += __shfl_xor(blk, d);
+  if (lane == 0 && blk) atomicAdd(&s_b, blk);
+  __syncthreads();
+  const int n = s_n;
+  if (tid == 0) {
+    neighn[ia] = n;
+    nblk[ia] = s_b;
+  }
+  if (n > FB_NB_CAP) return;   // the general kernels take the whole build
+  bool self = false;
+  for (int i = tid; i < n; i += W) {
+    const unsigned key = s_key[i];
+    int rank = 0;
+    for (int j = 0; j < n; j++) rank += s_key[j] < key ? 1 : 0;
+    keys[(int64_t)ia * FB_NB_CAP + rank] = key;
+    if (key == (unsigned)li) {
+      neigh_self[ia] = rank + 1;
+      self = true;
+    }
+  }
+  if (!__syncthreads_or(self) && tid == 0) {
+    neigh_self[ia] = -999;
+    atomicOr(status, ST_SELF);
+  }
+}
+
+// offsets of every atom's neighbours and block elements, on the device and in
+// page-locked host memory (h_off: [natoms+1] pairs, [natoms+1] elements), and
+// the status word
+__global__ __launch_bounds__(1024) void k_list_scan(int natoms, const int *neighn, const int *nblk, int64_t *noff,
+                                                    int64_t *aboff, int64_t *h_off, const int *status,
+                                                    int *h_status) {
+  __shared__ int64_t s_w[16][2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int64_t run[2] = {0, 0};
+  for (int a0 = 0; a0 < natoms; a0 += 4096) {
+    const int a = a0 + 4 * tid;
+    int64_t e[4][2], mine[2] = {0, 0}, inc[2];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      e[u][0] = a + u < natoms ? neighn[a + u] : 0;
+      e[u][1] = a + u < natoms ? nblk[a + u] : 0;
+      mine[0] += e[u][0];
+      mine[1] += e[u][1];
+    }
+    inc[0] = mine[0];
+    inc[1] = mine[1];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t y0 = __shfl_up(inc[0], d), y1 = __shfl_up(inc[1], d);
+      if (lane >= d) {
+        inc[0] += y0;
+        inc[1] += y1;
+      }
+    }
+    if (lane == 63) {
+      s_w[wave][0] = inc[0];
+      s_w[wave][1] = inc[1];
+    }
+    __syncthreads();
+    int64_t off[2] = {run[0] + inc[0] - mine[0], run[1] + inc[1] - mine[1]};
+    for (int w = 0; w < 16; w++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        if (w < wave) off[q] += s_w[w][q];
+        run[q] += s_w[w][q];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (a + u < natoms) {
+        noff[a + u] = off[0];
+        aboff[a + u] = off[1];
+        h_off[a + u] = off[0];
+        h_off[natoms + 1 + a + u] = off[1];
+        off[0] += e[u][0];
+        off[1] += e[u][1];
+      }
+  }
+  if (tid == 0) {
+    noff[natoms] = run[0];
+    aboff[natoms] = run[1];
+    h_off[natoms] = run[0];
+    h_off[2 * natoms + 1] = run[1];
+    *h_status = *status;
+  }
+}
+
+// a wavefront per atom
+__global__ __launch_bounds__(256) void k_nb_place(DView v, const unsigned *keys, const int64_t *aboff, NbOut o,
+                                                  int *status) {
+  const int ia = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (ia >= v.natoms) return;
+  const int s = v.atom_struct[ia], off = v.st[s].atom_off, li = ia - off;
+  const int n = v.neighn[ia], in1 = v.imass[ia], norb1 = v.sp.norb[in1 - 1];
+  const int64_t p0 = v.noff[ia];
+  int64_t b = aboff[ia];
+  const double *xls = v.xl + (int64_t)s * FB_NIMG * 3;
+  for (int k0 = 0; k0 < n; k0 += 64) {
+    const int k = k0 + lane;
+    const bool on = k < n;
+    const unsigned key = on ? keys[(int64_t)ia * FB_NB_CAP + k] : 0u;
+    const int lj = (int)(key & ((1u << NB_SHIFT) - 1u)), mb = (int)(key >> NB_SHIFT), ja = off + lj;
+    const int in2 = v.imass[ja], size = on ? norb1 * v.sp.norb[in2 - 1] : 0;
+    int inc = size;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(inc, d);
+      if (lane >= d) inc += y;
+    }
+    if (on) {
+      const int64_t p = p0 + k;
+      o.neigh_j[p] = lj + 1;
+      o.neigh_b[p] = mb;
+      o.pair_atom[p] = ia;
+      o.rec[p] = make_int4(ia, ja, s * FB_NIMG + mb, in1 | (in2 << 16));
+      o.boff[p] = b + inc - size;
+#pragma unroll
+      for (int q = 0; q < 3; q++) o.disp[3 * p + q] = xls[3 * mb + q] + v.ratom[3 * ja + q] - v.ratom[3 * ia + q];
+      int c[3];
+      image_coords(mb, c);
+      const unsigned want = ((unsigned)image_of(-c[0], -c[1], -c[2]) << NB_SHIFT) | (unsigned)li;
+      const unsigned *kj = keys + (int64_t)ja * FB_NB_CAP;
+      const int nj = v.neighn[ja];
+      int lo = 0, hi = nj;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (kj[mid] < want) lo = mid + 1;
+        else hi = mid;
+      }
+      const bool found = lo < nj && kj[lo] == want;
+      if (!found) atomicOr(status, ST_BACK);
+      o.neigh_back[p] = found ? lo + 1 : -999;
+    }
+    b += __shfl(inc, 63);
+  }
+  if (ia == v.natoms - 1 && lane == 0) o.boff[p0 + n] = b;
+}
+
 // displacement of every neighbour pair, xl(jbeta) + r_j - r_i with the
 // reference's evaluation order (M_neighbors.f90:766-769 compares it with r2 - r1)
 __global__ void k_pair_disp(DView v, double *disp) {
@@ -205,11 +505,11 @@ __global__ void k_neigh_back(DView v, int *neigh_back, int *status) {
 #define TGT_LDS(FILL) (((FILL) ? 0 : 56) + 20 + 4)
 #define TGT_NMAX 768      // neighbours per atom: 61 KB
 
-template <bool FILL>
-__global__ __launch_bounds__(LWG) void k_targets(DView v, TgtSum *sum, unsigned long long *mask, int nword, int *pcnt,
+template <bool FILL, int W>
+__global__ __launch_bounds__(W) void k_targets(DView v, TgtSum *sum, unsigned long long *mask, int nword, int *pcnt,
                                                  TgtOut out) {
   extern __shared__ __align__(16) unsigned char s_mem[];
-  __shared__ int s_wave[LWG / 64];
+  __shared__ int s_wave[W / 64];
   const int ia = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int s = v.atom_struct[ia];
   const DStruct S = v.st[s];
@@ -222,7 +522,7 @@ __global__ __launch_bounds__(LWG) void k_targets(DView v, TgtSum *sum, unsigned 
   unsigned short *sSeg = reinterpret_cast<unsigned short *>(sPre + n), *sOrd = sSeg + n;
   const int in1 = v.imass[ia];
   const double rc1 = v.sp.rcmax[in1 - 1];
-  for (int k = tid; k < n; k += LWG) {
+  for (int k = tid; k < n; k += W) {
     const int at = S.atom_off + v.neigh_j[o + k] - 1, b = v.neigh_b[o + k];
     int c[3];
     image_coords(b, c);
@@ -243,7 +543,7 @@ __global__ __launch_bounds__(LWG) void k_targets(DView v, TgtSum *sum, unsigned 
   }
   __syncthreads();
   // order of the neighbours by (ialpha, ib); the entries are distinct
-  for (int k = tid; k < n; k += LWG) {
+  for (int k = tid; k < n; k += W) {
     const int at = sAt[k], ib = sIb[k];
     int rank = 0;
     for (int j = 0; j < n; j++) rank += (sAt[j] < at || (sAt[j] == at && sIb[j] < ib)) ? 1 : 0;
@@ -254,11 +554,11 @@ __global__ __launch_bounds__(LWG) void k_targets(DView v, TgtSum *sum, unsigned 
     base = sum[ia];
     // first triplet and segment of every target
     int run = 0, srun = 0;
-    for (int k0 = 0; k0 < n; k0 += LWG) {
+    for (int k0 = 0; k0 < n; k0 += W) {
       const int k = k0 + tid, c = k < n ? sCnt[k] : 0;
       int tot, stot;
-      const int pos = run + block_scan_count(c, s_wave, &tot);
-      const int sg = srun + block_rank(c > 0, s_wave, &stot);
+      const int pos = run + block_scan_count<W>(c, s_wave, &tot);
+      const int sg = srun + block_rank<W>(c > 0, s_wave, &stot);
       if (k < n) {
         sPre[k] = pos;
         sSeg[k] = (unsigned short)sg;
@@ -274,7 +574,7 @@ __global__ __launch_bounds__(LWG) void k_targets(DView v, TgtSum *sum, unsigned 
     if (ia == v.natoms - 1 && tid == 0) out.seg_off[base.seg + srun] = base.trip + run;
   }
   __syncthreads();
-  for (int p = wave; p < n; p += LWG / 64) {
+  for (int p = wave; p < n; p += W / 64) {
     const int ja = sAt[p], cp = sImg[p];
     const int px = (cp & 15) - 4, py = (cp >> 4 & 15) - 4, pz = (cp >> 8 & 15) - 4;
     const bool target = !(ja == ia && px == 0 && py == 0 && pz == 0);   // not the self entry
@@ -377,7 +677,8 @@ __global__ __launch_bounds__(LWG) void k_targets(DView v, TgtSum *sum, unsigned 
 
 // exclusive prefix of the atoms' totals in place (entry natoms: the totals);
 // one workgroup, four atoms per thread and pass
-__global__ __launch_bounds__(1024) void k_target_scan(int natoms, TgtSum *sum) {
+__global__ __launch_bounds__(1024) void k_target_scan(int natoms, TgtSum *sum, int64_t *h_toff, TgtSum *h_tot,
+                                                      const int *status, int *h_status) {
   __shared__ int64_t s_t[16];
   __shared__ int s_i[16][4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -425,13 +726,21 @@ __global__ __launch_bounds__(1024) void k_target_scan(int natoms, TgtSum *sum) {
     off.seg += inc.seg - mine.seg;
     for (int c = 0; c < 3; c++) off.tile[c] += inc.tile[c] - mine.tile[c];
     for (int u = 0; u < 4; u++) {
-      if (a + u < natoms) sum[a + u] = off;
+      if (a + u < natoms) {
+        sum[a + u] = off;
+        h_toff[a + u] = off.trip;
+      }
       off.trip += e[u].trip;
       off.seg += e[u].seg;
       for (int c = 0; c < 3; c++) off.tile[c] += e[u].tile[c];
     }
   }
-  if (tid == 0) sum[natoms] = run;
+  if (tid == 0) {
+    sum[natoms] = run;
+    h_toff[natoms] = run.trip;
+    *h_tot = run;
+    *h_status = *status;
+  }
 }
 
 // common neighbours of ialpha in the reference's list order (fb_get_common,
@@ -634,10 +943,33 @@ int fbk_cell_count(const DView &v, int *cnt, int *atom_cell, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-int fbk_cell_fill(const DView &v, const int *atom_cell, int *cursor, int *cell_atoms, hipStream_t st) {
+int fbk_cell_fill(const DView &v, const int *atom_cell, int *cursor, int *cell_atoms, CellAtom *cell_rec,
+                  hipStream_t st) {
   if (v.natoms == 0) return 0;
   hipLaunchKernelGGL(k_cell_fill, dim3((unsigned)((v.natoms + 255) / 256)), dim3(256), 0, st, v, atom_cell, cursor,
-                     cell_atoms);
+                     cell_atoms, cell_rec);
+  return (int)hipGetLastError();
+}
+int fbk_cells(const DView &v, int ncells, int64_t *cell_start, int *cell_atoms, CellAtom *cell_rec, hipStream_t st) {
+  if (ncells > FB_CELLS_ONE) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_cells, dim3(1), dim3(1024), 0, st, v, ncells, cell_start, cell_atoms, cell_rec);
+  return (int)hipGetLastError();
+}
+int fbk_nb_find(const DView &v, const CellAtom *cell_rec, int *neighn, int *nblk, unsigned *keys, int *neigh_self,
+                int64_t *noff, int64_t *aboff, int64_t *h_off, int *h_status, hipStream_t st) {
+  if (v.natoms == 0) return (int)hipErrorInvalidValue;
+  if (v.natoms <= LIST_WIDE)
+    hipLaunchKernelGGL(k_nb_find<1024>, dim3((unsigned)v.natoms), dim3(1024), 0, st, v, cell_rec, neighn, nblk, keys,
+                       neigh_self, v.status);
+  else
+    hipLaunchKernelGGL(k_nb_find<256>, dim3((unsigned)v.natoms), dim3(256), 0, st, v, cell_rec, neighn, nblk, keys,
+                       neigh_self, v.status);
+  hipLaunchKernelGGL(k_list_scan, dim3(1), dim3(1024), 0, st, v.natoms, neighn, nblk, noff, aboff, h_off, v.status,
+                     h_status);
+  return (int)hipGetLastError();
+}
+int fbk_nb_place(const DView &v, const unsigned *keys, const int64_t *aboff, const NbOut &o, hipStream_t st) {
+  hipLaunchKernelGGL(k_nb_place, dim3((unsigned)((v.natoms + 3) / 4)), dim3(256), 0, st, v, keys, aboff, o, v.status);
   return (int)hipGetLastError();
 }
 
@@ -692,19 +1024,31 @@ int fbk_common_fill(const DView &v, int scan, const int64_t *toff, int4 *trip, i
 // most neighbours per atom that the target-order kernels take
 int fbk_targets_nmax(void) { return TGT_NMAX; }
 
-int fbk_targets_count(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, hipStream_t st) {
+int fbk_targets_count(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, int64_t *h_toff,
+                      TgtSum *h_tot, int *h_status, hipStream_t st) {
   if (nmax > TGT_NMAX) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_targets<false>, dim3((unsigned)v.natoms), dim3(LWG), TGT_LDS(false) * (size_t)nmax, st, v, sum,
-                     mask, (nmax + 63) / 64, pcnt, TgtOut{});
-  hipLaunchKernelGGL(k_target_scan, dim3(1), dim3(1024), 0, st, v.natoms, sum);
+  const dim3 grid((unsigned)v.natoms);
+  const size_t lds = TGT_LDS(false) * (size_t)nmax;
+  if (v.natoms <= LIST_WIDE)
+    hipLaunchKernelGGL((k_targets<false, 1024>), grid, dim3(1024), lds, st, v, sum, mask, (nmax + 63) / 64, pcnt,
+                       TgtOut{});
+  else
+    hipLaunchKernelGGL((k_targets<false, LWG>), grid, dim3(LWG), lds, st, v, sum, mask, (nmax + 63) / 64, pcnt,
+                       TgtOut{});
+  hipLaunchKernelGGL(k_target_scan, dim3(1), dim3(1024), 0, st, v.natoms, sum, h_toff, h_tot, v.status,
+                     h_status);
   return (int)hipGetLastError();
 }
 
 int fbk_targets_fill(const DView &v, int nmax, TgtSum *sum, unsigned long long *mask, int *pcnt, const TgtOut &out,
                      hipStream_t st) {
   if (nmax > TGT_NMAX) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_targets<true>, dim3((unsigned)v.natoms), dim3(LWG), TGT_LDS(true) * (size_t)nmax, st, v, sum,
-                     mask, (nmax + 63) / 64, pcnt, out);
+  const dim3 grid((unsigned)v.natoms);
+  const size_t lds = TGT_LDS(true) * (size_t)nmax;
+  if (v.natoms <= LIST_WIDE)
+    hipLaunchKernelGGL((k_targets<true, 1024>), grid, dim3(1024), lds, st, v, sum, mask, (nmax + 63) / 64, pcnt, out);
+  else
+    hipLaunchKernelGGL((k_targets<true, LWG>), grid, dim3(LWG), lds, st, v, sum, mask, (nmax + 63) / 64, pcnt, out);
   return (int)hipGetLastError();
 }
 

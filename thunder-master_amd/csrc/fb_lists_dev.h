@@ -9,6 +9,7 @@
 
 // ordered block-wide exclusive scan of a predicate; returns this thread's
 // position, writes the block total to *total (all threads)
+template <int W = LWG>
 __device__ __forceinline__ int block_rank(bool pred, int *s_wave, int *total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned long long m = __ballot(pred);
@@ -17,7 +18,7 @@ __device__ __forceinline__ int block_rank(bool pred, int *s_wave, int *total) {
   __syncthreads();
   int off = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < LWG / 64; w++) {
+  for (int w = 0; w < W / 64; w++) {
     int c = s_wave[w];
     if (w < wave) off += c;
     tot += c;
@@ -42,6 +43,7 @@ __device__ __forceinline__ bool image_may_hit(const DStruct &S, const double *xl
 
 // ordered block-wide exclusive scan of per-thread counts; returns this
 // thread's offset, writes the block total to *total (all threads)
+template <int W = LWG>
 __device__ __forceinline__ int block_scan_count(int c, int *s_wave, int *total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int x = c;
@@ -54,7 +56,7 @@ __device__ __forceinline__ int block_scan_count(int c, int *s_wave, int *total) 
   __syncthreads();
   int off = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < LWG / 64; w++) {
+  for (int w = 0; w < W / 64; w++) {
     const int t = s_wave[w];
     if (w < wave) off += t;
     tot += t;

@@ -334,7 +334,7 @@ int fb_mlp_gradients_noalloc(fb_ctx *ctx, int nme, const float *params, int n, c
  * FB_TUNE_GRAPH: 1 (default) replays fb_assemble_all from a captured HIP
  * graph, 0 enqueues its launches directly.  FB_TUNE_FORCE_KERNEL: the force
  * kernels for s/p species, 1 (default) = compile-time block shapes, 0 = the
- * generic shell loops; both give the same values.  The McWEDA density and
+ * generic shell loops; their values agree to rounding.  The McWEDA density and
  * pseudopotential kernels follow the same switch.
  * FB_TUNE_FUSED: 0 runs the neutral mixed-precision H+S build as two
  * launches (2c, then 3c, the 2c one on a second stream), 3 or 4 as one

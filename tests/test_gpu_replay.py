@@ -1,0 +1,47 @@
+"""Builds replayed from a graph that is updated for new lists, other charges and
+another precision: every one, with eager work and host synchronisations in
+between, equals the eager result."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from fireball_hip import synth
+from fireball_hip.lib import HS_MATS, Assembler
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("charged", [False, True])
+def test_updated_graph_equals_eager_builds(charged):
+    sp = synth.CHNO_SPECIES
+    st = synth.random_box(synth.chno_counts(40), 1.0, 0.9, 5, sp)
+    other = st.ratom + np.random.default_rng(2).normal(0.0, 0.02, st.ratom.shape)
+    dq = np.random.default_rng(3).normal(0.0, 0.05, (2, st.natoms, 4)) * np.array([1.0, 1.0, 0.0, 0.0])
+
+    def build(asm, k):
+        if charged:
+            q = np.ascontiguousarray(dq[k % 2])
+            asm._check(asm.L.fb_set_charges(asm.h, 0, q.ctypes.data_as(C.POINTER(C.c_double))))
+        asm.assemble_all()
+        return {m: asm.blocks(m) for m in HS_MATS}
+
+    asm = Assembler(synth.make_tables(sp), precision="fp64")
+    asm.add_structure(st)
+    for step in range(3):
+        asm.set_positions(0, other if step % 2 else st.ratom)
+        asm.build_lists()
+        for precision in ("fp64", "mixed"):
+            asm.set_precision(precision)
+            asm.enable_timing(True)   # eager launches
+            eager = [build(asm, k) for k in range(2)]
+            asm.timings(64)
+            asm.enable_timing(False)
+            for k in range(4):
+                got = build(asm, k)
+                for m in HS_MATS:
+                    assert np.array_equal(got[m], eager[k % 2][m]), (step, precision, k, m)
+                if k == 1:
+                    asm.assemble_S()
+                    asm.synchronize()
+    asm.close()

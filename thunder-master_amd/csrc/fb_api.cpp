@@ -34,6 +34,7 @@ int fbk_tiles_atom(int natoms, const int64_t *pair_off, const int64_t *seg_off, 
                    int ch, int fill, int *cnt, const int64_t *tile_off, int4 *tiles, hipStream_t st);
 int fbk_gather_i64(int n, const int64_t *src, const int64_t *idx, int64_t *dst, hipStream_t st);
 int fbk_cell_count(const DView &v, int *cnt, int *atom_cell, hipStream_t st);
+int fbk_copy_in(const void *src, void *dst, int64_t n16, hipStream_t st);
 int fbk_cell_fill(const DView &v, const int *atom_cell, int *cursor, int *cell_atoms, CellAtom *cell_rec,
                   hipStream_t st);
 int fbk_cells(const DView &v, int ncells, int64_t *cell_start, int *cell_atoms, CellAtom *cell_rec, hipStream_t st);
@@ -268,11 +269,18 @@ struct fb_ctx {
   int nwg2c = 0;
 
   std::vector<HStruct> structs;
-  bool structs_dirty = true;
+  bool structs_dirty = true, charges_dirty = false;
   std::vector<DStruct> h_st;
   std::vector<int> h_imass;
   int natoms = 0;
-  DevBuf d_st, d_xl, d_ratom, d_imass, d_atom_struct, d_dQ, d_qin;
+  // what the structures put on the device, in one block and one copy
+  DevBuf d_in;
+  HostBuf h_in;
+  hipEvent_t ev_in = nullptr;    // the last copy out of h_in
+  enum { IN_RATOM, IN_DQ, IN_QIN, IN_XL, IN_ST, IN_IMASS, IN_ASTR, IN_N };
+  size_t in_off[IN_N] = {0};
+  template <typename T> T *in(int k) const { return (T *)((char *)d_in.p + in_off[k]); }
+  bool cells_ok = false;         // the cells are those of the uploaded structures
 
   DevBuf d_neighn, d_noff, d_neigh_j, d_neigh_b, d_neigh_back, d_neigh_self, d_pair_atom, d_pair_rec, d_pair_perm, d_bsz, d_boff;
   DevBuf d_ncommon, d_toff, d_trip_orig, d_tpair_orig, d_trip, d_tpair, d_perm_in, d_perm, d_flag, d_segincl,
@@ -469,13 +477,13 @@ struct fb_ctx {
     v.cell_bits = cell_bits;
     v.nstruct = (int)structs.size();
     v.natoms = natoms;
-    v.st = d_st.as<DStruct>();
-    v.xl = d_xl.as<double>();
-    v.ratom = d_ratom.as<double>();
-    v.imass = d_imass.as<int>();
-    v.atom_struct = d_atom_struct.as<int>();
-    v.dQ = d_dQ.as<double>();
-    v.qin = d_qin.as<double>();
+    v.st = in<DStruct>(IN_ST);
+    v.xl = in<double>(IN_XL);
+    v.ratom = in<double>(IN_RATOM);
+    v.imass = in<int>(IN_IMASS);
+    v.atom_struct = in<int>(IN_ASTR);
+    v.dQ = in<double>(IN_DQ);
+    v.qin = in<double>(IN_QIN);
     v.npairs = npairs;
     v.neighn = d_neighn.as<int>();
     v.noff = d_noff.as<int64_t>();
@@ -600,12 +608,12 @@ struct fb_ctx {
 
   ~fb_ctx() {
     DevBuf *bufs[] = {&d_cell2c, &d_idx2c, &d_grp3c, &d_idx3c, &d_tab2c, &d_tab2c32, &d_tab3c, &d_tab3c32, &d_tab3c32q,
-                      &d_mu, &d_nu, &d_mv, &d_grid2c, &d_pden, &d_wg2c, &d_cell_cnt, &d_cell_start, &d_cell_atoms, &d_atom_cell, &d_pair_disp, &d_tile_cnt, &d_tile_off, &d_gidx, &d_gout, &d_st, &d_xl, &d_ratom, &d_imass, &d_atom_struct, &d_dQ,
+                      &d_mu, &d_nu, &d_mv, &d_grid2c, &d_pden, &d_wg2c, &d_cell_cnt, &d_cell_start, &d_cell_atoms, &d_atom_cell, &d_pair_disp, &d_tile_cnt, &d_tile_off, &d_gidx, &d_gout, &d_in,
                       &d_neighn, &d_noff, &d_neigh_j, &d_neigh_b, &d_neigh_back, &d_neigh_self, &d_pair_atom, &d_pair_rec, &d_pair_perm,
                       &d_bsz, &d_boff, &d_ncommon, &d_toff, &d_trip_orig, &d_tpair_orig, &d_trip, &d_tpair,
                       &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_cell_rec, &d_nblk, &d_nb_keys, &d_aboff, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
                       &d_mlp, &d_mlp_err, &d_mlp_count, &d_queue, &d_meth3c,
-                      &d_status, &d_idx3r, &d_qin, &d_wbsz, &d_wboff, &d_pp_map, &d_px_map, &d_px_point,
+                      &d_status, &d_idx3r, &d_wbsz, &d_wboff, &d_pp_map, &d_px_map, &d_px_point,
                       &d_inv_pp, &d_inv_px, &d_cand_cnt, &d_cand_off, &d_cand_j, &d_cand_b, &d_pc_n, &d_pc_off,
                       &d_pc_trip, &d_pc_tpair, &d_pc_trip_s, &d_pc_tpair_s, &d_pc_perm_in, &d_pc_perm, &d_pc_flag,
                       &d_pc_segincl, &d_pc_seg_off, &d_pc_seg_pair, &d_pc_trip_seg, &d_pc_tgt, &d_pc_mp, &d_pc_tiles, &d_ppp_disp, &d_pk_size, &d_pk_off, &d_pk_key, &d_pk_idx, &d_sv_bsz, &d_sv_off,
@@ -621,6 +629,8 @@ struct fb_ctx {
     reset_events();
     for (auto e : pool) (void)hipEventDestroy(e);
     h_list.release();
+    h_in.release();
+    if (ev_in) (void)hipEventDestroy(ev_in);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     if (h_status) (void)hipHostFree(h_status);
@@ -746,6 +756,7 @@ int fb_create(fb_ctx **out, int device) {
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->ev_in, hipEventDisableTiming);
   if (e != hipSuccess) return create_failed(ctx, "streams", e);
   e = scratch_take(device, &ctx->scratch_slot, &ctx->scratch);
   if (e != hipSuccess) return create_failed(ctx, "scratch address", e);
@@ -1313,7 +1324,7 @@ int fb_set_charges(fb_ctx *ctx, int is, const double *dQ) {
   auto &s = ctx->structs[is];
   std::fill(s.dQ.begin(), s.dQ.end(), 0.0);
   if (dQ) std::memcpy(s.dQ.data(), dQ, sizeof(double) * s.natoms * FB_MAXSH);
-  ctx->structs_dirty = true;  // charges change no list, but must be re-uploaded
+  ctx->charges_dirty = true;  // charges change no list, but must be re-uploaded
   // only the Vna blocks depend on the shell charges: S, T and dipole_z stay valid,
   // as in a self-consistent loop that re-assembles Vna per charge update
   ctx->done[FB_MAT_VNA] = ctx->done[FB_MAT_VNAO] = 0;
@@ -1330,14 +1341,45 @@ int fb_set_qin(fb_ctx *ctx, int is, const double *qin) {
   return FB_OK;
 }
 
+// [off, off + bytes) of the staged inputs to the device.  Up to 1 MB a kernel
+// reads the page-locked memory itself: it follows the stream's kernels
+// directly, where a copy engine is waited for (build with new charges of 501
+// atoms: seven copies 159 us, one by the engine 168 us, by the kernel 147 us).
+static int send_in(fb_ctx *ctx, size_t off, size_t bytes) {
+  char *dst = (char *)ctx->d_in.p + off;
+  const char *src = (const char *)ctx->h_in.p + off;
+  if (bytes <= (1u << 20)) {
+    const int rc = fbk_copy_in(src, dst, (int64_t)((bytes + 15) / 16), ctx->stream);
+    if (rc) return ctx->fail(FB_E_HIP, "upload structures", (hipError_t)rc);
+  } else {
+    FB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+  }
+  FB_HIP(hipEventRecord(ctx->ev_in, ctx->stream));
+  return FB_OK;
+}
+
 static int upload_structures(fb_ctx *ctx) {
   const int ns = (int)ctx->structs.size();
   int natoms = 0;
   for (auto &s : ctx->structs) natoms += s.natoms;
   ctx->natoms = natoms;
-  std::vector<double> ratom((size_t)natoms * 3), dq((size_t)natoms * FB_MAXSH), xl((size_t)ns * FB_NIMG * 3, 0.0);
-  std::vector<double> qin((size_t)natoms * FB_MAXSH, 0.0);
-  std::vector<int> imass(natoms), astr(natoms);
+  const size_t bytes[fb_ctx::IN_N] = {sizeof(double) * 3 * natoms,          sizeof(double) * FB_MAXSH * natoms,
+                                      sizeof(double) * FB_MAXSH * natoms,   sizeof(double) * 3 * FB_NIMG * ns,
+                                      sizeof(DStruct) * ns,                 sizeof(int) * natoms,
+                                      sizeof(int) * natoms};
+  size_t total = 0;
+  for (int k = 0; k < fb_ctx::IN_N; k++) {
+    ctx->in_off[k] = total;
+    total += (bytes[k] + 255) & ~(size_t)255;
+  }
+  FB_HIP(hipEventSynchronize(ctx->ev_in));
+  FB_HIP(ctx->h_in.ensure(total));
+  FB_HIP(ctx->d_in.ensure(total));
+  auto at = [&](int k) { return (char *)ctx->h_in.p + ctx->in_off[k]; };
+  for (int k : {(int)fb_ctx::IN_QIN, (int)fb_ctx::IN_XL}) std::memset(at(k), 0, bytes[k]);
+  double *const ratom = (double *)at(fb_ctx::IN_RATOM), *const dq = (double *)at(fb_ctx::IN_DQ);
+  double *const qin = (double *)at(fb_ctx::IN_QIN), *const xl = (double *)at(fb_ctx::IN_XL);
+  int *const imass = (int *)at(fb_ctx::IN_IMASS), *const astr = (int *)at(fb_ctx::IN_ASTR);
   ctx->h_st.assign(ns, DStruct{});
   int off = 0, max_atoms = 0;
   int64_t ncells = 0;
@@ -1393,16 +1435,32 @@ static int upload_structures(fb_ctx *ctx) {
   ctx->ncells = ncells;
   // per-image bitmap of the neighbour search in LDS (32 KB at most), else the full scan
   ctx->cell_bits = (max_atoms <= 262144 && ncells < (1ll << 31)) ? (max_atoms + 31) / 32 : 0;
-  ctx->h_imass = imass;
-  RC(upload(ctx, ctx->d_ratom, ratom.data(), ratom.size() * sizeof(double), "upload ratom"));
-  RC(upload(ctx, ctx->d_imass, imass.data(), imass.size() * sizeof(int), "upload imass"));
-  RC(upload(ctx, ctx->d_atom_struct, astr.data(), astr.size() * sizeof(int), "upload atom_struct"));
-  RC(upload(ctx, ctx->d_dQ, dq.data(), dq.size() * sizeof(double), "upload dQ"));
-  RC(upload(ctx, ctx->d_qin, qin.data(), qin.size() * sizeof(double), "upload Qin"));
-  RC(upload(ctx, ctx->d_xl, xl.data(), xl.size() * sizeof(double), "upload xl"));
-  RC(upload(ctx, ctx->d_st, ctx->h_st.data(), ctx->h_st.size() * sizeof(DStruct), "upload structs"));
-  ctx->structs_dirty = false;
+  ctx->h_imass.assign(imass, imass + natoms);
+  std::memcpy(at(fb_ctx::IN_ST), ctx->h_st.data(), sizeof(DStruct) * ns);
+  RC(send_in(ctx, 0, total));
+  ctx->cells_ok = false;
+  ctx->structs_dirty = ctx->charges_dirty = false;
   return FB_OK;
+}
+
+// after fb_set_charges: the charges alone
+static int upload_charges(fb_ctx *ctx) {
+  FB_HIP(hipEventSynchronize(ctx->ev_in));
+  const size_t off = ctx->in_off[fb_ctx::IN_DQ];
+  char *at = (char *)ctx->h_in.p + off;
+  for (auto &s : ctx->structs) {
+    const size_t n = sizeof(double) * FB_MAXSH * s.natoms;
+    std::memcpy(at, s.dQ.data(), n);
+    at += n;
+  }
+  RC(send_in(ctx, off, at - ((char *)ctx->h_in.p + off)));
+  ctx->charges_dirty = false;
+  return FB_OK;
+}
+
+static int upload_changes(fb_ctx *ctx) {
+  if (ctx->structs_dirty) return upload_structures(ctx);
+  return ctx->charges_dirty ? upload_charges(ctx) : FB_OK;
 }
 
 static int ensure_tmp(fb_ctx *ctx, size_t bytes) {
@@ -1661,7 +1719,7 @@ static int triplets_by_sort(fb_ctx *ctx) {
 // atoms binned into their structure's cells (counting sort; order inside a
 // cell is free: the search orders its results)
 static int build_cells(fb_ctx *ctx) {
-  if (ctx->cell_bits == 0) return FB_OK;
+  if (ctx->cell_bits == 0 || ctx->cells_ok) return FB_OK;
   hipStream_t st = ctx->stream;
   const int N = ctx->natoms;
   const int64_t C = ctx->ncells;
@@ -1670,6 +1728,7 @@ static int build_cells(fb_ctx *ctx) {
   FB_HIP(ctx->d_cell_rec.ensure(sizeof(CellAtom) * std::max(N, 1)));
   CellAtom *rec = ctx->d_cell_rec.as<CellAtom>();
   DView v = ctx->view();
+  ctx->cells_ok = true;
   // one workgroup up to 8192 atoms: 14 us at 2048 atoms where the separate
   // launches take 36, and 4 us more per further 1024
   if (C <= FB_CELLS_ONE && N <= 8192)
@@ -1896,7 +1955,7 @@ static int pre_assemble(fb_ctx *ctx, const char *what) {
   if (!ctx->lists_ok) return ctx->fail(FB_E_ORDER, (std::string(what) + " before build_lists").c_str());
   FB_HIP(hipSetDevice(ctx->device));
   RC(ctx->settle("previous assemble_all"));
-  if (ctx->structs_dirty) RC(upload_structures(ctx));
+  RC(upload_changes(ctx));
   RC(ctx->clear_status());
   return FB_OK;
 }
@@ -2024,7 +2083,9 @@ static int enqueue_build(fb_ctx *ctx, int charged) {
 
 // One H+S build as fb_assemble_all runs it: replayed from the captured graph
 // (captured again when its key changes), or enqueued directly with per-kernel
-// timing, with graphs off or on the null stream.
+// timing, with graphs off or on the null stream.  A geometry step changes the
+// key and leaves the graph's nodes: the executable graph is then updated with
+// the new launches (1 us), where destroying and instantiating it took 140 us.
 static int launch_build(fb_ctx *ctx, int charged) {
   if (ctx->timing || !ctx->use_graph || ctx->stream == nullptr) return enqueue_build(ctx, charged);
   // the graph holds kernel arguments by value: any change of lists, precision,
@@ -2033,8 +2094,7 @@ static int launch_build(fb_ctx *ctx, int charged) {
                          ctx->method3c) * 8 + ctx->fused) * 2 + ctx->persist) * 2 + ctx->k2c) * 4096) +
                    (ctx->mlp_gen & 4095);
   if (ctx->graph_key != key || !ctx->gexec) {
-    if (ctx->gexec) { (void)hipGraphExecDestroy(ctx->gexec); ctx->gexec = nullptr; }
-    if (ctx->graph) { (void)hipGraphDestroy(ctx->graph); ctx->graph = nullptr; }
+    ctx->graph_key = -1;
     FB_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_build(ctx, charged);
     hipGraph_t g = nullptr;
@@ -2044,8 +2104,19 @@ static int launch_build(fb_ctx *ctx, int charged) {
       return rc;
     }
     if (e != hipSuccess) return ctx->fail(FB_E_HIP, "graph capture", e);
+    if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
     ctx->graph = g;
-    FB_HIP(hipGraphInstantiate(&ctx->gexec, g, nullptr, nullptr, 0));
+    if (ctx->gexec) {
+      hipGraphNode_t node = nullptr;
+      hipGraphExecUpdateResult res = hipGraphExecUpdateSuccess;
+      FB_HIP(hipStreamSynchronize(ctx->stream));   // no replay may be reading the arguments
+      if (hipGraphExecUpdate(ctx->gexec, g, &node, &res) != hipSuccess || res != hipGraphExecUpdateSuccess) {
+        (void)hipGetLastError();   // other nodes: a new executable graph
+        (void)hipGraphExecDestroy(ctx->gexec);
+        ctx->gexec = nullptr;
+      }
+    }
+    if (!ctx->gexec) FB_HIP(hipGraphInstantiate(&ctx->gexec, g, nullptr, nullptr, 0));
     ctx->graph_key = key;
   }
   FB_HIP(hipGraphLaunch(ctx->gexec, ctx->stream));
@@ -2061,9 +2132,9 @@ int fb_assemble_all(fb_ctx *ctx) {
   if (!ctx) return FB_E_ARG;
   if (!ctx->lists_ok) return ctx->fail(FB_E_ORDER, "assemble_all before build_lists");
   FB_HIP(hipSetDevice(ctx->device));
-  if (ctx->structs_dirty) {
+  if (ctx->structs_dirty || ctx->charges_dirty) {
     RC(ctx->settle("previous assemble_all"));
-    RC(upload_structures(ctx));
+    RC(upload_changes(ctx));
   }
   RC(launch_build(ctx, any_charge(ctx)));
   ctx->pending = true;
@@ -2729,6 +2800,7 @@ int fb_set_species_pp(fb_ctx *ctx, const int *nssh_pp, const int *lssh_pp, const
   ctx->hpp = h;
   ctx->pp_species = true;
   ctx->pp_lists_ok = false;
+  ctx->structs_dirty = true;   // the cells are as wide as the longest cutoff
   ctx->tables_ok = false;   // the projector tables are checked against the PP shells at commit
   return FB_OK;
 }
@@ -2770,10 +2842,11 @@ int fb_build_lists_pp(fb_ctx *ctx, int64_t *npp, int64_t *nppp, int64_t *ntrip) 
   if (ctx->structs.empty()) return ctx->fail(FB_E_ORDER, "build_lists_pp without structures");
   FB_HIP(hipSetDevice(ctx->device));
   RC(ctx->settle("previous assemble_all"));
-  RC(upload_structures(ctx));
+  RC(upload_changes(ctx));
   RC(ctx->clear_status());
   const int N = ctx->natoms;
   hipStream_t st = ctx->stream;
+  RC(build_cells(ctx));
   RC(pp_list_pass(ctx, PPL_PP));
   RC(pp_list_pass(ctx, PPL_PPX));
   // neighbors_PPp: candidate ranges, first-seen dedup, copy
@@ -3003,7 +3076,7 @@ static int pp_step(fb_ctx *ctx, int step) {
     return ctx->fail(FB_E_ORDER, (std::string(names[step]) + " before " + names[step - 1]).c_str());
   FB_HIP(hipSetDevice(ctx->device));
   RC(ctx->settle("previous assemble_all"));
-  if (ctx->structs_dirty) RC(upload_structures(ctx));
+  RC(upload_changes(ctx));
   RC(ctx->clear_status());
   DView v = ctx->view();
   DPP q = ctx->pview();
@@ -3342,7 +3415,7 @@ int fb_autotune(fb_ctx *ctx, int nrep, int *chosen) {
   if (nrep < 1) nrep = 5;
   FB_HIP(hipSetDevice(ctx->device));
   RC(ctx->settle("assemble_all"));
-  if (ctx->structs_dirty) RC(upload_structures(ctx));
+  RC(upload_changes(ctx));
   struct Events {
     hipEvent_t a = nullptr, b = nullptr;
     ~Events() {

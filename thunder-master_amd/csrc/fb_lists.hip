@@ -21,6 +21,12 @@
 // 1000 atoms, 256 threads 61 / 49, 1024 threads 57 / 60 us.
 #define LIST_WIDE 512
 
+// n16 16-byte words from page-locked host memory
+__global__ void k_copy_in(const int4 *src, int4 *dst, int64_t n16) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n16; i += (int64_t)gridDim.x * blockDim.x)
+    dst[i] = src[i];
+}
+
 // atoms binned by cell (counting sort of the neighbour search)
 __global__ void k_cell_count(DView v, int *cnt, int *atom_cell) {
   const int ia = blockIdx.x * blockDim.x + threadIdx.x;
@@ -943,6 +949,12 @@ int fbk_cell_count(const DView &v, int *cnt, int *atom_cell, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+int fbk_copy_in(const void *src, void *dst, int64_t n16, hipStream_t st) {
+  if (n16 == 0) return 0;
+  hipLaunchKernelGGL(k_copy_in, dim3((unsigned)std::min<int64_t>((n16 + 255) / 256, 256)), dim3(256), 0, st,
+                     (const int4 *)src, (int4 *)dst, n16);
+  return (int)hipGetLastError();
+}
 int fbk_cell_fill(const DView &v, const int *atom_cell, int *cursor, int *cell_atoms, CellAtom *cell_rec,
                   hipStream_t st) {
   if (v.natoms == 0) return 0;

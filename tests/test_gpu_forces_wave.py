@@ -93,3 +93,30 @@ def test_near_collinear(sine, charged):
         synth.random_dQ([st], sp)
     ref = compare(synth.make_tables(sp), st)
     assert np.max(np.abs(ref["f3naa"])) > 0.0
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 6])
+@pytest.mark.parametrize("charged", [False, True])
+def test_pair_forces_on_every_route_equal_the_generic_kernels(n, charged):
+    """Few, some and many pairs: a workgroup per item, several items per workgroup, a lane per pair."""
+    st = synth.diamond_si((n, n, n), sigma=0.05, seed=2)
+    if charged:
+        synth.random_dQ([st], [synth.SI])
+        st.dQ[::5] = 0.0
+    ts = synth.make_tables([synth.SI])
+    got = []
+    for generic in (False, True):
+        asm = Assembler(ts, precision="fp64")
+        asm.add_structure(st)
+        asm.build_lists()
+        asm.assemble_all()
+        if generic:
+            asm.set_tuning(3, 0)
+        r = np.random.default_rng(7).normal(0.0, 0.3, len(asm.blocks("S")))
+        asm.set_denmat(r)
+        asm.dassemble()
+        f = asm.forces()
+        got.append([asm.dblocks(m) for m in ("S", "T", "DIP")] + [f["vna_atom"], f["vna_ontop"]])
+        asm.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

@@ -20,6 +20,8 @@
 // second kernel sums them per atom in three fixed orders (list order for
 // ialpha, target-pair order for iatom, a stable jatom order for jatom) with a
 // fixed wavefront tree: deterministic, no atomics.
+#include <type_traits>
+
 #include "fb_device.h"
 #include "fb_forces.h"
 
@@ -32,19 +34,6 @@ __device__ __forceinline__ double d_levi(int i, int j, int k) {
   return ((i == 1 && j == 2) || (i == 2 && j == 3) || (i == 3 && j == 1)) ? 1.0 : -1.0;
 }
 __device__ __forceinline__ double d_delk(int i, int j) { return i == j ? 1.0 : 0.0; }
-
-// v[k] for a k that is not a compile-time constant, without addressing a
-// private array (which would put it in scratch memory): a blend with exact
-// 0/1 weights, equal to v[k] (finite values)
-__device__ __forceinline__ double sel3(const double *v, int k) {
-  const double w0 = (k == 0) ? 1.0 : 0.0, w1 = (k == 1) ? 1.0 : 0.0, w2 = (k == 2) ? 1.0 : 0.0;
-  return (v[0] * w0 + v[1] * w1) + v[2] * w2;
-}
-__device__ __forceinline__ void put3(double *v, int k, double x) {
-  v[0] = (k == 0) ? x : v[0];
-  v[1] = (k == 1) ? x : v[1];
-  v[2] = (k == 2) ? x : v[2];
-}
 
 #define EPS_(e, i, j) (e)[3 * ((j) - 1) + (i) - 1]
 #define DEP_(d, ix, imu, k) (d)[((ix) - 1) + 3 * ((imu) - 1) + 9 * ((k) - 1)]
@@ -83,6 +72,34 @@ __device__ inline void d_Depsilon_2c(const double *r1, const double *r2, double 
       DEP_(deps, ix, imu, 2) = ic * (sum + (EPS_(eps, imu, 2) * ic) * (r1dotr2 * r2[ix - 1] - r2mag2 * r1[ix - 1]));
       DEP_(deps, ix, imu, 3) = -((d_delk(imu, ix) - EPS_(eps, imu, 3) * EPS_(eps, ix, 3)) * iz);
     }
+}
+
+// the nine of them of one component ix (1-based), [imu - 1 + 3 (k - 1)]
+__device__ __forceinline__ void d_Depsilon_2c_row(const double *r1, const double *r2, double z, const double *eps,
+                                                  int ix, double *dep) {
+#pragma unroll
+  for (int i = 0; i < 9; i++) dep[i] = 0.0;
+  if (z < 1.0e-5) return;
+  double ca0 = r2[1] * r1[2] - r2[2] * r1[1];
+  double ca1 = r2[2] * r1[0] - r2[0] * r1[2];
+  double ca2 = r2[0] * r1[1] - r2[1] * r1[0];
+  double crossmag = sqrt(ca0 * ca0 + ca1 * ca1 + ca2 * ca2);
+  if (fabs(crossmag) < 1.0e-3) return;
+  double r2mag2 = r2[0] * r2[0] + r2[1] * r2[1] + r2[2] * r2[2];
+  double r1dotr2 = r1[0] * r2[0] + r1[1] * r2[1] + r1[2] * r2[2];
+  double iz = 1.0 / z, ic = 1.0 / crossmag;
+  const double r1x = ix == 1 ? r1[0] : (ix == 2 ? r1[1] : r1[2]), r2x = ix == 1 ? r2[0] : (ix == 2 ? r2[1] : r2[2]);
+  const double e3x = ix == 1 ? EPS_(eps, 1, 3) : (ix == 2 ? EPS_(eps, 2, 3) : EPS_(eps, 3, 3));
+#pragma unroll
+  for (int imu = 1; imu <= 3; imu++) {
+    double sum = d_levi(ix, imu, 1) * r2[0] + d_levi(ix, imu, 2) * r2[1] + d_levi(ix, imu, 3) * r2[2];
+    dep[imu - 1] = (EPS_(eps, imu, 1) * e3x * iz) - (EPS_(eps, imu, 1) * (ic * ic)) * (r2mag2 * r1x - r1dotr2 * r2x) +
+                   iz * ic *
+                       (d_delk(imu, ix) * (r2mag2 - r1dotr2) - r1[imu - 1] * r2x - r2[imu - 1] * r2x +
+                        2.0 * r1x * r2[imu - 1]);
+    dep[imu + 2] = ic * (sum + (EPS_(eps, imu, 2) * ic) * (r1dotr2 * r2x - r2mag2 * r1x));
+    dep[imu + 5] = -((d_delk(imu, ix) - EPS_(eps, imu, 3) * e3x) * iz);
+  }
 }
 
 // dera3 = d eps / d ratm and der13 = d eps / d r1 of the 3c frame epsilon(rhat, sighat)
@@ -1170,11 +1187,336 @@ __global__ __launch_bounds__(WD2S) void k_d2c_sp(DView v, DForce Fo, int mask) {
   if (status) atomicOr(v.status, status);
 }
 
+// -------------------------------------------- 2c, s/p, three wavefronts per pair
+// Dblocks of S, T and dipole_z and the vna_ontop and vna_atom forces of a pair
+// (M_Dassemble_2c_DOGS.f90).  A workgroup takes 64 pairs and one of the five
+// items; its three wavefronts hold the same pairs, lane = pair, and wavefront
+// w forms component w of every derivative: the rotation, its derivative and
+// the contraction with the density (the longest part) for one component
+// instead of three.  What the components share is split the same way and
+// exchanged through LDS: the 21 reciprocals of the 7-point window (seven per
+// wavefront), its products and derivative weights (two or three points), the
+// matrix elements (two).  Every value is formed by the reference's operations
+// in their order.
+// Bound by the latency of that dependent binary64 arithmetic: k_d2c_sp's lane
+// per pair needs more than 256 registers (one wavefront per SIMD) and a launch
+// per part.  Charged droplet of 151 atoms, 4245 pairs: 228 -> 44 us.
+#define D2_P 64                 // pairs per workgroup
+
+struct D2Lds {
+  double buf[48 * D2_P];        // Dblocks as they are stored
+  double F[6][D2_P], dF[6][D2_P], prod[7][D2_P], pden[7][D2_P], xsum[7][D2_P];
+  __device__ double *recip() { return buf; }   // [21][D2_P] 1 / (xx_is - xx_ip), is < ip
+};
+
+__device__ __forceinline__ int recip_index(int is, int ip) { return is * (13 - is) / 2 + ip - is - 1; }   // is < ip
+
+// The 7-point window, its products and derivative weights (M_Fdata_2c.f90:
+// 470-540) for the lanes with need set; all three wavefronts call it.
+__device__ __forceinline__ void d2_window(const DView &v, D2Lds &S, int w, int lane, bool need, int grid, double x,
+                                          int &ileft) {
+  double dx = 0.0;
+  if (need) {
+    const DGrid2c gr = grid_scalar(v, grid);
+    dx = gr.dx;
+    ileft = window7(x, gr.dx, gr.nx);
+    for (int k = 0; k < 7; k++) {
+      const int q = 7 * w + k;
+      int is = 0, base = 0;
+      while (q >= base + 6 - is) base += 6 - is++;
+      const int ip = is + 1 + q - base;
+      // the reference's division; the pairs ip < is by exact negation (fl(a - b) = -fl(b - a))
+      S.recip()[q * D2_P + lane] = 1.0 / ((double)(ileft + is - 1) * dx - (double)(ileft + ip - 1) * dx);
+    }
+  }
+  __syncthreads();
+  if (need) {
+    double d[7];
+#pragma unroll
+    for (int k = 0; k < 7; k++) d[k] = x - (double)(ileft + k - 1) * dx;
+    for (int is = w; is < 7; is += 3) {
+      double p = 1.0, q = 1.0, xs = 0.0;
+#pragma unroll
+      for (int ip = 0; ip < 7; ip++)
+        if (ip != is) {
+          const double r = is < ip ? S.recip()[recip_index(is, ip) * D2_P + lane]
+                                   : -S.recip()[recip_index(ip, is) * D2_P + lane];
+          q = q * r;
+          p = p * d[ip] * r;
+        }
+#pragma unroll
+      for (int jp = 0; jp < 7; jp++)
+        if (jp != is) {
+          double xp = 1.0;
+#pragma unroll
+          for (int kp = 0; kp < 7; kp++)
+            if (kp != jp && kp != is) xp = xp * d[kp];
+          xs = xs + xp;
+        }
+      S.prod[is][lane] = p;
+      S.pden[is][lane] = q;
+      S.xsum[is][lane] = xs;
+    }
+  }
+  __syncthreads();
+}
+
+// Values and x-derivatives of one canonical 2c cell (getDMEs_Fdata_2c) into
+// S.F and S.dF, for the lanes with on set; all three wavefronts call it with
+// the same arguments.  Returns the lane's status.
+__device__ __forceinline__ int d2_interp(const DView &v, D2Lds &S, int w, int lane, bool on, int sp2, int slot,
+                                         int isub, double x, int nme, int &grid, int &ileft) {
+  int st = 0;
+  DCell2c c{};
+  if (on) {
+    if (cell_scalar(v, sp2, slot, isub, c) < 0) st = ST_NO_TABLE;
+    else if (x < 0.0) st = ST_X_NEG;
+    else if (x > c.xmax * (1.0 + 1.0e-5)) st = ST_X_RANGE;
+  }
+  const bool go = on && st == 0, origin = x < 1.0e-5, need = go && !origin && c.grid != grid;
+  __syncthreads();   // the last interpolation has been read
+  if (__ballot(need)) {   // the same in all three
+    d2_window(v, S, w, lane, need, c.grid, x, ileft);
+    if (need) grid = c.grid;
+  }
+  if (go) {
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int m = 2 * w + k;
+      if (m >= nme) break;
+      const double *tab = v.tab2c + c.off;
+      double f = 0.0, df = 0.0;
+      if (origin) {
+        f = tab[m];
+      } else {
+        const double *base = tab + (int64_t)(ileft - 1) * nme + m;
+        double b[7];
+#pragma unroll
+        for (int is = 0; is < 7; is++) b[is] = base[is * nme];
+#pragma unroll
+        for (int is = 0; is < 7; is++) f = f + b[is] * S.prod[is][lane];
+#pragma unroll
+        for (int is = 0; is < 7; is++)
+          df = df + b[is] * S.pden[is][lane] * S.xsum[is][lane];
+      }
+      S.F[m][lane] = f;
+      S.dF[m][lane] = df;
+    }
+  }
+  __syncthreads();
+  return st;
+}
+
+// component w of the rotated derivative block of the last interpolation
+template <int CLS>
+__device__ __forceinline__ void d2_block(const D2Lds &S, int lane, const double *pm, const double *dpm, double eta,
+                                         bool far, double *F, double *X) {
+  constexpr int NME = nme2c_of(CLS);
+  double DM[6];
+#pragma unroll
+  for (int m = 0; m < NME; m++) {
+    F[m] = S.F[m][lane];
+    DM[m] = far ? -eta * S.dF[m][lane] : 0.0;
+  }
+  drot2c_sp<CLS>(pm, dpm, F, DM, X);
+}
+
+// f - rho [dq] X P_eq2 over the block
+template <int CLS>
+__device__ __forceinline__ double d2_contract(const D2Lds &S, int lane, const double *pm, const double *dpm, double eta,
+                                              bool far, const double *rho, double dq, bool use_dq, double f) {
+  constexpr int NBL = ((CLS & 2) ? 4 : 1) * ((CLS & 1) ? 4 : 1);
+  double F[6], X[16];
+  d2_block<CLS>(S, lane, pm, dpm, eta, far, F, X);
+#pragma unroll
+  for (int i = 0; i < NBL; i++) {
+    if (use_dq) f = f - rho[i] * dq * X[i] * FB_P_EQ2;
+    else f = f - rho[i] * X[i] * FB_P_EQ2;
+  }
+  return f;
+}
+
+// a charged vna_atom term (M_Dassemble_2c_DOGS.f90:1080-1199)
+template <int CLS>
+__device__ __forceinline__ double d2_charged(const D2Lds &S, int lane, const double *pm, const double *dpm, double eta,
+                                             double z, double smooth, double Dsmooth, const double *rho,
+                                             const double *sself, double dQ, double f) {
+  constexpr int NA = CLS == CLS_SPSP ? 16 : 1;
+  double F[6], X[16], bx[16];
+  d2_block<CLS>(S, lane, pm, dpm, eta, z > 1.0e-4, F, X);
+  rot2c_sp<double>(CLS, pm, F, bx);
+#pragma unroll
+  for (int i = 0; i < NA; i++) {
+    const double emnpl = (z > 1.0e-4) ? sself[i] / z : 0.0;
+    const double vdem = (z > 1.0e-4) ? eta * sself[i] / (z * z) : 0.0;
+    f = f - rho[i] * FB_P_EQ2 * dQ *
+                (smooth * X[i] - eta * Dsmooth * bx[i] + (1.0 - smooth) * vdem + eta * Dsmooth * emnpl);
+  }
+  return f;
+}
+
+// items: 4 bits each, 0 to 2 the Dblock of S, T and dipole_z, 3 vna_ontop, 4 vna_atom
+template <bool CHG>
+__global__ __launch_bounds__(3 * D2_P, 2) void k_d2c_split(DView v, DForce Fo, int items, int nitem) {
+  __shared__ D2Lds S;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t p0 = (int64_t)blockIdx.x * D2_P, pe = min(p0 + (int64_t)D2_P, v.npairs);
+  const int64_t p = p0 + lane;
+  const bool act = p < pe;
+  int ia = 0, ja = 0, in1 = 1, in2 = 1, cls = 0;
+  bool self = false;
+  double z = 0.0, pm[9], dpm[9], eta = 0.0;
+  if (act) {
+    ia = v.pair_atom[p];
+    const int s = v.atom_struct[ia];
+    ja = v.st[s].atom_off + v.neigh_j[p] - 1;
+    const int mb = v.neigh_b[p];
+    in1 = v.imass[ia];
+    in2 = v.imass[ja];
+    const double *xls = v.xl + (int64_t)s * FB_NIMG * 3;
+    double r1[3], r2[3], sighat[3], eps[9], dep[9];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      r1[q] = v.ratom[3 * ia + q];
+      r2[q] = v.ratom[3 * ja + q] + xls[3 * mb + q];
+    }
+    z = d_distance(r1, r2);
+    if (z < 1.0e-5) { sighat[0] = 0.0; sighat[1] = 0.0; sighat[2] = 1.0; }
+    else {
+#pragma unroll
+      for (int q = 0; q < 3; q++) sighat[q] = (r2[q] - r1[q]) / z;
+    }
+    d_epsilon(r2, sighat, eps);
+    d_pmat<double>(eps, pm);
+    d_Depsilon_2c_row(r1, r2, z, eps, w + 1, dep);
+    // d_dpmat of this component
+    dpm[0] = dep[4]; dpm[3] = dep[7]; dpm[6] = dep[1];
+    dpm[1] = dep[5]; dpm[4] = dep[8]; dpm[7] = dep[2];
+    dpm[2] = dep[3]; dpm[5] = dep[6]; dpm[8] = dep[0];
+    eta = w == 0 ? eps[6] : (w == 1 ? eps[7] : eps[8]);
+    self = (ja == ia && mb == 0);
+    cls = (v.sp.norb[in1 - 1] == 4 ? 2 : 0) + (v.sp.norb[in2 - 1] == 4 ? 1 : 0);
+  }
+  const int sp2 = in1 | (in2 << 16), nme = cls == 3 ? 6 : (cls == 0 ? 1 : 2);
+  const bool far = z > 1.0e-3;
+  int status = 0, grid = -1, ileft = 1;
+  for (int k = blockIdx.y; k < nitem; k += gridDim.y) {
+    const int item = items >> (4 * k) & 15;
+    if (item < 3) {
+      const int slot = item == 0 ? SLOT_S : (item == 1 ? SLOT_T : SLOT_DIP);
+      const int st = d2_interp(v, S, w, lane, act, sp2, slot, 0, z, nme, grid, ileft);
+      status |= st;
+      const int64_t b0 = v.boff[p0], nb = 3 * (v.boff[pe] - b0);
+      if (act && !st) {
+        double *const dst = S.buf + 3 * (v.boff[p] - b0) + w;
+        auto put = [&](auto c) {
+          constexpr int CLS = decltype(c)::value, NBL = ((CLS & 2) ? 4 : 1) * ((CLS & 1) ? 4 : 1);
+          double F[6], X[16];
+          d2_block<CLS>(S, lane, pm, dpm, eta, far, F, X);
+#pragma unroll
+          for (int i = 0; i < NBL; i++) dst[3 * i] = X[i];
+        };
+        switch (cls) {
+          case 3: put(std::integral_constant<int, 3>()); break;
+          case 2: put(std::integral_constant<int, 2>()); break;
+          case 1: put(std::integral_constant<int, 1>()); break;
+          default: put(std::integral_constant<int, 0>()); break;
+        }
+      }
+      __syncthreads();
+      // consecutive lanes store consecutive addresses: a lane's own block would leave partly written lines
+      double *const out = Fo.dmat[item] + 3 * b0;
+      for (int64_t k = threadIdx.x; k < nb; k += 3 * D2_P) out[k] = S.buf[k];
+    } else if (item == 3) {
+      // vna_ontop (M_Dassemble_2c_DOGS.f90:679-863): left and right, each its
+      // neutral term and the charged shells of its atom
+      double f = 0.0;
+      const double *rho = Fo.rho + (act ? v.boff[p] : 0);
+      const int nsh = CHG ? 2 : 0;
+      for (int side = 0; side < 2; side++)
+        for (int isorp = 0; isorp <= nsh; isorp++) {
+          bool on = act && !self;
+          double dQ = 0.0;
+          if (on && isorp > 0) {
+            if (isorp <= v.sp.nssh[(side ? in2 : in1) - 1]) dQ = v.dQ[(side ? ja : ia) * FB_MAXSH + isorp - 1];
+            on = dQ != 0.0;
+          }
+          if (!__ballot(on)) continue;   // the same in all three wavefronts
+          const int st = d2_interp(v, S, w, lane, on, sp2, side ? SLOT_ONR : SLOT_ONL, isorp, z, nme, grid, ileft);
+          status |= st;
+          if (!on || st) continue;
+          switch (cls) {
+            case 3: f = d2_contract<3>(S, lane, pm, dpm, eta, far, rho, dQ, isorp > 0, f); break;
+            case 2: f = d2_contract<2>(S, lane, pm, dpm, eta, far, rho, dQ, isorp > 0, f); break;
+            case 1: f = d2_contract<1>(S, lane, pm, dpm, eta, far, rho, dQ, isorp > 0, f); break;
+            default: f = d2_contract<0>(S, lane, pm, dpm, eta, far, rho, dQ, isorp > 0, f); break;
+          }
+        }
+      if (act) Fo.fontop[3 * p + w] = f;
+    } else {
+      // vna_atom (M_Dassemble_2c_DOGS.f90:866-1199) on iatom's orbitals: the
+      // neutral term, then the charged shells of jatom
+      double f = 0.0;
+      const bool sp = cls & 2;
+      const int nmea = sp ? 6 : 1, nsh = CHG ? 2 : 0;
+      const int64_t bself = act ? v.boff[v.noff[ia] + v.neigh_self[ia] - 1] : 0;
+      const double *rho = Fo.rho + bself, *sself = v.mat[FB_MAT_S] + bself;
+      double smooth = 0.0, Dsmooth = 0.0;
+      if (nsh > 0 && act) {
+        const double rend = v.sp.rcmin[in1 - 1] + v.sp.rcmin[in2 - 1];
+        smooth = d_smoother(z, rend, 0.8);
+        Dsmooth = d_Dsmoother(z, rend, 0.8);
+      }
+      for (int isorp = 0; isorp <= nsh; isorp++) {
+        bool on = act;
+        double dQ = 0.0;
+        if (on && isorp > 0) {
+          if (isorp <= v.sp.nssh[in2 - 1]) dQ = v.dQ[ja * FB_MAXSH + isorp - 1];
+          on = dQ != 0.0;
+        }
+        if (!__ballot(on)) continue;
+        const int st = d2_interp(v, S, w, lane, on, sp2, SLOT_ATOM, isorp, z, nmea, grid, ileft);
+        status |= st;
+        if (!on || st) continue;
+        if (isorp == 0)
+          f = sp ? d2_contract<CLS_SPSP>(S, lane, pm, dpm, eta, far, rho, 0.0, false, f)
+                 : d2_contract<CLS_SS>(S, lane, pm, dpm, eta, far, rho, 0.0, false, f);
+        else if constexpr (CHG)
+          f = sp ? d2_charged<CLS_SPSP>(S, lane, pm, dpm, eta, z, smooth, Dsmooth, rho, sself, dQ, f)
+                 : d2_charged<CLS_SS>(S, lane, pm, dpm, eta, z, smooth, Dsmooth, rho, sself, dQ, f);
+      }
+      if (act) Fo.fatom[3 * p + w] = f;
+    }
+  }
+  if (status) atomicOr(v.status, status);
+}
+
 // ---------------------------------------------------------------- 3c, s/p
 #include "fb_d3c_wave.h"
 
+// Few pairs go to k_d2c_split, an item per workgroup up to 128 groups and half
+// of the items above.  With more pairs one lane per pair fills the chip, and
+// the split form's shared arithmetic, done by three wavefronts, is what
+// remains; neutral lists of several rounds of workgroups are its again, whose
+// pairs of other classes diverge in fewer registers.  Measured, k_d2c_sp /
+// split, neutral and charged: Si 7,560 pairs 53 / 27, 120 / 48 us; 17,930 pairs
+// 58 / 39, 120 / 91; 35,016 pairs 70 / 60, 131 / 132; 60,502 pairs 73 / 78,
+// 134 / 175; 143,410 pairs 186 / 167, 353 / 393; C/H/N/O 137,950 pairs 225 /
+// 157, 488 / 399.
 extern "C" int fbk_d2c_sp(const DView &v, const DForce &f, int mask, hipStream_t st) {
   if (v.npairs == 0) return 0;
+  const int64_t groups = (v.npairs + D2_P - 1) / D2_P;
+  if (groups <= 560 || (!v.any_dq && groups >= 1536)) {
+    // the long items first
+    int items = 0, n = 0;
+    for (int item : {3, 4, 0, 1, 2})
+      if (mask & (item < 3 ? 1 << item : 8)) items |= item << (4 * n++);
+    if (n == 0) return 0;
+    const dim3 grid((unsigned)groups, (unsigned)(groups <= 128 ? n : (groups <= 560 ? (n + 1) / 2 : 1)));
+    if (v.any_dq) hipLaunchKernelGGL(k_d2c_split<true>, grid, dim3(3 * D2_P), 0, st, v, f, items, n);
+    else hipLaunchKernelGGL(k_d2c_split<false>, grid, dim3(3 * D2_P), 0, st, v, f, items, n);
+    return (int)hipGetLastError();
+  }
   const dim3 grid((unsigned)((v.npairs + WD2S - 1) / WD2S));
   if (mask & 7) hipLaunchKernelGGL(k_d2c_sp<0>, grid, dim3(WD2S), 0, st, v, f, mask);
   if (mask & 8) {

@@ -317,9 +317,9 @@ int fb_mlp_forward(fb_ctx *ctx, int nme, const float *params, const float *oscal
  * the call allocates nothing, copies nothing to or from the host and does not
  * synchronize (work is enqueued on the context's stream).  n is at most
  * FB_MLP_NOALLOC_MAX_BATCH (FB_E_CAPACITY beyond).  A context has one of the
- * four parts, and a fifth context of a GPU shares one: calls of one context
- * on several streams, or of more than four contexts, that overlap in time on
- * one GPU race, so order them on one stream or synchronize between them.  The
+ * four parts to itself, and one that finds none free gets as much memory in
+ * fb_create.  Calls of one context that overlap in time on several streams
+ * race, so order them on one stream or synchronize between them.  The
  * gradients equal those of fb_mlp_gradients on the same batch. */
 #define FB_MLP_NOALLOC_MAX_BATCH 2048
 int fb_mlp_gradients_noalloc(fb_ctx *ctx, int nme, const float *params, int n, const float *X, const float *T,

@@ -1,6 +1,7 @@
 """Builds replayed from a graph that is updated for new lists, other charges and
-another precision: every one, with eager work and host synchronisations in
-between, equals the eager result."""
+another precision equal the eager builds, with eager work and host
+synchronisations in between; contexts that work at the same time do not share
+work arrays."""
 import ctypes as C
 
 import numpy as np
@@ -8,6 +9,7 @@ import pytest
 
 from fireball_hip import synth
 from fireball_hip.lib import HS_MATS, Assembler
+from test_zz_no_alloc import DeviceArrays
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +47,31 @@ def test_updated_graph_equals_eager_builds(charged):
                     asm.assemble_S()
                     asm.synchronize()
     asm.close()
+
+
+def test_gradients_of_many_contexts_do_not_share_work_arrays():
+    """Seven contexts, each on its own stream, more than the library's fixed
+    scratch has parts: enqueued together, each with its own parameters."""
+    rng = np.random.default_rng(4)
+    n, nm, ts = 2048, 8576, synth.make_tables([synth.SI])
+    asms = [Assembler(ts, precision="mixed") for _ in range(7)]
+    with DeviceArrays() as d:
+        P = [d.put(0.2 * rng.standard_normal(nm)) for _ in asms]
+        X, T = d.put(rng.uniform(-1.0, 1.0, (n, 3))), d.put(rng.normal(0.0, 0.5, (n, 64)))
+        G, loss = [d.filled(nm, 0.0) for _ in asms], [d.filled(1, 0.0) for _ in asms]
+
+        def gradients(together):
+            for k, a in enumerate(asms):
+                a.mlp_gradients_noalloc(10, P[k], n, X, T, G[k], loss[k])
+                if not together:
+                    a.synchronize()
+            for a in asms:
+                a.synchronize()
+            return [d.get(g, nm) for g in G]
+
+        want = gradients(False)
+        for _ in range(20):
+            for got, w in zip(gradients(True), want):
+                assert np.array_equal(got, w)
+        for a in asms:
+            a.close()

@@ -232,8 +232,8 @@ bool same_list(const MeList &a, const std::vector<int> &mu, const std::vector<in
 
 struct fb_ctx {
   int device = 0;
-  float *scratch = nullptr;   // this context's part of the device's scratch array (fb_mlp_gradients_noalloc)
-  int scratch_slot = -1;
+  float *scratch = nullptr;   // work arrays of fb_mlp_gradients_noalloc: a part of the device's scratch array
+  int scratch_slot = -1;      // or, where all parts are taken (-1), d_scratch
   int ncu = 256;              // compute units of the device
   int fused = 0;              // FB_TUNE_FUSED: 0 separate 2c/3c launches, 3 or 4 one launch (waves per SIMD)
   int persist = 0;            // FB_TUNE_PERSIST: the one launch's 3c waves take tiles from a queue
@@ -298,6 +298,7 @@ struct fb_ctx {
   };
   int64_t *list_off(int which) const { return (int64_t *)h_list.p + (size_t)which * (natoms + 1); }
   ListTail *list_tail() const { return (ListTail *)list_off(3); }
+  DevBuf d_scratch;
   DevBuf d_cell_rec, d_nblk, d_nb_keys, d_aboff;   // neighbour search in one pass
   int64_t order_ntrip = 0;
   bool lists_ok = false;
@@ -611,7 +612,7 @@ struct fb_ctx {
                       &d_mu, &d_nu, &d_mv, &d_grid2c, &d_pden, &d_wg2c, &d_cell_cnt, &d_cell_start, &d_cell_atoms, &d_atom_cell, &d_pair_disp, &d_tile_cnt, &d_tile_off, &d_gidx, &d_gout, &d_in,
                       &d_neighn, &d_noff, &d_neigh_j, &d_neigh_b, &d_neigh_back, &d_neigh_self, &d_pair_atom, &d_pair_rec, &d_pair_perm,
                       &d_bsz, &d_boff, &d_ncommon, &d_toff, &d_trip_orig, &d_tpair_orig, &d_trip, &d_tpair,
-                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_cell_rec, &d_nblk, &d_nb_keys, &d_aboff, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
+                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_scratch, &d_cell_rec, &d_nblk, &d_nb_keys, &d_aboff, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
                       &d_mlp, &d_mlp_err, &d_mlp_count, &d_queue, &d_meth3c,
                       &d_status, &d_idx3r, &d_wbsz, &d_wboff, &d_pp_map, &d_px_map, &d_px_point,
                       &d_inv_pp, &d_inv_px, &d_cand_cnt, &d_cand_off, &d_cand_j, &d_cand_b, &d_pc_n, &d_pc_off,
@@ -699,8 +700,9 @@ extern "C" {
 // partial gradients and the losses of FB_MLP_NOALLOC_MAX_BATCH rows, at fixed
 // offsets) in this file-scope device array instead of allocating them.  Each
 // GPU holds its own copy until the process ends, in NA_SLOTS parts: a context
-// takes the least used part for its lifetime, so that up to NA_SLOTS contexts
-// of a GPU do not share one.  The host never passes the array's name to a
+// has a free part to itself for its lifetime, and one that finds none gets
+// memory of its own in fb_create, so that no two contexts share work arrays.
+// The host never passes the array's name to a
 // kernel: fb_create looks up its device address once per device (with that
 // device current) and every use goes through that address.
 namespace {
@@ -710,36 +712,46 @@ constexpr int NA_SLOTS = 4;
 constexpr int NA_MAXDEV = 64;
 std::mutex g_scratch_mu;
 float *g_scratch_dev[NA_MAXDEV] = {};
-int g_scratch_use[NA_MAXDEV][NA_SLOTS] = {};
+bool g_scratch_use[NA_MAXDEV][NA_SLOTS] = {};
 }  // namespace
 static __device__ __align__(256) float scratch[NA_SLOTS * NA_FLOATS];
 
-// a part of this GPU's scratch array for a context; the device must be current
-static hipError_t scratch_take(int device, int *slot, float **out) {
+// work arrays for a context; the device must be current
+static hipError_t scratch_take(fb_ctx *ctx) {
+  const int device = ctx->device;
   if (device < 0 || device >= NA_MAXDEV) return hipErrorInvalidDevice;
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (!g_scratch_dev[device]) {
-    void *ptr = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess) return e;
-    g_scratch_dev[device] = static_cast<float *>(ptr);
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    if (!g_scratch_dev[device]) {
+      void *ptr = nullptr;
+      const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+      if (e != hipSuccess) return e;
+      g_scratch_dev[device] = static_cast<float *>(ptr);
+    }
+    bool *const use = g_scratch_use[device];
+    for (int k = 0; k < NA_SLOTS; k++)
+      if (!use[k]) {
+        use[k] = true;
+        ctx->scratch_slot = k;
+        ctx->scratch = g_scratch_dev[device] + k * NA_FLOATS;
+        return hipSuccess;
+      }
   }
-  int *const use = g_scratch_use[device];
-  *slot = (int)(std::min_element(use, use + NA_SLOTS) - use);
-  use[*slot]++;
-  *out = g_scratch_dev[device] + *slot * NA_FLOATS;
-  return hipSuccess;
+  const hipError_t e = ctx->d_scratch.ensure(sizeof(float) * NA_FLOATS);
+  ctx->scratch = ctx->d_scratch.as<float>();
+  return e;
 }
 
-static void scratch_give(int device, int slot) {
+static void scratch_give(fb_ctx *ctx) {
+  if (ctx->scratch_slot < 0) return;
   std::lock_guard<std::mutex> lock(g_scratch_mu);
-  g_scratch_use[device][slot]--;
+  g_scratch_use[ctx->device][ctx->scratch_slot] = false;
 }
 
 static thread_local std::string g_create_err = "null context";
 
 static int create_failed(fb_ctx *ctx, const char *what, hipError_t e) {
-  if (ctx->scratch_slot >= 0) scratch_give(ctx->device, ctx->scratch_slot);
+  scratch_give(ctx);
   delete ctx;
   g_create_err = std::string("fb_create: ") + what + ": " + hipGetErrorString(e);
   return FB_E_HIP;
@@ -758,7 +770,7 @@ int fb_create(fb_ctx **out, int device) {
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->ev_in, hipEventDisableTiming);
   if (e != hipSuccess) return create_failed(ctx, "streams", e);
-  e = scratch_take(device, &ctx->scratch_slot, &ctx->scratch);
+  e = scratch_take(ctx);
   if (e != hipSuccess) return create_failed(ctx, "scratch address", e);
   e = hipDeviceGetAttribute(&ctx->ncu, hipDeviceAttributeMultiprocessorCount, device);
   if (e != hipSuccess) return create_failed(ctx, "device attributes", e);
@@ -776,7 +788,7 @@ int fb_destroy(fb_ctx *ctx) {
   if (!ctx) return FB_E_ARG;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
-  scratch_give(ctx->device, ctx->scratch_slot);
+  scratch_give(ctx);
   delete ctx;
   return FB_OK;
 }

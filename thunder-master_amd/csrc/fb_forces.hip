@@ -11,7 +11,8 @@
 // Dsmoother (b.FUNCTIONS/Dsmoother.f90).  Expressions keep the reference's
 // evaluation order (the library is compiled with -ffp-contract=off).
 //
-// Layout: 2c work is one wavefront per central atom with one lane per pair
+// Layout of the generic kernels (the s/p ones are below and in
+// fb_d3c_wave.h): 2c work is one wavefront per central atom with one lane per pair
 // (the atom's pairs are contiguous), so the per-pair outputs (Dblocks, the two
 // force vectors) are stored without any reduction.  3c work is one thread per
 // triplet in the list (reference) order; each thread contracts its rotated

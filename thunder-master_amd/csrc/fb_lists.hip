@@ -2,9 +2,9 @@
 // c.SYSTEM/M_neighbors.f90 (find_neighbors :356-519, find_common_neighbors
 // :681-812).
 //
-// One workgroup per central atom walks the candidates in the reference's order
-// (image mbeta outer, atom jatom inner; or ineigh outer, jneigh inner for the
-// triplets) in chunks of the workgroup size; an ordered compaction (wave
+// The general kernels, one workgroup per central atom, walk the candidates in
+// the reference's order (image mbeta outer, atom jatom inner; or ineigh outer,
+// jneigh inner for the triplets) in chunks of the workgroup size; an ordered compaction (wave
 // ballot + cross-wave prefix in LDS) appends the accepted candidates, so no
 // sort is needed and the list order is the reference's.  Distances use the
 // reference's expression with contraction off.  Images whose bounding box lies

@@ -1034,8 +1034,11 @@ int fb_commit_tables(fb_ctx *ctx) {
   auto append_theta = [](std::vector<double> &slab, const HCell3c *const *th) {
     const size_t n = th[0]->data.size(), o = slab.size();
     slab.resize(o + n * FB_NTHETA);
-    for (int t = 0; t < FB_NTHETA; t++)
-      for (size_t e = 0; e < n; e++) slab[o + e * FB_NTHETA + t] = th[t]->data[e];
+    const double *src[FB_NTHETA];
+    for (int t = 0; t < FB_NTHETA; t++) src[t] = th[t]->data.data();
+    double *dst = slab.data() + o;
+    for (size_t e = 0; e < n; e++)
+      for (int t = 0; t < FB_NTHETA; t++) *dst++ = src[t][e];
   };
   for (auto &kv : groups) {
     const HCell3c *th[FB_NTHETA] = {nullptr};

@@ -42,6 +42,23 @@ def test_bcna_bits(n, charged):
         assert np.array_equal(asm.blocks(m), o[m]), m
 
 
+@pytest.mark.parametrize("n", [3, 17, 66])
+def test_bcna_bits_of_shell_charges_that_cancel(n):
+    st = droplet(n, [synth.SI])
+    st.dQ = np.zeros((n, 4))
+    st.dQ[:, 0] = np.random.default_rng(5).uniform(0.1, 0.4, n)
+    st.dQ[:, 1] = -st.dQ[:, 0]
+    st.dQ[3::4] = 0.0
+    ts = synth.make_tables([synth.SI])
+    asm = Assembler(ts, precision="fp64")
+    asm.add_structure(st)
+    asm.build_lists()
+    asm.assemble_all()
+    o = oracle.System(oracle.Tables(ts), st).run_all()
+    for m in HS_MATS:
+        assert np.array_equal(asm.blocks(m), o[m]), m
+
+
 @pytest.mark.parametrize("n", [3, 17, 66, 67])
 def test_density_bits(n):
     sp = synth.CHNO_SPECIES if n < 60 else [synth.SI, synth.H_SP]

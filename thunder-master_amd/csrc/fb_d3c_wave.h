@@ -350,6 +350,7 @@ __global__ __launch_bounds__(64, 2) void k_d3c_wave(DView v, DForce Fo) {
     }
     D3Sums S = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     double Eq = 0.0, Q = 0.0, stinky = 0.0;
+    bool charged = false;   // any shell of ialpha: of charges that cancel, E still follows the smoothing
     // ialpha - iatom and ialpha - jatom, and the smoothing of each
     auto arms = [&](double *a, double *b, double &d13, double &d23, double &e1, double &e2) {
 #pragma unroll
@@ -454,8 +455,12 @@ __global__ __launch_bounds__(64, 2) void k_d3c_wave(DView v, DForce Fo) {
           dQ = v.dQ[ial * FB_MAXSH + sh];
           if (dQ != 0.0) {
             gid = v.idx3c[(in12 * v.sp.ns + (in3 - 1)) * FB_MAXSUB3 + sh + 1];
-            if (gid < 0) status |= ST_NO_TABLE;
-            else Q += dQ;
+            if (gid < 0) {
+              status |= ST_NO_TABLE;
+            } else {
+              Q += dQ;
+              charged = true;
+            }
           }
         }
         if (__ballot(gid >= 0)) one_term(0.0, gid, stinky * dQ, dQ);
@@ -470,7 +475,7 @@ __global__ __launch_bounds__(64, 2) void k_d3c_wave(DView v, DForce Fo) {
       const double t1 = fma_(S.tz, ct, S.tx);
       double dA[3] = {0.0, 0.0, 0.0}, dB[3] = {0.0, 0.0, 0.0}, wA[3] = {0.0, 0.0, 0.0}, wB[3] = {0.0, 0.0, 0.0};
       double dE = 0.0;
-      if (CHG && Q != 0.0) {
+      if (CHG && charged) {
         // smoothed monopole: the density contracted with S, dipole_z and their Dblocks per target pair
         double a[3], b[3], d13, d23, e1, e2;
         arms(a, b, d13, d23, e1, e2);

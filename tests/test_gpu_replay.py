@@ -1,6 +1,7 @@
 """Builds replayed from a graph that is updated for new lists, other charges and
 another precision equal the eager builds, with eager work and host
-synchronisations in between; contexts that work at the same time do not share
+synchronisations in between, on one stream or several, without waiting for
+earlier builds; contexts that work at the same time do not share
 work arrays."""
 import ctypes as C
 
@@ -47,6 +48,80 @@ def test_updated_graph_equals_eager_builds(charged):
                     asm.assemble_S()
                     asm.synchronize()
     asm.close()
+
+
+class Hip:
+    """Streams (default priority) and events of the HIP runtime."""
+    NOT_READY = 600
+
+    def __init__(self):
+        self.lib = C.CDLL("libamdhip64.so")
+
+    def call(self, name, *args):
+        assert getattr(self.lib, name)(*args) == 0, name
+
+    def stream(self):
+        s = C.c_void_p()
+        self.call("hipStreamCreateWithFlags", C.byref(s), C.c_uint(1))
+        return s
+
+    def event(self):
+        e = C.c_void_p()
+        self.call("hipEventCreateWithFlags", C.byref(e), C.c_uint(2))
+        return e
+
+
+def silicon(stream):
+    """1728 atoms on a stream, and the blocks of both precisions."""
+    asm = Assembler(synth.make_tables([synth.SI]), precision="mixed")
+    asm._check(asm.L.fb_set_stream(asm.h, stream))
+    asm.add_structure(synth.diamond_si((6, 6, 6), sigma=0.05, seed=2))
+    asm.build_lists()
+    want = {}
+    for p in ("mixed", "fp64"):
+        asm.set_precision(p)
+        asm.assemble_all()
+        want[p] = {m: asm.blocks(m) for m in HS_MATS}
+    return asm, want
+
+
+def test_a_change_of_precision_does_not_wait_for_earlier_builds():
+    hip = Hip()
+    stream, ev = hip.stream(), hip.event()
+    asm, want = silicon(stream)
+    for _ in range(100):   # some 20 ms of binary64 builds
+        asm.assemble_all(sync=False)
+    hip.call("hipEventRecord", ev, stream)
+    asm.set_precision("mixed")
+    asm.assemble_all(sync=False)
+    state = hip.lib.hipEventQuery(ev)
+    asm.synchronize()
+    for m in HS_MATS:
+        assert np.array_equal(asm.blocks(m), want["mixed"][m]), m
+    asm.close()
+    assert state == Hip.NOT_READY
+
+
+def test_builds_on_two_streams_in_turn():
+    """Each stream waits on the device for the other's last build; the host waits for none."""
+    hip = Hip()
+    streams, ev = [hip.stream(), hip.stream()], hip.event()
+    asm, want = silicon(streams[0])
+    for turn in range(3):
+        for k in range(8):
+            p = ("mixed", "fp64")[(k // 2 + turn) % 2]
+            asm.set_precision(p)
+            for _ in range(3):
+                asm.assemble_all(sync=False)
+            hip.call("hipEventRecord", ev, streams[k % 2])
+            hip.call("hipStreamWaitEvent", streams[1 - k % 2], ev, C.c_uint(0))
+            asm._check(asm.L.fb_set_stream(asm.h, streams[1 - k % 2]))
+        asm.synchronize()
+        for m in HS_MATS:
+            assert np.array_equal(asm.blocks(m), want[p][m]), (turn, m)
+    asm.assemble_all(sync=False)
+    asm._check(asm.L.fb_set_stream(asm.h, streams[1]))
+    asm.close()   # waits for the stream that was left
 
 
 def test_gradients_of_many_contexts_do_not_share_work_arrays():

@@ -384,7 +384,14 @@ struct fb_ctx {
   bool pending = false;
   // captured H+S build
   hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  hipGraphExec_t gexec = nullptr;   // its replays are all on `stream`
+  // executable graphs that made way while a replay might still run, and the
+  // event after which none does (null: unknown)
+  struct OldGraph {
+    hipGraphExec_t exec;
+    hipEvent_t done;
+  };
+  std::vector<OldGraph> old_graphs;
   long graph_key = -1;
   long lists_gen = 0;
   bool use_graph = true;
@@ -601,6 +608,46 @@ struct fb_ctx {
     return fail(FB_E_HIP, where);
   }
 
+  bool capturing() const {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+  }
+
+  // destroy the old graphs whose replays are over, or all of them (the device
+  // has been waited for)
+  void drop_old_graphs(bool all) {
+    size_t kept = 0;
+    for (auto &g : old_graphs) {
+      if (all || (g.done && hipEventQuery(g.done) == hipSuccess)) {
+        (void)hipGraphExecDestroy(g.exec);
+        if (g.done) (void)hipEventDestroy(g.done);
+      } else {
+        old_graphs[kept++] = g;
+      }
+    }
+    old_graphs.resize(kept);
+    (void)hipGetLastError();   // an event that is not ready is no error
+  }
+
+  // gexec makes way for another one, without a wait unless eight others are
+  // still running
+  void retire_graph() {
+    if (!gexec) return;
+    drop_old_graphs(false);
+    if (old_graphs.size() >= 8 && hipDeviceSynchronize() == hipSuccess) drop_old_graphs(true);
+    OldGraph g{gexec, nullptr};
+    if (!capturing() && hipEventCreateWithFlags(&g.done, hipEventDisableTiming) == hipSuccess &&
+        hipEventRecord(g.done, stream) != hipSuccess) {
+      (void)hipEventDestroy(g.done);
+      g.done = nullptr;
+    }
+    (void)hipGetLastError();
+    old_graphs.push_back(g);
+    gexec = nullptr;
+  }
+
   int clear_status() {
     hipError_t e = hipMemsetAsync(d_status.p, 0, sizeof(int), stream);
     if (e != hipSuccess) return fail(FB_E_HIP, "status clear", e);
@@ -632,6 +679,7 @@ struct fb_ctx {
     h_list.release();
     h_in.release();
     if (ev_in) (void)hipEventDestroy(ev_in);
+    drop_old_graphs(true);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     if (h_status) (void)hipHostFree(h_status);
@@ -788,6 +836,7 @@ int fb_destroy(fb_ctx *ctx) {
   if (!ctx) return FB_E_ARG;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  (void)hipDeviceSynchronize();   // streams that were set before may still run its work
   scratch_give(ctx);
   delete ctx;
   return FB_OK;
@@ -813,7 +862,12 @@ int fb_read_positions(const char *basisfile, int nspecies, const int *nZ, const 
 
 int fb_set_stream(fb_ctx *ctx, void *s) {
   if (!ctx) return FB_E_ARG;
-  ctx->stream = s ? (hipStream_t)s : ctx->own_stream;
+  const hipStream_t to = s ? (hipStream_t)s : ctx->own_stream;
+  if (to != ctx->stream && ctx->gexec) {
+    FB_HIP(hipSetDevice(ctx->device));
+    ctx->retire_graph();   // a replay may still run on the stream that is left
+  }
+  ctx->stream = to;
   ctx->graph_key = -1;  // a captured graph is tied to its stream's device
   return FB_OK;
 }
@@ -2100,7 +2154,9 @@ static int enqueue_build(fb_ctx *ctx, int charged) {
 // (captured again when its key changes), or enqueued directly with per-kernel
 // timing, with graphs off or on the null stream.  A geometry step changes the
 // key and leaves the graph's nodes: the executable graph is then updated with
-// the new launches (1 us), where destroying and instantiating it took 140 us.
+// the new launches (1 us), where instantiating one takes 140 us.  While a
+// replay may still be reading the old arguments it is left alone and a new one
+// instantiated, so that a change of key does not wait for earlier builds.
 static int launch_build(fb_ctx *ctx, int charged) {
   if (ctx->timing || !ctx->use_graph || ctx->stream == nullptr) return enqueue_build(ctx, charged);
   // the graph holds kernel arguments by value: any change of lists, precision,
@@ -2124,12 +2180,13 @@ static int launch_build(fb_ctx *ctx, int charged) {
     if (ctx->gexec) {
       hipGraphNode_t node = nullptr;
       hipGraphExecUpdateResult res = hipGraphExecUpdateSuccess;
-      FB_HIP(hipStreamSynchronize(ctx->stream));   // no replay may be reading the arguments
-      if (hipGraphExecUpdate(ctx->gexec, g, &node, &res) != hipSuccess || res != hipGraphExecUpdateSuccess) {
-        (void)hipGetLastError();   // other nodes: a new executable graph
-        (void)hipGraphExecDestroy(ctx->gexec);
+      if (hipStreamQuery(ctx->stream) != hipSuccess) {
+        ctx->retire_graph();
+      } else if (hipGraphExecUpdate(ctx->gexec, g, &node, &res) != hipSuccess || res != hipGraphExecUpdateSuccess) {
+        (void)hipGraphExecDestroy(ctx->gexec);   // other nodes
         ctx->gexec = nullptr;
       }
+      (void)hipGetLastError();
     }
     if (!ctx->gexec) FB_HIP(hipGraphInstantiate(&ctx->gexec, g, nullptr, nullptr, 0));
     ctx->graph_key = key;

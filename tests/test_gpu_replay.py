@@ -124,6 +124,52 @@ def test_builds_on_two_streams_in_turn():
     asm.close()   # waits for the stream that was left
 
 
+def test_charges_are_not_sent_into_a_capture():
+    """The call is refused, the capture goes on, and the next build has the charges."""
+    hip = Hip()
+    stream = hip.stream()
+    sp = synth.CHNO_SPECIES
+    st = synth.random_box(synth.chno_counts(40), 1.0, 0.9, 5, sp)
+    synth.random_dQ([st], sp)
+    asm = Assembler(synth.make_tables(sp), precision="fp64")
+    asm._check(asm.L.fb_set_stream(asm.h, stream))
+    asm.add_structure(st)
+    asm.build_lists()
+    asm.set_tuning(2, 0)   # direct launches: a build can be captured by the caller
+    vna = []
+
+    def charges(scale):
+        q = np.ascontiguousarray(scale * st.dQ)
+        asm._check(asm.L.fb_set_charges(asm.h, 0, q.ctypes.data_as(C.POINTER(C.c_double))))
+
+    for scale in (1.0, 2.0, 3.0):
+        charges(scale)
+        asm.assemble_all()
+        vna.append(asm.blocks("VNA"))
+    for scale, call in ((1.0, asm.L.fb_assemble_all), (2.0, asm.L.fb_assemble_vna_2c)):
+        charges(scale)
+        hip.call("hipStreamBeginCapture", stream, C.c_int(1))
+        graph = C.c_void_p()
+        try:
+            assert call(asm.h) == -9   # FB_E_HIP
+        finally:
+            hip.call("hipStreamEndCapture", stream, C.byref(graph))
+            hip.call("hipGraphDestroy", graph)
+        for again in (scale, 3.0):
+            charges(again)
+            asm.assemble_all()
+            assert np.array_equal(asm.blocks("VNA"), vna[int(again) - 1])
+    # with the charges sent, a captured build is the build
+    hip.call("hipStreamBeginCapture", stream, C.c_int(1))
+    graph = C.c_void_p()
+    try:
+        asm.assemble_all(sync=False)
+    finally:
+        hip.call("hipStreamEndCapture", stream, C.byref(graph))
+    hip.call("hipGraphDestroy", graph)
+    asm.close()
+
+
 def test_gradients_of_many_contexts_do_not_share_work_arrays():
     """Seven contexts, each on its own stream, more than the library's fixed
     scratch has parts: enqueued together, each with its own parameters."""

@@ -1427,7 +1427,17 @@ static int send_in(fb_ctx *ctx, size_t off, size_t bytes) {
   return FB_OK;
 }
 
+// A copy into a stream that the caller captures would run at each replay, from
+// staging memory that holds other values by then, and not now; the event after
+// it could not be waited for any more.
+static int no_capture(fb_ctx *ctx) {
+  if (!ctx->capturing()) return FB_OK;
+  return ctx->fail(FB_E_HIP, "changed structures or charges cannot be sent while the stream is captured: "
+                             "assemble once before the capture");
+}
+
 static int upload_structures(fb_ctx *ctx) {
+  RC(no_capture(ctx));
   const int ns = (int)ctx->structs.size();
   int natoms = 0;
   for (auto &s : ctx->structs) natoms += s.natoms;
@@ -1514,6 +1524,7 @@ static int upload_structures(fb_ctx *ctx) {
 
 // after fb_set_charges: the charges alone
 static int upload_charges(fb_ctx *ctx) {
+  RC(no_capture(ctx));
   FB_HIP(hipEventSynchronize(ctx->ev_in));
   const size_t off = ctx->in_off[fb_ctx::IN_DQ];
   char *at = (char *)ctx->h_in.p + off;

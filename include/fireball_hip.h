@@ -312,15 +312,18 @@ int fb_mlp_forward(fb_ctx *ctx, int nme, const float *params, const float *oscal
  * with every argument in device memory: params [8576] (fb_mlp_gradients
  * layout), X [n][3] and T [n][64] in; grads [8576] and loss (one float: the
  * mean squared error over the valid output slots) out.  The work arrays
- * (partial gradients, per-row losses) live in a fixed scratch array of the
- * library, four parts of about 4.4 MB per GPU, held until the process ends;
- * the call allocates nothing, copies nothing to or from the host and does not
- * synchronize (work is enqueued on the context's stream).  n is at most
- * FB_MLP_NOALLOC_MAX_BATCH (FB_E_CAPACITY beyond).  A context has one of the
- * four parts to itself, and one that finds none free gets as much memory in
- * fb_create.  Calls of one context that overlap in time on several streams
- * race, so order them on one stream or synchronize between them.  The
- * gradients equal those of fb_mlp_gradients on the same batch. */
+ * (partial gradients, per-row losses) live in scratch memory of the library,
+ * four parts of about 4.4 MB per GPU (more where more contexts are alive at
+ * once), held until the process ends; the call allocates nothing, copies
+ * nothing to or from the host and does not synchronize (work is enqueued on
+ * the context's stream).  n is at most FB_MLP_NOALLOC_MAX_BATCH
+ * (FB_E_CAPACITY beyond).  A context has a part to itself until fb_destroy,
+ * which waits for the GPU and passes the part on.  Calls of one context that
+ * overlap in time on several streams race, so order them on one stream or
+ * synchronize between them.  A captured call may be replayed after fb_destroy
+ * too; it then must not overlap in time with calls of a context created after
+ * that, which may have the same part.  The gradients equal those of
+ * fb_mlp_gradients on the same batch. */
 #define FB_MLP_NOALLOC_MAX_BATCH 2048
 int fb_mlp_gradients_noalloc(fb_ctx *ctx, int nme, const float *params, int n, const float *X, const float *T,
                              float *grads, float *loss);

@@ -196,3 +196,51 @@ def test_gradients_of_many_contexts_do_not_share_work_arrays():
                 assert np.array_equal(got, w)
         for a in asms:
             a.close()
+
+
+def test_captured_gradients_outlive_their_context():
+    """Captured in the first and in the sixth context of seven (a fixed and a
+    further part of the scratch), replayed after all are destroyed, with eager
+    work and synchronisations between the replays."""
+    hip = Hip()
+    rng = np.random.default_rng(8)
+    n, nm, ts = 700, 8576, synth.make_tables([synth.SI])
+    with DeviceArrays() as d:
+        X, T = d.put(rng.uniform(-1.0, 1.0, (n, 3))), d.put(rng.normal(0.0, 0.5, (n, 64)))
+        P = [d.put(0.2 * rng.standard_normal(nm)) for _ in range(2)]
+        G, loss = [d.filled(nm, 0.0) for _ in P], [d.filled(1, 0.0) for _ in P]
+        asms = [Assembler(ts, precision="mixed") for _ in range(7)]
+        stream, execs, want = hip.stream(), [], []
+        for k, a in enumerate((asms[0], asms[5])):
+            a.mlp_gradients_noalloc(10, P[k], n, X, T, G[k], loss[k])
+            a.synchronize()
+            want.append((d.get(G[k], nm), d.get(loss[k], 1)))
+            a._check(a.L.fb_set_stream(a.h, stream))
+            g, e = C.c_void_p(), C.c_void_p()
+            hip.call("hipStreamBeginCapture", stream, C.c_int(1))
+            a.mlp_gradients_noalloc(10, P[k], n, X, T, G[k], loss[k])
+            hip.call("hipStreamEndCapture", stream, C.byref(g))
+            hip.call("hipGraphInstantiate", C.byref(e), g, None, None, C.c_size_t(0))
+            execs.append(e)
+        for a in asms:
+            a.close()
+        other = Assembler(ts, precision="mixed")   # has one of the parts
+        other.add_structure(synth.diamond_si((2, 2, 2), sigma=0.05, seed=2))
+        for _ in range(4):
+            zero = np.zeros(nm, np.float32)
+            for k in range(2):
+                hip.call("hipMemcpy", C.c_void_p(G[k]), zero.ctypes.data_as(C.c_void_p), C.c_size_t(zero.nbytes),
+                         C.c_int(1))
+                hip.call("hipGraphLaunch", execs[k], stream)
+            hip.call("hipStreamSynchronize", stream)
+            for k in range(2):
+                assert np.array_equal(d.get(G[k], nm), want[k][0])
+                assert np.array_equal(d.get(loss[k], 1), want[k][1])
+            other.build_lists()
+            other.assemble_all()
+            other.mlp_gradients_noalloc(10, P[0], n, X, T, G[1], loss[1])
+            other.synchronize()
+            assert np.array_equal(d.get(G[1], nm), want[0][0])
+        for e in execs:
+            hip.call("hipGraphExecDestroy", e)
+        other.close()

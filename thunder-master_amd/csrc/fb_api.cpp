@@ -232,8 +232,7 @@ bool same_list(const MeList &a, const std::vector<int> &mu, const std::vector<in
 
 struct fb_ctx {
   int device = 0;
-  float *scratch = nullptr;   // work arrays of fb_mlp_gradients_noalloc: a part of the device's scratch array
-  int scratch_slot = -1;      // or, where all parts are taken (-1), d_scratch
+  float *scratch = nullptr;   // work arrays of fb_mlp_gradients_noalloc: a part of the device's scratch
   int ncu = 256;              // compute units of the device
   int fused = 0;              // FB_TUNE_FUSED: 0 separate 2c/3c launches, 3 or 4 one launch (waves per SIMD)
   int persist = 0;            // FB_TUNE_PERSIST: the one launch's 3c waves take tiles from a queue
@@ -298,7 +297,6 @@ struct fb_ctx {
   };
   int64_t *list_off(int which) const { return (int64_t *)h_list.p + (size_t)which * (natoms + 1); }
   ListTail *list_tail() const { return (ListTail *)list_off(3); }
-  DevBuf d_scratch;
   DevBuf d_cell_rec, d_nblk, d_nb_keys, d_aboff;   // neighbour search in one pass
   int64_t order_ntrip = 0;
   bool lists_ok = false;
@@ -659,7 +657,7 @@ struct fb_ctx {
                       &d_mu, &d_nu, &d_mv, &d_grid2c, &d_pden, &d_wg2c, &d_cell_cnt, &d_cell_start, &d_cell_atoms, &d_atom_cell, &d_pair_disp, &d_tile_cnt, &d_tile_off, &d_gidx, &d_gout, &d_in,
                       &d_neighn, &d_noff, &d_neigh_j, &d_neigh_b, &d_neigh_back, &d_neigh_self, &d_pair_atom, &d_pair_rec, &d_pair_perm,
                       &d_bsz, &d_boff, &d_ncommon, &d_toff, &d_trip_orig, &d_tpair_orig, &d_trip, &d_tpair,
-                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_scratch, &d_cell_rec, &d_nblk, &d_nb_keys, &d_aboff, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
+                      &d_perm_in, &d_perm, &d_flag, &d_segincl, &d_seg_off, &d_seg_pair, &d_trip_seg, &d_pair_tgt, &d_trip_aux, &d_tgt_sum, &d_tgt_mask, &d_tgt_cnt, &d_cell_rec, &d_nblk, &d_nb_keys, &d_aboff, &d_tiles[0], &d_tiles[1], &d_tiles[2], &d_tmp,
                       &d_mlp, &d_mlp_err, &d_mlp_count, &d_queue, &d_meth3c,
                       &d_status, &d_idx3r, &d_wbsz, &d_wboff, &d_pp_map, &d_px_map, &d_px_point,
                       &d_inv_pp, &d_inv_px, &d_cand_cnt, &d_cand_off, &d_cand_j, &d_cand_b, &d_pc_n, &d_pc_off,
@@ -748,8 +746,11 @@ extern "C" {
 // partial gradients and the losses of FB_MLP_NOALLOC_MAX_BATCH rows, at fixed
 // offsets) in this file-scope device array instead of allocating them.  Each
 // GPU holds its own copy until the process ends, in NA_SLOTS parts: a context
-// has a free part to itself for its lifetime, and one that finds none gets
-// memory of its own in fb_create, so that no two contexts share work arrays.
+// has a free part to itself for its lifetime, so that no two contexts share
+// work arrays.  One that finds none gets a further part, allocated in
+// fb_create and as lasting as the others: a captured call may be replayed after
+// fb_destroy.  fb_destroy gives a part back for the next context, so there are
+// as many as contexts were alive at once, four at least.
 // The host never passes the array's name to a
 // kernel: fb_create looks up its device address once per device (with that
 // device current) and every use goes through that address.
@@ -759,8 +760,9 @@ constexpr int64_t NA_FLOATS = NA_OFF_ROW + FB_MLP_NOALLOC_MAX_BATCH;
 constexpr int NA_SLOTS = 4;
 constexpr int NA_MAXDEV = 64;
 std::mutex g_scratch_mu;
-float *g_scratch_dev[NA_MAXDEV] = {};
-bool g_scratch_use[NA_MAXDEV][NA_SLOTS] = {};
+size_t g_scratch_parts[NA_MAXDEV] = {};   // parts there are
+// parts that no context has; never destructed, as contexts may go at exit
+std::vector<float *> *const g_scratch_free = new std::vector<float *>[NA_MAXDEV];
 }  // namespace
 static __device__ __align__(256) float scratch[NA_SLOTS * NA_FLOATS];
 
@@ -768,32 +770,32 @@ static __device__ __align__(256) float scratch[NA_SLOTS * NA_FLOATS];
 static hipError_t scratch_take(fb_ctx *ctx) {
   const int device = ctx->device;
   if (device < 0 || device >= NA_MAXDEV) return hipErrorInvalidDevice;
-  {
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    if (!g_scratch_dev[device]) {
-      void *ptr = nullptr;
-      const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-      if (e != hipSuccess) return e;
-      g_scratch_dev[device] = static_cast<float *>(ptr);
-    }
-    bool *const use = g_scratch_use[device];
-    for (int k = 0; k < NA_SLOTS; k++)
-      if (!use[k]) {
-        use[k] = true;
-        ctx->scratch_slot = k;
-        ctx->scratch = g_scratch_dev[device] + k * NA_FLOATS;
-        return hipSuccess;
-      }
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  std::vector<float *> &parts = g_scratch_free[device];
+  void *ptr = nullptr;
+  size_t &n = g_scratch_parts[device];
+  parts.reserve(std::max<size_t>(n + 1, NA_SLOTS));   // room to give every part back
+  if (n == 0) {
+    const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+    if (e != hipSuccess) return e;
+    for (n = 0; n < NA_SLOTS; n++) parts.push_back(static_cast<float *>(ptr) + (NA_SLOTS - 1 - n) * NA_FLOATS);
   }
-  const hipError_t e = ctx->d_scratch.ensure(sizeof(float) * NA_FLOATS);
-  ctx->scratch = ctx->d_scratch.as<float>();
-  return e;
+  if (parts.empty()) {
+    const hipError_t e = hipMalloc(&ptr, sizeof(float) * NA_FLOATS);
+    if (e != hipSuccess) return e;
+    ctx->scratch = static_cast<float *>(ptr);
+    n++;
+  } else {
+    ctx->scratch = parts.back();
+    parts.pop_back();
+  }
+  return hipSuccess;
 }
 
 static void scratch_give(fb_ctx *ctx) {
-  if (ctx->scratch_slot < 0) return;
+  if (!ctx->scratch) return;
   std::lock_guard<std::mutex> lock(g_scratch_mu);
-  g_scratch_use[ctx->device][ctx->scratch_slot] = false;
+  g_scratch_free[ctx->device].push_back(ctx->scratch);
 }
 
 static thread_local std::string g_create_err = "null context";
@@ -836,8 +838,9 @@ int fb_destroy(fb_ctx *ctx) {
   if (!ctx) return FB_E_ARG;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
-  (void)hipDeviceSynchronize();   // streams that were set before may still run its work
-  scratch_give(ctx);
+  // streams that were set before may still run its work; where the wait fails
+  // (a capture goes on somewhere), its scratch is nobody's any more
+  if (hipDeviceSynchronize() == hipSuccess) scratch_give(ctx);
   delete ctx;
   return FB_OK;
 }

@@ -1,6 +1,8 @@
 """Tiles of the pseudopotential triplets around a wavefront's window of 64
 segments per atom, and PP lists built without the structure's own lists.  Lists
 and blocks equal the oracle's."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -39,3 +41,35 @@ def test_segments_around_a_window(n):
     for k in ("SVNL", "VNL"):
         assert np.array_equal(asm.pp_blocks(k), ref[k]), k
     asm.close()
+
+
+def test_longer_cutoffs_on_structures_that_are_on_the_gpu():
+    """fb_set_species between two PP list builds: the second equals a fresh context's."""
+    sp = synth.with_pp([synth.SI])
+    ts = synth.add_pp_tables(synth.make_tables(sp))
+    st = synth.diamond_si((4, 4, 4), sigma=0.05, seed=2)
+
+    def cutoffs(asm, scale):
+        nssh, lssh = np.array([2], np.int32), np.array([[0, 1, 0, 0]], np.int32)
+        rc = scale * np.array([[*sp[0].rcutoffA, 0.0, 0.0]])
+        asm._check(asm.L.fb_set_species(asm.h, 1, None, nssh.ctypes.data_as(C.POINTER(C.c_int)),
+                                        lssh.ctypes.data_as(C.POINTER(C.c_int)),
+                                        rc.ctypes.data_as(C.POINTER(C.c_double))))
+        asm._check(asm.L.fb_commit_tables(asm.h))
+
+    fresh = Assembler(ts, precision="fp64")
+    fresh.add_structure(st)
+    fresh.build_lists_pp()
+    want = fresh.pp_lists()
+    asm = Assembler(ts, precision="fp64")
+    cutoffs(asm, 0.6)
+    asm.add_structure(st)
+    asm.build_lists_pp()
+    assert not np.array_equal(asm.pp_lists()["pp_n"], want["pp_n"])
+    cutoffs(asm, 1.0)
+    asm.build_lists_pp()
+    got = asm.pp_lists()
+    for k in PP_LIST_KEYS:
+        assert np.array_equal(got[k], want[k]), k
+    asm.close()
+    fresh.close()

@@ -920,6 +920,7 @@ int fb_set_species(fb_ctx *ctx, int ns, const int *nZ, const int *nssh, const in
   ctx->maxsh = 1;
   for (int i = 0; i < ns; i++) ctx->maxsh = std::max(ctx->maxsh, sp.nssh[i]);
   ctx->species_set = true;
+  ctx->structs_dirty = true;   // the cells are as wide as the longest cutoff
   ctx->tables_ok = false;
   ctx->lists_ok = false;
   ctx->pp_lists_ok = false;

@@ -73,3 +73,50 @@ def test_longer_cutoffs_on_structures_that_are_on_the_gpu():
         assert np.array_equal(got[k], want[k]), k
     asm.close()
     fresh.close()
+
+
+def test_cells_after_a_list_build_that_failed():
+    """Wider PP cutoffs on the GPU, a PP list build refused under capture, then the same build outside."""
+    sp = synth.with_pp([synth.SI])
+    ts = synth.add_pp_tables(synth.make_tables(sp))
+    st = synth.diamond_si((4, 4, 4), sigma=0.05, seed=2)
+
+    def pp_cutoff(asm, rc):
+        npp, lpp, clv = np.array([2], np.int32), np.array([[0, 1, 0, 0]], np.int32), np.array([[-2.6, 1.3, 0.0, 0.0]])
+        rpp = np.array([rc])
+        asm._check(asm.L.fb_set_species_pp(asm.h, npp.ctypes.data_as(C.POINTER(C.c_int)),
+                                           lpp.ctypes.data_as(C.POINTER(C.c_int)),
+                                           rpp.ctypes.data_as(C.POINTER(C.c_double)),
+                                           clv.ctypes.data_as(C.POINTER(C.c_double))))
+        asm._check(asm.L.fb_commit_tables(asm.h))
+
+    fresh = Assembler(ts, precision="fp64")
+    pp_cutoff(fresh, 4.0)
+    fresh.add_structure(st)
+    fresh.build_lists_pp()
+    want = fresh.pp_lists()
+    hip = C.CDLL("libamdhip64.so")
+    stream, graph = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), C.c_uint(1)) == 0
+    asm = Assembler(ts, precision="fp64")
+    asm._check(asm.L.fb_set_stream(asm.h, stream))
+    asm.add_structure(st)
+    asm.build_lists()
+    pp_cutoff(asm, 4.0)
+    asm.assemble_all()   # sends the structures
+    assert hip.hipStreamBeginCapture(stream, C.c_int(1)) == 0
+    try:
+        n = C.c_int64()
+        assert asm.L.fb_build_lists_pp(asm.h, C.byref(n), C.byref(n), C.byref(n)) != 0
+    finally:
+        hip.hipStreamEndCapture(stream, C.byref(graph))
+        if graph.value:
+            hip.hipGraphDestroy(graph)
+    hip.hipGetLastError()
+    asm._check(asm.L.fb_set_stream(asm.h, None))   # the capture's stream stays invalid
+    asm.build_lists_pp()
+    got = asm.pp_lists()
+    for k in PP_LIST_KEYS:
+        assert np.array_equal(got[k], want[k]), k
+    asm.close()
+    fresh.close()

@@ -1812,26 +1812,29 @@ static int build_cells(fb_ctx *ctx) {
   FB_HIP(ctx->d_cell_rec.ensure(sizeof(CellAtom) * std::max(N, 1)));
   CellAtom *rec = ctx->d_cell_rec.as<CellAtom>();
   DView v = ctx->view();
-  ctx->cells_ok = true;
   // one workgroup up to 8192 atoms: 14 us at 2048 atoms where the separate
   // launches take 36, and 4 us more per further 1024
-  if (C <= FB_CELLS_ONE && N <= 8192)
-    return ctx->launch("cells", [&] {
+  if (C <= FB_CELLS_ONE && N <= 8192) {
+    RC(ctx->launch("cells", [&] {
       return fbk_cells(v, (int)C, ctx->d_cell_start.as<int64_t>(), ctx->d_cell_atoms.as<int>(), rec, st);
-    });
-  FB_HIP(ctx->d_cell_cnt.ensure(sizeof(int) * C));
-  FB_HIP(ctx->d_atom_cell.ensure(sizeof(int) * std::max(N, 1)));
-  RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
-  RC(ctx->launch("cell_count", [&] {
-    return fbk_cell_count(v, ctx->d_cell_cnt.as<int>(), ctx->d_atom_cell.as<int>(), st);
-  }));
-  RC(scan_i32(ctx, ctx->d_cell_cnt.as<int>(), ctx->d_cell_start.as<int64_t>(), C));
-  RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
-  v = ctx->view();
-  return ctx->launch("cell_fill", [&] {
-    return fbk_cell_fill(v, ctx->d_atom_cell.as<int>(), ctx->d_cell_cnt.as<int>(), ctx->d_cell_atoms.as<int>(), rec,
-                         st);
-  });
+    }));
+  } else {
+    FB_HIP(ctx->d_cell_cnt.ensure(sizeof(int) * C));
+    FB_HIP(ctx->d_atom_cell.ensure(sizeof(int) * std::max(N, 1)));
+    RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
+    RC(ctx->launch("cell_count", [&] {
+      return fbk_cell_count(v, ctx->d_cell_cnt.as<int>(), ctx->d_atom_cell.as<int>(), st);
+    }));
+    RC(scan_i32(ctx, ctx->d_cell_cnt.as<int>(), ctx->d_cell_start.as<int64_t>(), C));
+    RC(ctx->launch("cell_clear", [&] { return fbk_fill_i32(ctx->d_cell_cnt.as<int>(), C, 0, st); }));
+    v = ctx->view();
+    RC(ctx->launch("cell_fill", [&] {
+      return fbk_cell_fill(v, ctx->d_atom_cell.as<int>(), ctx->d_cell_cnt.as<int>(), ctx->d_cell_atoms.as<int>(), rec,
+                           st);
+    }));
+  }
+  ctx->cells_ok = !ctx->capturing();   // launches that the caller captures have not run
+  return FB_OK;
 }
 
 static int ensure_pairs(fb_ctx *ctx) {

@@ -233,6 +233,8 @@ bool same_list(const MeList &a, const std::vector<int> &mu, const std::vector<in
 struct fb_ctx {
   int device = 0;
   float *scratch = nullptr;   // work arrays of fb_mlp_gradients_noalloc: a part of the device's scratch
+  bool scratch_used = false;  // on the current stream, and on one that was left
+  bool scratch_left = false;
   int ncu = 256;              // compute units of the device
   int fused = 0;              // FB_TUNE_FUSED: 0 separate 2c/3c launches, 3 or 4 one launch (waves per SIMD)
   int persist = 0;            // FB_TUNE_PERSIST: the one launch's 3c waves take tiles from a queue
@@ -837,10 +839,13 @@ int fb_create(fb_ctx **out, int device) {
 int fb_destroy(fb_ctx *ctx) {
   if (!ctx) return FB_E_ARG;
   (void)hipSetDevice(ctx->device);
-  (void)hipStreamSynchronize(ctx->stream);
-  // streams that were set before may still run its work; where the wait fails
-  // (a capture goes on somewhere), its scratch is nobody's any more
-  if (hipDeviceSynchronize() == hipSuccess) scratch_give(ctx);
+  const bool waited = hipStreamSynchronize(ctx->stream) == hipSuccess;
+  // streams that were set before may still run its work; scratch that may
+  // still be written, where a capture elsewhere forbids the wait, is not
+  // passed on
+  if (hipDeviceSynchronize() == hipSuccess || (!ctx->scratch_left && (waited || !ctx->scratch_used)))
+    scratch_give(ctx);
+  (void)hipGetLastError();
   delete ctx;
   return FB_OK;
 }
@@ -869,6 +874,10 @@ int fb_set_stream(fb_ctx *ctx, void *s) {
   if (to != ctx->stream && ctx->gexec) {
     FB_HIP(hipSetDevice(ctx->device));
     ctx->retire_graph();   // a replay may still run on the stream that is left
+  }
+  if (to != ctx->stream && ctx->scratch_used) {
+    ctx->scratch_left = true;
+    ctx->scratch_used = false;
   }
   ctx->stream = to;
   ctx->graph_key = -1;  // a captured graph is tied to its stream's device
@@ -2704,6 +2713,7 @@ int fb_mlp_gradients_noalloc(fb_ctx *ctx, int nme, const float *params, int n, c
     return ctx->fail(FB_E_CAPACITY, "mlp_gradients_noalloc: batch larger than FB_MLP_NOALLOC_MAX_BATCH (2048)");
   FB_HIP(hipSetDevice(ctx->device));
   float *const sc = ctx->scratch;
+  ctx->scratch_used = true;
   return mlp_fwd_bwd(ctx, sc, sc + NA_OFF_ROW, params, grads, nme, n, X, T, loss);
 }
 

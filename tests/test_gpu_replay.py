@@ -172,28 +172,32 @@ def test_charges_are_not_sent_into_a_capture():
 
 def test_gradients_of_many_contexts_do_not_share_work_arrays():
     """Seven contexts, each on its own stream, more than the library's fixed
-    scratch has parts: enqueued together, each with its own parameters."""
+    scratch has parts: enqueued together, each with its own parameters, targets,
+    batch and element count.  Gradients and losses are those of serial calls."""
     rng = np.random.default_rng(4)
-    n, nm, ts = 2048, 8576, synth.make_tables([synth.SI])
+    nm, ts = 8576, synth.make_tables([synth.SI])
+    rows, nme = [2048, 1999, 1024, 2048, 700, 1500, 2033], [10, 3, 10, 1, 10, 3, 10]
     asms = [Assembler(ts, precision="mixed") for _ in range(7)]
     with DeviceArrays() as d:
         P = [d.put(0.2 * rng.standard_normal(nm)) for _ in asms]
-        X, T = d.put(rng.uniform(-1.0, 1.0, (n, 3))), d.put(rng.normal(0.0, 0.5, (n, 64)))
+        X = d.put(rng.uniform(-1.0, 1.0, (2048, 3)))
+        T = [d.put(rng.normal(0.0, 0.5, (n, 64))) for n in rows]
         G, loss = [d.filled(nm, 0.0) for _ in asms], [d.filled(1, 0.0) for _ in asms]
 
         def gradients(together):
             for k, a in enumerate(asms):
-                a.mlp_gradients_noalloc(10, P[k], n, X, T, G[k], loss[k])
+                a.mlp_gradients_noalloc(nme[k], P[k], rows[k], X, T[k], G[k], loss[k])
                 if not together:
                     a.synchronize()
             for a in asms:
                 a.synchronize()
-            return [d.get(g, nm) for g in G]
+            return [(d.get(g, nm), d.get(x, 1)) for g, x in zip(G, loss)]
 
         want = gradients(False)
+        assert len({float(w[1][0]) for w in want}) == len(want)
         for _ in range(20):
             for got, w in zip(gradients(True), want):
-                assert np.array_equal(got, w)
+                assert np.array_equal(got[0], w[0]) and np.array_equal(got[1], w[1])
         for a in asms:
             a.close()
 

@@ -292,13 +292,15 @@ struct fb_ctx {
   DevBuf d_mat[FB_NMAT];
   int64_t npairs = 0, ntrip = 0, nseg = 0, blen = 0;
   std::vector<int64_t> h_noff, h_toff, h_boff_struct;
-  HostBuf h_list;   // natoms + 1 pair, block element and triplet offsets, then ListTail
+  HostBuf h_list;   // natoms + 1 pair, block element and triplet offsets, ListTail, 2c workgroups
   struct ListTail {
     TgtSum tgt;
     int status;
   };
   int64_t *list_off(int which) const { return (int64_t *)h_list.p + (size_t)which * (natoms + 1); }
   ListTail *list_tail() const { return (ListTail *)list_off(3); }
+  size_t list_wg_off() const { return (sizeof(int64_t) * 3 * (natoms + 1) + sizeof(ListTail) + 15) & ~(size_t)15; }
+  int *list_wg() const { return (int *)((char *)h_list.p + list_wg_off()); }   // natoms + 1, room for whole words
   DevBuf d_cell_rec, d_nblk, d_nb_keys, d_aboff;   // neighbour search in one pass
   int64_t order_ntrip = 0;
   bool lists_ok = false;
@@ -1423,19 +1425,23 @@ int fb_set_qin(fb_ctx *ctx, int is, const double *qin) {
   return FB_OK;
 }
 
-// [off, off + bytes) of the staged inputs to the device.  Up to 1 MB a kernel
-// reads the page-locked memory itself: it follows the stream's kernels
+// bytes of page-locked memory to the device, both 16-byte aligned.  Up to 1 MB
+// a kernel reads the page-locked memory itself: it follows the stream's kernels
 // directly, where a copy engine is waited for (build with new charges of 501
 // atoms: seven copies 159 us, one by the engine 168 us, by the kernel 147 us).
-static int send_in(fb_ctx *ctx, size_t off, size_t bytes) {
-  char *dst = (char *)ctx->d_in.p + off;
-  const char *src = (const char *)ctx->h_in.p + off;
-  if (bytes <= (1u << 20)) {
-    const int rc = fbk_copy_in(src, dst, (int64_t)((bytes + 15) / 16), ctx->stream);
-    if (rc) return ctx->fail(FB_E_HIP, "upload structures", (hipError_t)rc);
-  } else {
+// It moves whole 16-byte words, so both sides have room for the last one.
+static int copy_in(fb_ctx *ctx, void *dst, const void *src, size_t bytes, const char *what) {
+  if (bytes > (1u << 20)) {
     FB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    return FB_OK;
   }
+  const int rc = fbk_copy_in(src, dst, (int64_t)((bytes + 15) / 16), ctx->stream);
+  return rc ? ctx->fail(FB_E_HIP, what, (hipError_t)rc) : FB_OK;
+}
+
+// [off, off + bytes) of the staged inputs
+static int send_in(fb_ctx *ctx, size_t off, size_t bytes) {
+  RC(copy_in(ctx, (char *)ctx->d_in.p + off, (const char *)ctx->h_in.p + off, bytes, "upload structures"));
   FB_HIP(hipEventRecord(ctx->ev_in, ctx->stream));
   return FB_OK;
 }
@@ -1639,25 +1645,29 @@ static int ensure_triplets(fb_ctx *ctx, int64_t T) {
 
 // 2c workgroups: whole atoms, at most 16 atoms and FB_2C_PCAP pairs each (an
 // atom with more neighbours gets a workgroup of its own, run in passes), and
-// the order of the pairs inside
+// the order of the pairs inside.  Their first atoms are written to page-locked
+// memory, which the next build writes again only after it has waited for the
+// stream.
 static int pair_order(fb_ctx *ctx) {
-  std::vector<int> wg;
-  wg.push_back(0);
-  int na = 0;
+  int *const wg = ctx->list_wg();
+  int nwg = 0, na = 0;
   int64_t np = 0;
+  wg[0] = 0;
   for (int a = 0; a < ctx->natoms; a++) {
     int64_t n = ctx->h_noff[a + 1] - ctx->h_noff[a];
     if (na > 0 && (na == 16 || np + n > FB_2C_PCAP)) {
-      wg.push_back(a);
+      wg[++nwg] = a;
       na = 0;
       np = 0;
     }
     na++;
     np += n;
   }
-  wg.push_back(ctx->natoms);
-  ctx->nwg2c = (int)wg.size() - 1;
-  RC(upload(ctx, ctx->d_wg2c, wg.data(), wg.size() * sizeof(int), "upload wg2c"));
+  wg[++nwg] = ctx->natoms;
+  ctx->nwg2c = nwg;
+  const size_t bytes = sizeof(int) * (nwg + 1);
+  FB_HIP(ctx->d_wg2c.ensure(bytes + 16));
+  RC(copy_in(ctx, ctx->d_wg2c.p, wg, bytes, "upload wg2c"));
   DView v = ctx->view();
   return ctx->launch("pair_perm", [&] { return fbk_pair_perm(v, ctx->d_pair_perm.as<unsigned char>(), ctx->stream); });
 }
@@ -1958,7 +1968,7 @@ int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
   FB_HIP(ctx->d_neighn.ensure(sizeof(int) * N));
   FB_HIP(ctx->d_noff.ensure(sizeof(int64_t) * (N + 1)));
   FB_HIP(ctx->d_neigh_self.ensure(sizeof(int) * N));
-  FB_HIP(ctx->h_list.ensure(sizeof(int64_t) * 3 * (N + 1) + sizeof(fb_ctx::ListTail)));
+  FB_HIP(ctx->h_list.ensure(ctx->list_wg_off() + sizeof(int) * (N + 1) + 16));
   RC(build_cells(ctx));
   int nmax = 0;
   ctx->h_noff.resize(N + 1);

@@ -9,7 +9,8 @@
 // getDMEs_Fdata_3c (e.FDATA/M_Fdata_3c.f90:549-846), Depsilon_2c / Depsilon_3c
 // (b.FUNCTIONS), Dtwister / Drotate (c.SYSTEM/M_Drotations.f90:102-298) and
 // Dsmoother (b.FUNCTIONS/Dsmoother.f90).  Expressions keep the reference's
-// evaluation order (the library is compiled with -ffp-contract=off).
+// evaluation order (the library is compiled with -ffp-contract=off), except in
+// the s/p 3c kernels of fb_d3c_wave.h.
 //
 // Layout of the generic kernels (the s/p ones are below and in
 // fb_d3c_wave.h): 2c work is one wavefront per central atom with one lane per pair
@@ -1201,7 +1202,7 @@ __global__ __launch_bounds__(WD2S) void k_d2c_sp(DView v, DForce Fo, int mask) {
 // in their order.
 // Bound by the latency of that dependent binary64 arithmetic: k_d2c_sp's lane
 // per pair needs more than 256 registers (one wavefront per SIMD) and a launch
-// per part.  Charged droplet of 151 atoms, 4245 pairs: 228 -> 44 us.
+// per part.  Charged droplet of 151 atoms, 4245 pairs: 228 -> 48 us.
 #define D2_P 64                 // pairs per workgroup
 
 struct D2Lds {
@@ -1498,12 +1499,20 @@ __global__ __launch_bounds__(3 * D2_P, 2) void k_d2c_split(DView v, DForce Fo, i
 // Few pairs go to k_d2c_split, an item per workgroup up to 128 groups and half
 // of the items above.  With more pairs one lane per pair fills the chip, and
 // the split form's shared arithmetic, done by three wavefronts, is what
-// remains; neutral lists of several rounds of workgroups are its again, whose
-// pairs of other classes diverge in fewer registers.  Measured, k_d2c_sp /
-// split, neutral and charged: Si 7,560 pairs 53 / 27, 120 / 48 us; 17,930 pairs
-// 58 / 39, 120 / 91; 35,016 pairs 70 / 60, 131 / 132; 60,502 pairs 73 / 78,
-// 134 / 175; 143,410 pairs 186 / 167, 353 / 393; C/H/N/O 137,950 pairs 225 /
-// 157, 488 / 399.
+// remains.  The rule knows the length of the list and whether shells are
+// charged: it is drawn for lists of one pair class, whose k_d2c_sp is at its
+// best.  Measured, k_d2c_sp / split in us, neutral and charged:
+//   Si     7,560 pairs  53 / 27, 120 / 48     60,510 pairs  75 / 76, 138 / 170
+//         17,930        58 / 39, 120 / 91     80,680       122 / 97, 233 / 225
+//         35,010        72 / 64, 133 / 128    94,118       124 / 109, 238 / 249
+//         42,016        72 / 66, 135 / 147   109,802       126 / 128, 247 / 302
+//         50,426        73 / 74, 136 / 168   143,422       180 / 159, 357 / 384
+// Lists of several classes, whose lanes diverge in k_d2c_sp, are faster in the
+// split form at every length, so above 560 groups (neutral: up to 1536) they
+// take the slower one:
+//   C/H/N/O  22,636     96 / 48, 194 / 98     63,914       100 / 77, 198 / 184
+//            34,798     99 / 63, 194 / 132    96,160       158 / 109, 343 / 270
+//            49,798    100 / 74, 200 / 178   137,264       215 / 153, 484 / 394
 extern "C" int fbk_d2c_sp(const DView &v, const DForce &f, int mask, hipStream_t st) {
   if (v.npairs == 0) return 0;
   const int64_t groups = (v.npairs + D2_P - 1) / D2_P;

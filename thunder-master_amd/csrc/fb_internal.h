@@ -108,25 +108,26 @@ struct DStruct {
   int cn[3], cell_off;
 };
 
-// Totals of one atom's targets (triplets, segments, tiles per 3c chunk), or
-// their exclusive prefix over the atoms; and what the target-order triplet
-// kernel writes (DView holds the same arrays)
 // an atom as the neighbour search reads it, in cell order
 struct CellAtom {
   double r[3], rc;              // home position, largest cutoff of its species
 };
 #define FB_CELLS_ONE 4096       // cells that one workgroup's LDS counts
 #define FB_NB_CAP 256           // neighbours per atom of the one-pass search
+// what the one-pass search's placing kernel writes (DView holds the same arrays)
 struct NbOut {
   int *neigh_j, *neigh_b, *neigh_back, *pair_atom;
   int4 *rec;
   int64_t *boff;
   double *disp;
 };
+// totals of one atom's targets (triplets, segments, tiles per 3c chunk), or
+// their exclusive prefix over the atoms
 struct TgtSum {
   int64_t trip;
   int seg, tile[3];
 };
+// what the target-order triplet kernel writes (the same)
 struct TgtOut {
   int4 *trip;
   int *trip_pair, *trip_seg, *trip_aux;

@@ -387,6 +387,7 @@ struct fb_ctx {
   // captured H+S build
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;   // its replays are all on `stream`
+  bool replaying = false;           // one since the stream was last waited for
   // executable graphs that made way while a replay might still run, and the
   // event after which none does (null: unknown)
   struct OldGraph {
@@ -588,6 +589,7 @@ struct fb_ctx {
     hipError_t e = hipMemcpyAsync(h_status, d_status.p, sizeof(int), hipMemcpyDeviceToHost, stream);
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return fail(FB_E_HIP, where, e);
+    replaying = false;
     const int st = *h_status;
     if (st) {
       e = hipMemsetAsync(d_status.p, 0, sizeof(int), stream);
@@ -1988,6 +1990,7 @@ int fb_build_lists(fb_ctx *ctx, int64_t *npairs_total, int64_t *ntrip_total) {
     ctx->done[i] = 0;
   }
   FB_HIP(hipStreamSynchronize(st));
+  ctx->replaying = false;
   ctx->lists_ok = true;
   ctx->lists_gen++;
   if (general) ctx->order_gen = ctx->lists_gen;   // triplets_by_sort formed it
@@ -2217,7 +2220,7 @@ static int launch_build(fb_ctx *ctx, int charged) {
     if (ctx->gexec) {
       hipGraphNode_t node = nullptr;
       hipGraphExecUpdateResult res = hipGraphExecUpdateSuccess;
-      if (hipStreamQuery(ctx->stream) != hipSuccess) {
+      if (ctx->replaying && hipStreamQuery(ctx->stream) != hipSuccess) {
         ctx->retire_graph();
       } else if (hipGraphExecUpdate(ctx->gexec, g, &node, &res) != hipSuccess || res != hipGraphExecUpdateSuccess) {
         (void)hipGraphExecDestroy(ctx->gexec);   // other nodes
@@ -2228,6 +2231,7 @@ static int launch_build(fb_ctx *ctx, int charged) {
     if (!ctx->gexec) FB_HIP(hipGraphInstantiate(&ctx->gexec, g, nullptr, nullptr, 0));
     ctx->graph_key = key;
   }
+  ctx->replaying = true;
   FB_HIP(hipGraphLaunch(ctx->gexec, ctx->stream));
   return FB_OK;
 }
